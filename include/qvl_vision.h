@@ -121,11 +121,14 @@ int qvl_dense(void* stream, int32_t dtype, int32_t epilogue, const void* d_x, in
               void* d_y, int64_t ldc, int64_t m, int64_t n, int64_t k);
 
 /* qvl_dense with a workspace for split-K: bf16, when the tiles do not fill whole rounds of the
- * GPU's compute units, the last round's tiles are split along K; fp32, when the 128 x 128 tiles
- * fill at most half of the workgroup slots (two per compute unit), every tile is split along K
- * into up to 8 parts. The parts' fp32 partials go to `d_workspace` and a second kernel sums them
- * (in part order) before the epilogue: same results up to fp32 summation order. Without enough
- * workspace it behaves exactly like qvl_dense.
+ * GPU's compute units, the last round's tiles are split along K. The parts' fp32 partials go to
+ * `d_workspace` and a second kernel sums them (in part order) before the epilogue: same results up
+ * to fp32 summation order. fp32: where the workspace holds both operands again, each is written there
+ * as two f16 terms per value with a power-of-two factor per row, and the Dense runs as three f16 MFMA
+ * products into fp32 accumulators (nearer to float64 than the fp32 MFMA; rows or weights that hold
+ * infinities or NaN get fp32 sums); else, when the 128 x 128 tiles of the fp32 MFMA kernel fill at
+ * most half of the workgroup slots (two per compute unit), every tile is split along K into up to 8
+ * parts. Without enough workspace it behaves exactly like qvl_dense.
  * qvl_dense_workspace_size gives the bytes that always suffice on the current device. */
 int qvl_dense_workspace_size(size_t* bytes);
 int qvl_dense_ws(void* stream, int32_t dtype, int32_t epilogue, const void* d_x, int64_t lda,
@@ -159,6 +162,11 @@ int qvl_set_gemm_plan(int32_t tile, int32_t split_mode, int32_t group_n);
  * most 2x the compute units; else one group), 1 = one group, 2 = two groups. Outputs of 1 and 2 differ
  * only in fp32 summation order. No counterpart in the reference. */
 int qvl_set_attention_plan(int32_t key_groups);
+
+/* Tile override for the fp32 Dense with a workspace, FROM THE CALLING THREAD ONLY (thread-local), for tests
+ * and tuning: 0 = the default rules, 1..4 = f16-split operands on 64x128 (two-stage ring), 64x128 (three
+ * stages), 128x256 or 256x256 tiles, 5 = the fp32 MFMA kernel. No counterpart in the reference. */
+int qvl_set_f32_plan(int32_t tile);
 
 /* LayerNorm over the last axis: fp32 mean / biased variance / rsqrt(var + eps), affine, cast
  * back (model.py:375-388). cols must be a multiple of 8 and <= 8192. bf16 or fp32. */

@@ -88,6 +88,19 @@ __device__ __forceinline__ int xcd_remap(int wg, int n) {
   return xcd < r ? xcd * (q + 1) + idx : r * (q + 1) + (xcd - r) * q + idx;
 }
 
+// Tile t -> (row tile, column tile). Tiles are ordered in panels of group_n column tiles, row tile
+// by row tile within a panel, so the tiles that one XCD runs in one round (a contiguous range, see
+// xcd_remap) form a block of about (cus/8)/group_n row tiles by group_n column tiles, and the
+// operand bytes that XCD's L2 fetches per round are ~rows*|x tile| + cols*|w tile| instead of the
+// whole weight matrix (row-major order puts all column tiles of 2 row tiles in one round).
+__device__ __forceinline__ void tile_coords(int tile, int tiles_m, int tiles_n, int group_n, int& tm, int& tn) {
+  const int panel = tile / (tiles_m * group_n);
+  const int width = min(group_n, tiles_n - panel * group_n);
+  const int r = tile - panel * tiles_m * group_n;
+  tm = r / width;
+  tn = panel * group_n + r % width;
+}
+
 }  // namespace qvl
 
 // Error plumbing shared by the host entry points (set_error in qvl_meta.cpp, check_launch in

@@ -1,0 +1,482 @@
+// fp32 Dense on the f16 matrix cores: each fp32 operand is written as two f16 terms of a power-of-two
+// multiple of it, x 2^e = hi + lo + r (|r| <= 2^-23 |x 2^e|: 11 + 11 significant bits and lo's sign), and
+//   x . w = 2^-(ex + ew) (hi_x . hi_w + hi_x . lo_w + lo_x . hi_w) + (lo_x . lo_w and r terms)
+// runs as three v_mfma_f32_32x32x16_f16 products into one fp32 accumulator. The dropped terms are at most
+// 2^-22 of a product, random in sign; the f16 products themselves are exact in fp32. One fp32 accumulation
+// chain takes 3 K / 16 instruction steps against K / 2 for v_mfma_f32_32x32x2_f32, so the result is nearer to
+// float64 than the fp32 MFMA's: normal operands, K = 1024 / 4096: 3.6e-7 / 7.1e-7 of the result's norm (less
+// where K is split) against 5.7e-7 / 1.1e-6, at 3/16 of its matrix time (MI355X: 2.5 PFLOP/s f16 against 157
+// TFLOP/s fp32).
+//
+// Split rows: a row of K values (K a multiple of 32) is K / 32 groups of [32 hi | 32 lo] f16, 128 bytes a
+// group: the same bytes as the fp32 row, and one group is one k-step's LDS row of the bf16 GEMM's layout. The
+// exponent is per row, so that the row's largest value lands in [2^14, 2^15): values down to 2^-17 of it keep
+// 22 bits, smaller ones an absolute error of 2^-39 of it.
+#include <math.h>
+
+#include <algorithm>
+
+#include "qvl_kernels.h"
+
+namespace qvl {
+
+typedef _Float16 f16;
+typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+
+// The power of two that takes values up to `mx` (finite, >= 0) into f16 range: mx * s in [2^14, 2^15).
+// Clamped to normal fp32 values of s and 1 / s; zero and non-finite maxima give 1.
+__device__ __forceinline__ float split_scale(float mx) {
+  const int ex = (int)(__float_as_uint(mx) >> 23);   // biased exponent (mx >= 0); 0: zero or denormal
+  if (ex == 0 || ex == 255) return mx > 0.f && ex == 0 ? 0x1p126f : 1.0f;
+  return __uint_as_float((uint32_t)min(127 + 14 - (ex - 127), 253) << 23);
+}
+
+__device__ __forceinline__ void split4(const f32x4& v, float s, f16x4& hi, f16x4& lo) {
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const float t = v[e] * s;
+    hi[e] = (f16)t;
+    lo[e] = (f16)(t - (float)hi[e]);
+  }
+}
+
+// Writes columns c..c+3 (c a multiple of 4) of a split row.
+__device__ __forceinline__ void store_split4(f16* row, int c, const f16x4& hi, const f16x4& lo) {
+  f16* g = row + (c >> 5) * 64 + (c & 31);
+  *reinterpret_cast<f16x4*>(g) = hi;
+  *reinterpret_cast<f16x4*>(g + 32) = lo;
+}
+
+// ---------------------------------------------------------------------------------------------
+// fp32 rows -> split rows: a row's maximum, then its values scaled and split. Memory bound (each row read
+// and written once): T = 64 or 256 threads hold a row in registers, CH chunks of 4 values each, so that
+// every load is in flight at once and long rows have as many waves as short ones. Rows of x (the first) and
+// of w share one launch.
+// ---------------------------------------------------------------------------------------------
+struct SplitRowsParams {
+  const float* src[2];
+  int64_t ld[2];
+  f16* dst[2];
+  float* inv[2];      // 2^-e of each row; NaN for a row that holds an infinity or a NaN
+  int rows[2];
+  int K;
+};
+
+template <int T, int CH>
+__global__ __launch_bounds__(256) void split_rows_kernel(SplitRowsParams p) {
+  constexpr int RPB = 256 / T;
+  __shared__ float wave_max[4];
+  const int first = (p.rows[0] + RPB - 1) / RPB, which = (int)blockIdx.x >= first;
+  const int t = threadIdx.x % T;
+  const int row = ((int)blockIdx.x - (which ? first : 0)) * RPB + threadIdx.x / T;
+  if (row >= p.rows[which]) return;                 // (a whole wave, or with T = 256 never)
+  const float* src = p.src[which] + (int64_t)row * p.ld[which];
+  f32x4 v[CH];
+#pragma unroll
+  for (int i = 0; i < CH; ++i) {
+    const int c = (t + i * T) * 4;
+    v[i] = c < p.K ? *reinterpret_cast<const f32x4*>(src + c) : f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+  // (the bits of |x| order as the values do, infinities and NaN above every finite one)
+  uint32_t mb = 0;
+#pragma unroll
+  for (int i = 0; i < CH; ++i)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) mb = max(mb, __float_as_uint(v[i][e]) & 0x7fffffffu);
+#pragma unroll
+  for (int o = 32; o >= 1; o >>= 1) mb = max(mb, (uint32_t)__shfl_xor((int)mb, o));
+  if constexpr (T == 256) {
+    if ((threadIdx.x & 63) == 0) wave_max[threadIdx.x >> 6] = __uint_as_float(mb);
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 4; ++i) mb = max(mb, __float_as_uint(wave_max[i]));
+  }
+  const float s = split_scale(__uint_as_float(mb));
+  f16* dst = p.dst[which] + (int64_t)row * 2 * p.K;
+#pragma unroll
+  for (int i = 0; i < CH; ++i) {
+    const int c = (t + i * T) * 4;
+    if (c >= p.K) break;
+    f16x4 hi, lo;
+    split4(v[i], s, hi, lo);
+    store_split4(dst, c, hi, lo);
+  }
+  if (t == 0) p.inv[which][row] = mb < 0x7f800000u ? 1.0f / s : __uint_as_float(0x7fc00000u);
+}
+
+constexpr int kSplitMaxK = 8192;   // the longest row split_rows takes
+
+static int split_rows(const SplitRowsParams& p, hipStream_t stream) {
+  const int waves = (p.rows[0] + 3) / 4 + (p.rows[1] + 3) / 4, blocks = p.rows[0] + p.rows[1];
+  if (p.K <= 1024) hipLaunchKernelGGL((split_rows_kernel<64, 4>), dim3(waves), dim3(256), 0, stream, p);
+  else if (p.K <= 2048) hipLaunchKernelGGL((split_rows_kernel<64, 8>), dim3(waves), dim3(256), 0, stream, p);
+  else if (p.K <= 4096) hipLaunchKernelGGL((split_rows_kernel<256, 4>), dim3(blocks), dim3(256), 0, stream, p);
+  else hipLaunchKernelGGL((split_rows_kernel<256, 8>), dim3(blocks), dim3(256), 0, stream, p);
+  return check_launch("split_rows");
+}
+
+// ---------------------------------------------------------------------------------------------
+// GEMM on split rows.
+// ---------------------------------------------------------------------------------------------
+template <int BM, int BN, int WM, int WN>
+struct SplitShape {
+  static constexpr int THREADS = 64 * WM * WN;
+  static constexpr int TM = BM / WM, TN = BN / WN, MB = TM / 32, NB = TN / 32;
+  static constexpr int PASS = THREADS / 8;               // rows one DMA pass covers
+  static constexpr int XPT = BM / PASS, WPT = BN / PASS;
+  static constexpr int STAGE = (BM + BN) * 64;           // f16 elements of one stage
+  static_assert(BM % PASS == 0 && BN % PASS == 0 && TM % 32 == 0 && TN % 32 == 0, "tile shape");
+};
+
+// LDS element offset of (row, 16-byte chunk) in 128-byte rows, swizzled as in the bf16 GEMM: the 16 rows
+// one clock of a fragment read touches fall on 16 distinct bank groups.
+__device__ __forceinline__ int split_lds_off(int row, int chunk) { return row * 64 + ((chunk ^ ((row >> 1) & 7)) << 3); }
+
+// y[m, n..n+3] = epi(v + bias), v already scaled back.
+template <int EPI>
+__device__ __forceinline__ void split_store4(const GemmSplitParams& p, int m, int n, f32x4 v, const f32x4& bias) {
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    v[e] += bias[e];
+    if constexpr (EPI == kEpiBiasGelu) v[e] = gelu_tanh(v[e]);
+  }
+  if constexpr (EPI == kEpiBiasResidual) v += *reinterpret_cast<const f32x4*>(p.res + (int64_t)m * p.ldr + n);
+  *reinterpret_cast<f32x4*>(p.y + (int64_t)m * p.ldc + n) = v;
+}
+
+// acc 2^-(ex + ew): the smaller factor first, so that neither step leaves the range unless the result does
+// (sums below 1 in the scaled domain are rounding noise of products of up to 2^30).
+__device__ __forceinline__ f32x4 split_unscale(f32x4 v, float sx, const f32x4& sw) {
+#pragma unroll
+  for (int e = 0; e < 4; ++e) v[e] = v[e] * fminf(sx, sw[e]) * fmaxf(sx, sw[e]);
+  return v;
+}
+
+__device__ __forceinline__ bool any_nan(const f32x4& v) { return v[0] != v[0] || v[1] != v[1] || v[2] != v[2] || v[3] != v[3]; }
+
+// Outputs of a row or column that holds infinities or NaN (its scale is NaN), as the fp32 operands give them:
+// serial fp32 sums, left at the first NaN. Rare, so written small and not fast.
+template <int EPI>
+__device__ __forceinline__ void split_serial4(const GemmSplitParams& p, int m, int n, const f32x4& bias) {
+  f32x4 v;
+#pragma unroll 1
+  for (int e = 0; e < 4; ++e) {
+    const float *x = p.xf + (int64_t)m * p.ldx, *w = p.wf + (int64_t)(n + e) * p.K;
+    float a = 0.f;
+#pragma unroll 1
+    for (int k = 0; k < p.K && a == a; ++k) a = fmaf(x[k], w[k], a);
+    v[0] = e == 0 ? a : v[0]; v[1] = e == 1 ? a : v[1]; v[2] = e == 2 ? a : v[2]; v[3] = e == 3 ? a : v[3];
+  }
+  split_store4<EPI>(p, m, n, v, bias);
+}
+
+template <int BM, int BN, int WM, int WN, int NS, int EPI>
+__global__ __launch_bounds__(64 * WM * WN, 2) void gemm_split_kernel(GemmSplitParams p) {
+  using S = SplitShape<BM, BN, WM, WN>;
+  extern __shared__ __attribute__((aligned(16))) f16 smem_h[];   // [NS][BM + BN][64]
+  const int tiles_n = (p.N + BN - 1) / BN, tiles_m = (p.M + BM - 1) / BM;
+  const int tiles = tiles_m * tiles_n;
+  // split-K: the units of one K part are consecutive, so one XCD's units share operand rows
+  const int unit = xcd_remap(blockIdx.x, tiles * p.split);
+  const int tile = unit % tiles, part_i = unit / tiles;
+  int tm, tn;
+  tile_coords(tile, tiles_m, tiles_n, p.group_n, tm, tn);
+  const int m0 = tm * BM, n0 = tn * BN;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave % WM, wn = wave / WM;
+  const int l32 = lane & 31, hh = lane >> 5;
+
+  // Operand DMA, as in the bf16 GEMM: one wave instruction fills 8 LDS rows of 128 bytes; rows past M or N
+  // lie past the resource's range and arrive as zeros.
+  const int lrow = wave * 8 + (lane >> 3);
+  const int lch = (lane & 7) ^ ((lrow >> 1) & 7);
+  const uint32_t rowb = (uint32_t)p.K * 4;
+  const uint32_t xv = (uint32_t)(m0 + lrow) * rowb + lch * 16, wv = (uint32_t)(n0 + lrow) * rowb + lch * 16;
+  const u32x4 rx = rsrc_words(p.x, (uint32_t)p.M * rowb), rw = rsrc_words(p.w, (uint32_t)p.N * rowb);
+  const uint32_t lds_base = lds_addr_of(smem_h);
+  auto dma_stage = [&](int kt, int stage) {
+    const uint32_t xa = lds_base + stage * S::STAGE * 2, wa = xa + BM * 128;
+#pragma unroll
+    for (int i = 0; i < S::XPT; ++i)
+      dma16(rx, xv, (uint32_t)(i * S::PASS) * rowb + kt * 128, xa + (i * S::PASS + wave * 8) * 128);
+#pragma unroll
+    for (int i = 0; i < S::WPT; ++i)
+      dma16(rw, wv, (uint32_t)(i * S::PASS) * rowb + kt * 128, wa + (i * S::PASS + wave * 8) * 128);
+  };
+  const int KT = p.K / 32;
+  const int kt0 = part_i * KT / p.split, kt1 = (part_i + 1) * KT / p.split;
+#pragma unroll
+  for (int s = 0; s < NS - 1; ++s)
+    if (kt0 + s < kt1) dma_stage(kt0 + s, s);
+
+  // The hi . hi products and (where the registers hold both) the 2^-11 smaller cross products in accumulators of
+  // their own: the large sums then round K / 16 times and not 3 K / 16.
+  constexpr bool TWO = S::NB * S::MB <= 4;
+  f32x16 acc[S::NB][S::MB], low[TWO ? S::NB : 1][TWO ? S::MB : 1];
+#pragma unroll
+  for (int a = 0; a < S::NB; ++a)
+#pragma unroll
+    for (int b = 0; b < S::MB; ++b) {
+      acc[a][b] = f32x16{};
+      if constexpr (TWO) low[a][b] = f32x16{};
+    }
+
+  // Half step h of a k-step (16 of its 32 values): hi fragments in chunks 2h + hh, lo in 4 + 2h + hh.
+  constexpr int NFR = S::NB + S::MB;
+  f16x8 fh[2][NFR], fl[2][NFR];
+  auto read_frags = [&](const f16* xs, int h, int slot) {
+    const f16* ws = xs + BM * 64;
+    const int ch = 2 * h + hh;
+#pragma unroll
+    for (int a = 0; a < S::NB; ++a) {
+      fh[slot][a] = *reinterpret_cast<const f16x8*>(ws + split_lds_off(wn * S::TN + a * 32 + l32, ch));
+      fl[slot][a] = *reinterpret_cast<const f16x8*>(ws + split_lds_off(wn * S::TN + a * 32 + l32, ch + 4));
+    }
+#pragma unroll
+    for (int b = 0; b < S::MB; ++b) {
+      fh[slot][S::NB + b] = *reinterpret_cast<const f16x8*>(xs + split_lds_off(wm * S::TM + b * 32 + l32, ch));
+      fl[slot][S::NB + b] = *reinterpret_cast<const f16x8*>(xs + split_lds_off(wm * S::TM + b * 32 + l32, ch + 4));
+    }
+  };
+  auto mfmas = [&](int slot) {
+    const f16x8 *wh = fh[slot], *wl = fl[slot], *xh = fh[slot] + S::NB, *xl = fl[slot] + S::NB;
+    auto products = [&](const f16x8* w, const f16x8* x, auto& sum) {
+#pragma unroll
+      for (int a = 0; a < S::NB; ++a)
+#pragma unroll
+        for (int b = 0; b < S::MB; ++b) sum[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(w[a], x[b], sum[a][b], 0, 0, 0);
+    };
+    if constexpr (TWO) {
+      products(wl, xh, low);
+      products(wh, xl, low);
+    } else {
+      products(wl, xh, acc);
+      products(wh, xl, acc);
+    }
+    products(wh, xh, acc);
+  };
+  constexpr int NMF = 3 * S::NB * S::MB;
+  auto wait_stage = [&](int kt) {   // every stage up to kt has landed (later ones may be in flight)
+    if (NS == 3 && kt + 1 < kt1) asm volatile("s_waitcnt vmcnt(%0)" :: "I"(S::XPT + S::WPT) : "memory");
+    else wait_dma();
+  };
+
+  wait_stage(kt0);
+  __syncthreads();
+  read_frags(smem_h, 0, 0);
+  int cur = 0;
+  for (int kt = kt0; kt < kt1; ++kt) {
+    const f16* xs = smem_h + cur * S::STAGE;
+    const bool more = kt + 1 < kt1;
+    const int nxt = cur + 1 == NS ? 0 : cur + 1;
+    if (kt + NS - 1 < kt1) dma_stage(kt + NS - 1, NS == 3 ? (cur == 0 ? 2 : cur - 1) : nxt);
+    read_frags(xs, 1, 1);
+    mfmas(0);
+#pragma unroll
+    for (int i = 0; i < NMF; ++i) {
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+      if (i < 2 * NFR) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+    }
+    mfmas(1);
+    wait_stage(kt + 1);
+    __syncthreads();
+    if (more) read_frags(smem_h + nxt * S::STAGE, 0, 0);
+    cur = nxt;
+  }
+
+  if constexpr (TWO) {
+#pragma unroll
+    for (int a = 0; a < S::NB; ++a)
+#pragma unroll
+      for (int b = 0; b < S::MB; ++b) acc[a][b] += low[a][b];
+  }
+
+  // Epilogue. Accumulator (a, b), register 4 g + e: token 32 b + l32, feature 32 a + 8 g + 4 hh + e of the
+  // wave's sub-tile. Each wave turns 32 tokens at a time through its own piece of the free ring (16-byte
+  // chunks XOR-swizzled by row), so that stores go out as whole TN-wide row pieces; no barrier is needed
+  // within a wave. A K part stores its raw sums.
+  constexpr int CH = S::TN / 4, RPI = 64 / CH;            // 16-byte chunks of a row, rows one read covers
+  float* stage = reinterpret_cast<float*>(smem_h) + wave * 32 * S::TN;
+  static_assert(WM * WN * 32 * S::TN * 4 <= NS * S::STAGE * 2 && 64 % CH == 0, "epilogue staging");
+  const int c = lane % CH, n = n0 + wn * S::TN + 4 * c;
+  const bool nok = n < p.N;
+  f32x4 sw = {}, bias = {};
+  if (p.split == 1 && nok) {
+    sw = *reinterpret_cast<const f32x4*>(p.sw + n);
+    bias = *reinterpret_cast<const f32x4*>(p.bias + n);
+  }
+  const bool w_nan = any_nan(sw);
+  const int64_t npad = (int64_t)tiles_n * BN;
+#pragma unroll
+  for (int b = 0; b < S::MB; ++b) {
+#pragma unroll
+    for (int a = 0; a < S::NB; ++a)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const int cc = 8 * a + 2 * g + hh;
+        *reinterpret_cast<f32x4*>(stage + l32 * S::TN + ((cc ^ (l32 % CH)) << 2)) =
+            f32x4{acc[a][b][4 * g], acc[a][b][4 * g + 1], acc[a][b][4 * g + 2], acc[a][b][4 * g + 3]};
+      }
+#pragma unroll
+    for (int i = 0; i < 32 / RPI; ++i) {
+      const int r = i * RPI + lane / CH, m = m0 + wm * S::TM + 32 * b + r;
+      const f32x4 v = *reinterpret_cast<const f32x4*>(stage + r * S::TN + ((c ^ (r % CH)) << 2));
+      if (m >= p.M) continue;
+      if (p.split > 1)
+        *reinterpret_cast<f32x4*>(p.part + ((int64_t)part_i * p.M + m) * npad + n) = v;
+      else if (nok) {
+        const float sx = p.sx[m];
+        if (sx == sx && !w_nan) split_store4<EPI>(p, m, n, split_unscale(v, sx, sw), bias);
+      }
+    }
+  }
+  if (p.split > 1 || !nok) return;
+#pragma unroll 1
+  for (int r = lane / CH; r < S::TM; r += RPI) {
+    const int m = m0 + wm * S::TM + r;
+    if (m >= p.M) break;
+    if (w_nan || p.sx[m] != p.sx[m]) split_serial4<EPI>(p, m, n, bias);
+  }
+}
+
+// Sums the K parts in order and applies the epilogue, one thread per 4 consecutive outputs.
+template <int EPI>
+__global__ __launch_bounds__(256) void gemm_split_reduce_kernel(GemmSplitParams p, int64_t npad) {
+  const int64_t q = (int64_t)blockIdx.x * 256 + threadIdx.x, quads = (int64_t)p.M * (p.N / 4);
+  if (q >= quads) return;
+  const int m = (int)(q / (p.N / 4)), n = (int)(q % (p.N / 4)) * 4;
+  const float* src = p.part + (int64_t)m * npad + n;
+  const int64_t stride = (int64_t)p.M * npad;
+  f32x4 v = *reinterpret_cast<const f32x4*>(src);
+  for (int s = 1; s < p.split; ++s) v += *reinterpret_cast<const f32x4*>(src + s * stride);
+  const f32x4 sw = *reinterpret_cast<const f32x4*>(p.sw + n), bias = *reinterpret_cast<const f32x4*>(p.bias + n);
+  const float sx = p.sx[m];
+  if (sx == sx && !any_nan(sw)) split_store4<EPI>(p, m, n, split_unscale(v, sx, sw), bias);
+  else split_serial4<EPI>(p, m, n, bias);
+}
+
+template <int BM, int BN, int WM, int WN, int NS, int EPI>
+static int launch_gemm_split(GemmSplitParams p, int split, hipStream_t stream) {
+  using S = SplitShape<BM, BN, WM, WN>;
+  constexpr int lds = NS * S::STAGE * 2;
+  static_assert(lds <= 163840, "LDS budget");
+  static const hipError_t attr = hipFuncSetAttribute((const void*)gemm_split_kernel<BM, BN, WM, WN, NS, EPI>,
+                                                     hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+  if (attr != hipSuccess) return set_error(QVL_ERR_LAUNCH, "gemm_split: cannot reserve %d bytes of LDS", lds);
+  const int tiles_n = (p.N + BN - 1) / BN, tiles = ((p.M + BM - 1) / BM) * tiles_n;
+  const int64_t npad = (int64_t)tiles_n * BN;
+  p.split = split;
+  p.group_n = std::min(4, tiles_n);
+  hipLaunchKernelGGL((gemm_split_kernel<BM, BN, WM, WN, NS, EPI>), dim3(tiles * p.split), dim3(S::THREADS), lds, stream, p);
+  int rc = check_launch("gemm_split");
+  if (rc || p.split == 1) return rc;
+  const int64_t blocks = ((int64_t)p.M * (p.N / 4) + 255) / 256;
+  hipLaunchKernelGGL(gemm_split_reduce_kernel<EPI>, dim3((unsigned)blocks), dim3(256), 0, stream, p, npad);
+  return check_launch("gemm_split_reduce");
+}
+
+// Tile plan of the calling thread (qvl_set_f32_plan): 0 = the rules below, 1..4 = kSplitTiles[tile - 1],
+// 5 = the fp32 MFMA kernel.
+static thread_local int t_f32_plan = 0;
+
+int gemm_f32_set_plan(int tile) {
+  if (tile < 0 || tile > 5) return set_error(QVL_ERR_INVALID_ARG, "f32 plan: tile=%d (0..5)", tile);
+  t_f32_plan = tile;
+  return QVL_OK;
+}
+
+// Tile and K split by a cost model of the launch, in microseconds: start + rounds * (K / split * per_k +
+// per_tile), rounds = workgroups per CU, where a last partial round costs its share of the CUs but at least
+// `part` of a round, and a launch of less than one round at least `one`; split-K adds its partials' traffic at
+// part_rate bytes/us. Fitted to 45 shapes from 49 to 18432 rows (MI355X, cold weights, every tile): what it
+// picks is 2 % slower than the best measured choice on average, 17 % at worst. For instance
+// 784 x 3072 x 1024 runs in 34 us, 8192 x 4096 x 1024 in 189 us (1.09 PFLOP/s of f16 products; 609 us on
+// v_mfma_f32_32x32x2_f32), 8192 x 1024 x 4096 in 181 us (365 us).
+struct SplitTile { int bm, bn, slots; double start, per_k, per_tile, part, one, part_rate; };   // slots: workgroups a CU holds
+constexpr SplitTile kSplitTiles[] = {
+    {64, 128, 3, 11.7, 14.1 / 1024, 0.0, 0.25, 1.20, 17.9e6},     // two-stage ring, 48 KB
+    {64, 128, 2, 5.1, 13.3 / 1024, 2.0, 0.81, 1.13, 6.9e6},       // three stages, 72 KB
+    {128, 256, 1, 0.2, 43.1 / 1024, 10.3, 0.88, 0.73, 8.0e6},     // three stages, 144 KB
+    {256, 256, 1, 0.0, 81.8 / 1024, 11.3, 0.86, 0.74, 7.9e6},     // two stages, 128 KB
+};
+
+static double split_cost(const SplitTile& t, const GemmSplitParams& p, int cus, int split) {
+  const int units = ((p.M + t.bm - 1) / t.bm) * ((p.N + t.bn - 1) / t.bn) * split;
+  const int tail = units % cus;
+  double rounds = units / cus + (tail ? std::max((double)tail / cus, t.part) : 0.0);
+  if (units < cus) rounds = std::max(rounds, t.one);
+  return t.start + rounds * (p.K / (double)split * t.per_k + t.per_tile) +
+         (split > 1 ? 8.0 * split * p.M * p.N / t.part_rate : 0.0);
+}
+
+template <int EPI>
+static int dispatch_gemm_split(const GemmSplitParams& p, hipStream_t stream) {
+  const int cus = gemm_device_cus();
+  int pick = 0, split = 1;
+  double best = 1e30;
+  for (int i = 0; i < 4; ++i) {
+    if (t_f32_plan >= 1 && t_f32_plan <= 4 && i != t_f32_plan - 1) continue;
+    // (256x256 tiles add every product to one accumulator, 3 K / 16 roundings: nearer to float64 than the fp32
+    // MFMA kernel where that does not split K, which is where its 128x128 tiles outnumber the CUs)
+    if (i == 3 && !t_f32_plan && ((p.M + 127) / 128) * ((p.N + 127) / 128) <= cus) continue;
+    const SplitTile& t = kSplitTiles[i];
+    const int tiles = ((p.M + t.bm - 1) / t.bm) * ((p.N + t.bn - 1) / t.bn);
+    const int64_t npad = round_up(p.N, t.bn);
+    for (int s = 1; s <= std::min(8, p.K / 32 / 4) || s == 1; ++s) {
+      if (s > 1 && (!p.part || (int64_t)s * p.M * npad > p.part_elems || tiles * s > t.slots * cus)) break;
+      const double c = split_cost(t, p, cus, s);
+      if (c < best) { best = c; pick = i; split = s; }
+    }
+  }
+  switch (pick) {
+    case 0: return launch_gemm_split<64, 128, 2, 2, 2, EPI>(p, split, stream);
+    case 1: return launch_gemm_split<64, 128, 2, 2, 3, EPI>(p, split, stream);
+    case 2: return launch_gemm_split<128, 256, 2, 4, 3, EPI>(p, split, stream);
+    default: return launch_gemm_split<256, 256, 4, 2, 2, EPI>(p, split, stream);
+  }
+}
+
+int gemm_split(const GemmSplitParams& p, int epi, hipStream_t stream) {
+  switch (epi) {
+    case kEpiBias: return dispatch_gemm_split<kEpiBias>(p, stream);
+    case kEpiBiasGelu: return dispatch_gemm_split<kEpiBiasGelu>(p, stream);
+    case kEpiBiasResidual: return dispatch_gemm_split<kEpiBiasResidual>(p, stream);
+  }
+  return set_error(QVL_ERR_INVALID_ARG, "gemm_split: epilogue %d", epi);
+}
+
+// Splits x [M, K] and w [N, K] into the front of the workspace (g.part) and runs the Dense on them; what is
+// left of the workspace takes split-K partials.
+static int64_t split_scales(int64_t M, int64_t N) { return round_up(M, 4) + round_up(N, 4); }
+
+// Whether a Dense whose operands are both fp32 runs on split rows: the workspace holds them, and splitting the
+// weights (N K values, read and written for this one call) pays. It does not for a few rows over many short
+// ones, where the fp32 MFMA kernel's time is one tile's K loop: 32 rows x 4096 x 1024 20.0 us against 20.8
+// (1: 17.9 against 23.1, 49: 21.7 against 22.2, 100: 25.8 against 24.0), 32 x 3072 x 1024 19.5 against 20.6;
+// but 32 x 1024 x 1024 18.2 against 14.9, 32 x 1024 x 4096 51.2 against 25.8, 32 x 4352 x 1152 30.9 against 21.8.
+bool gemm_f32_use_split(const GemmF32Params& g) {
+  if (t_f32_plan == 5 || !g.part || g.K > kSplitMaxK ||
+      g.part_elems < split_scales(g.M, g.N) + ((int64_t)g.M + g.N) * g.K)
+    return false;
+  return t_f32_plan != 0 || g.M > 64 || g.K > 1024 || g.N <= 2 * g.K;
+}
+
+int gemm_f32_split(const GemmF32Params& g, int epi, hipStream_t stream) {
+  const int64_t M = g.M, N = g.N, K = g.K, head = split_scales(M, N), used = head + (M + N) * K;
+  SplitRowsParams r{};
+  r.src[0] = g.x; r.ld[0] = g.lda; r.dst[0] = (f16*)(g.part + head); r.inv[0] = g.part; r.rows[0] = g.M;
+  r.src[1] = g.w; r.ld[1] = g.ldw; r.dst[1] = r.dst[0] + 2 * M * K; r.inv[1] = g.part + round_up(M, 4); r.rows[1] = g.N;
+  r.K = g.K;
+  QVL_TRY_RC(split_rows(r, stream));
+  GemmSplitParams p{};
+  p.x = r.dst[0]; p.sx = r.inv[0]; p.w = r.dst[1]; p.sw = r.inv[1];
+  p.bias = g.bias; p.res = g.res; p.ldr = g.ldr; p.y = g.y; p.ldc = g.ldc;
+  p.M = g.M; p.N = g.N; p.K = g.K;
+  p.xf = g.x; p.ldx = g.lda; p.wf = g.w;
+  p.part = g.part + used;          // (K is a multiple of 64: `used` is a multiple of 4)
+  p.part_elems = g.part_elems - used;
+  return gemm_split(p, epi, stream);
+}
+
+}  // namespace qvl

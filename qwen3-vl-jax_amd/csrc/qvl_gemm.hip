@@ -702,19 +702,6 @@ __device__ __forceinline__ void gemm_epilogue_rope72_lds(const GemmParams& p,
   }
 }
 
-// Tile t -> (row tile, column tile). Tiles are ordered in panels of group_n column tiles, row tile
-// by row tile within a panel, so the tiles that one XCD runs in one round (a contiguous range, see
-// xcd_remap) form a block of about (cus/8)/group_n row tiles by group_n column tiles, and the
-// operand bytes that XCD's L2 fetches per round are ~rows*|x tile| + cols*|w tile| instead of the
-// whole weight matrix (row-major order puts all column tiles of 2 row tiles in one round).
-__device__ __forceinline__ void tile_coords(int tile, int tiles_m, int tiles_n, int group_n, int& tm, int& tn) {
-  const int panel = tile / (tiles_m * group_n);
-  const int width = min(group_n, tiles_n - panel * group_n);
-  const int r = tile - panel * tiles_m * group_n;
-  tm = r / width;
-  tn = panel * group_n + r % width;
-}
-
 // Dynamic LDS of the GEMM. Elements [0, E): the operand ring (`stages` stages) or the epilogue
 // staging, whichever is larger. Above it: for a folded LayerNorm (LN kernels) the tile's BN columns'
 // (c, d) then its BM rows' (rstd, -mean * rstd), 8 bytes each; then the rotary epilogues'

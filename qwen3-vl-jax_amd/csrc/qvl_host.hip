@@ -71,6 +71,7 @@ static int dense_impl(void* stream, int32_t dtype, int32_t epi, const void* x, i
     p.bias = bias; p.res = (const float*)res; p.ldr = ldr; p.y = (float*)y; p.ldc = ldc;
     p.M = (int)m; p.N = (int)n; p.K = (int)k; p.Kp = (int)k;
     p.part = (float*)ws; p.part_elems = ws ? (int64_t)(ws_bytes / sizeof(float)) : 0;
+    if (gemm_f32_use_split(p)) return gemm_f32_split(p, epi, (hipStream_t)stream);
     return gemm_f32(p, epi, (hipStream_t)stream);
   }
   if (!aligned16(x) || !aligned16(w) || !aligned16(bias) || !aligned16(y) || lda % 8 || ldc % 4 ||
@@ -100,6 +101,8 @@ int qvl_dense(void* stream, int32_t dtype, int32_t epi, const void* x, int64_t l
 int qvl_set_gemm_plan(int32_t tile, int32_t split_mode, int32_t group_n) {
   return gemm_set_plan(tile, split_mode, group_n);
 }
+
+int qvl_set_f32_plan(int32_t tile) { return gemm_f32_set_plan(tile); }
 
 int qvl_set_attention_plan(int32_t key_groups) { return attention_set_plan(key_groups); }
 

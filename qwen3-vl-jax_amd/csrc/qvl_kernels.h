@@ -79,6 +79,21 @@ struct GemmF32Params {
   int split;
 };
 
+// fp32 Dense on two-way f16 split operands (qvl_f32_split.hip): x [M] and w [N] rows of K / 32 groups of
+// [32 hi | 32 lo] f16, sx / sw the rows' factors back to their fp32 values (NaN: a row that holds an infinity
+// or a NaN; its outputs are computed from xf [M, ldx] and wf [N, K] in fp32).
+struct GemmSplitParams {
+  const _Float16* x; const float* sx;
+  const _Float16* w; const float* sw;
+  const float* bias;
+  const float* res; int64_t ldr;   // residual, may alias y
+  float* y; int64_t ldc;
+  int M, N, K;
+  const float* xf; int64_t ldx; const float* wf;
+  float* part; int64_t part_elems; // split-K partials (set up by the launcher, as in GemmF32Params)
+  int split, group_n;
+};
+
 // Floats of split-K partial workspace that lets every GEMM of up to 256x256 tiles split its tail
 // on a device with `cus` compute units (one tail unit per CU, at most one tile of partials each).
 inline int64_t gemm_partials_elems(int cus) { return (int64_t)cus * 256 * 256; }
@@ -127,6 +142,9 @@ int rotary_table(const int* pos_hw, int n_tok, int head_dim, const float* inv_fr
                  hipStream_t stream);
 int cast_f32_bf16(const float* x, bf16* y, int64_t n, hipStream_t stream);
 int gemm_f32(GemmF32Params p, int epi, hipStream_t stream);
+bool gemm_f32_use_split(const GemmF32Params& g);
+int gemm_f32_split(const GemmF32Params& g, int epi, hipStream_t stream);
+int gemm_f32_set_plan(int tile);
 int layer_norm_f32(const float* x, int64_t ldx, const float* g, const float* b, float* y, int64_t ldy, int rows,
                    int cols, float eps, hipStream_t stream);
 int pos_embed_f32(const float* table, const int* idx, const float* wts, float* y, int n_tok, int dim,

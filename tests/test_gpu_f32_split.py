@@ -1,0 +1,106 @@
+"""The fp32 Dense on f16-split operands (qvl_dense_ws) against float64, tile by tile."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+torch = pytest.importorskip("torch")
+pytestmark = pytest.mark.gpu
+
+DEV = "cuda:0"
+
+
+@pytest.fixture
+def dense(pkg, lib):
+    """dense(plan, x, w, b, epi, r) -> y on torch fp32 tensors; w [N rounded up to 64, K]."""
+    cp = pkg.capi
+    nb = C.c_size_t()
+    cp.check(lib.qvl_dense_workspace_size(C.byref(nb)))
+    ws = torch.empty(nb.value, dtype=torch.uint8, device=DEV)
+
+    def run(plan, x, w, b, epi=0, r=None):
+        (M, K), N = x.shape, b.shape[0]
+        y = r.clone() if r is not None else torch.empty((M, N), device=DEV)      # the residual in place
+        cp.check(lib.qvl_set_f32_plan(plan))
+        cp.check(lib.qvl_dense_ws(torch.cuda.current_stream().cuda_stream, cp.QVL_DTYPE_F32, epi, x.data_ptr(), K,
+                                  w.data_ptr(), b.data_ptr(), y.data_ptr() if r is not None else None, N, y.data_ptr(),
+                                  N, M, N, K, ws.data_ptr(), nb.value))
+        return y
+    yield run
+    cp.check(lib.qvl_set_f32_plan(0))
+
+
+def operands(M, N, K, seed):
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    x = torch.randn((M, K), generator=g, device=DEV)
+    w = torch.zeros((-(-N // 64) * 64, K), device=DEV)
+    w[:N] = torch.randn((N, K), generator=g, device=DEV) * 0.05
+    b = torch.randn(N, generator=g, device=DEV)
+    return x, w, b, torch.randn((M, N), generator=g, device=DEV)
+
+
+def bound(x, w, N, K):
+    """|error| per element: the terms an f16 split drops (3 products of 2^-22 of |x w|), then one rounding of the
+    running sum, at most sum |x w|, per accumulation step (3 K / 16) and K part."""
+    s = x.abs().double() @ w[:N].abs().double().t()
+    return s * (3 * 2.0 ** -22 + (3 * K / 16 + 16) * 2.0 ** -24)
+
+
+# edges of the 64 / 128 / 256 tiles, one k-step pair (K = 64) and split-K (K >= 256), one row, one 4-column group
+@pytest.mark.parametrize("plan", [1, 2, 3, 4])
+@pytest.mark.parametrize("M,N,K", [(1, 4, 64), (63, 132, 64), (64, 128, 192), (65, 252, 256), (129, 256, 1024),
+                                   (257, 260, 320), (300, 1152, 4352), (31, 64, 8192)])
+def test_split_dense_vs_fp64(dense, plan, M, N, K):
+    x, w, b, r = operands(M, N, K, M + N + K)
+    ref = x.double() @ w[:N].double().t() + b.double()
+    tol = bound(x, w, N, K) + ref.abs() * 2.0 ** -23
+    assert torch.all((dense(plan, x, w, b).double() - ref).abs() <= tol)
+    y = dense(plan, x, w, b, 2, r)
+    assert torch.all((y.double() - ref - r.double()).abs() <= tol + (ref.abs() + r.abs()) * 2.0 ** -23)
+    # GELU: slope at most 1.13; its own fp32 arithmetic (exp2, reciprocal) within 4e-6 of max(|y|, 1)
+    y = dense(plan, x, w, b, 1)
+    gelu = torch.nn.functional.gelu(ref, approximate="tanh")
+    assert torch.all((y.double() - gelu).abs() <= 1.13 * tol + 4e-6 * gelu.abs().clamp(min=1.0))
+
+
+@pytest.mark.parametrize("M,N,K", [(784, 1024, 1024), (300, 512, 4096), (2304, 3072, 1024)])
+def test_split_dense_is_nearer_to_fp64_than_fp32_mfma(dense, M, N, K):
+    x, w, b, _ = operands(M, N, K, K)
+    ref = x.double() @ w.double().t() + b.double()
+    err = [((dense(p, x, w, b).double() - ref).norm() / ref.norm()).item() for p in (0, 1, 2, 3, 5)]
+    assert max(err[:4]) <= err[4], err
+
+
+def test_split_dense_row_scales(dense):
+    """Rows of every magnitude keep their relative error: the split's exponent is per row (of x and of w)."""
+    M, N, K = 130, 128, 256
+    x, w, b, _ = operands(M, N, K, 3)
+    b.zero_()
+    x *= (10.0 ** torch.linspace(-30, 18, M, device=DEV))[:, None]
+    w *= (10.0 ** torch.linspace(-7, 18, N, device=DEV))[:, None]
+    x[5], x[6, 1:], w[7] = 0.0, 0.0, 0.0
+    ref = x.double() @ w.double().t()
+    for plan in (1, 2, 3, 4):
+        y = dense(plan, x, w, b).double()
+        assert torch.all((y - ref).abs() <= bound(x, w, N, K))
+        assert not y[5].any() and not y[:, 7].any()
+
+
+@pytest.mark.parametrize("K", [128, 2048])          # without and with split-K
+def test_split_dense_infinities_and_nan(dense, K):
+    """Rows and weights that hold infinities or NaN give what the fp32 MFMA kernel gives; the others stay exact."""
+    M, N = 140, 192
+    x, w, b, r = operands(M, N, K, 7)
+    inf, nan = float("inf"), float("nan")
+    x[3, 7], x[9, 1], x[64, 5], x[64, 6], x[139, K - 1] = inf, nan, inf, -inf, -inf
+    w[5, 3], w[100, 2], w[8] = -inf, nan, w[8].bfloat16().float()      # (row 8's lo terms are zeros)
+    w[11, 7] = 0.0                                                      # inf * 0
+    for epi in (0, 1, 2):
+        want = dense(5, x, w, b, epi, r if epi == 2 else None)
+        for plan in (1, 2, 3, 4):
+            got = dense(plan, x, w, b, epi, r if epi == 2 else None)
+            assert torch.equal(torch.isnan(got), torch.isnan(want))
+            inf_at = torch.isinf(want)
+            assert torch.equal(got[inf_at], want[inf_at]) and torch.equal(torch.isinf(got), inf_at)
+            fine = torch.isfinite(want)
+            assert torch.allclose(got[fine], want[fine], rtol=1e-4, atol=1e-4)
