@@ -406,6 +406,30 @@ typedef struct qvl_vision_weights {
   const qvl_merger_weights* deepstack;       /* HOST array [n_deepstack]                       */
 } qvl_vision_weights;
 
+/* The fp32 tower's Dense weights once more as f16-split rows (two f16 terms per value, a power-of-two factor
+ * per row; 4 bytes a value, as the fp32 weights), made once when a tower is bound, so that the forward's Dense
+ * layers run on the f16 matrix cores without splitting the weights each time (qvl_dense_ws does that).
+ * bound: device floats, upper bounds on |output| of a Dense that follows a LayerNorm, whatever its input is:
+ * one per group of output rows (3 for qkv: q, k, v); unused for proj, fc2 and the patch embed. */
+typedef struct qvl_split_dense { const void* w; const float* scale; const float* bound; } qvl_split_dense;
+typedef struct qvl_split_block { qvl_split_dense qkv, proj, fc1, fc2; } qvl_split_block;
+typedef struct qvl_split_merger { qvl_split_dense fc1, fc2; } qvl_split_merger;
+typedef struct qvl_vision_split {
+  qvl_split_dense patch;
+  const qvl_split_block* blocks;             /* HOST array [depth]       */
+  qvl_split_merger merger;
+  const qvl_split_merger* deepstack;         /* HOST array [n_deepstack] */
+} qvl_vision_split;
+
+/* Split one packed fp32 weight [n_out][k_in] (k_in a multiple of 64, at most 8192): d_out_w [n_out][2 k_in] f16,
+ * d_out_scale [n_out] fp32. d_out_bound [groups + n_out] fp32: the largest sqrt(k_in) |gamma w_n| +
+ * |beta . w_n| + |bias_n| of each of `groups` equal groups of rows, then every row's; gamma / beta
+ * [ln_cols] (a multiple of 4) repeat along the row (NULL: 1 / 0). A non-finite bound (weights that hold infinities or NaN, or
+ * whose norms overflow) means the split must not be used. */
+int qvl_split_dense_weight(void* stream, const float* d_w, int64_t k_in, int64_t n_out, const float* d_bias,
+                           const float* d_gamma, const float* d_beta, int64_t ln_cols, int32_t groups,
+                           void* d_out_w, float* d_out_scale, float* d_out_bound);
+
 /* Window-attention metadata (model.py:769-799 `_get_window_index`, host side, bit-exact):
  * window_index [n_tokens/merge^2]: the merge group at each position of the window order (windows
  * of vit = window_size/merge/patch_size groups square, row-major per frame, groups row-major inside
@@ -458,6 +482,13 @@ int qvl_encode_vision(void* stream, const qvl_vision_config* cfg, const qvl_visi
                       const qvl_vision_metadata_dev* meta, const float* d_pixel_values,
                       void* d_tokens, void* const* d_deepstack, void* d_workspace,
                       size_t workspace_bytes);
+
+/* qvl_encode_vision for an fp32 tower (cfg->dtype QVL_DTYPE_F32; patch, MLP and 4 * hidden widths up to 8192)
+ * with its weights split beforehand: the same workspace size and results, nearer to float64. */
+int qvl_encode_vision_split(void* stream, const qvl_vision_config* cfg, const qvl_vision_weights* weights,
+                            const qvl_vision_split* split, const qvl_vision_metadata_dev* meta,
+                            const float* d_pixel_values, void* d_tokens, void* const* d_deepstack,
+                            void* d_workspace, size_t workspace_bytes);
 
 /* ------------------------------------------------------------------------------------------ */
 /* The steps either side of the tower: patchify before it, decoder-side injection after it.    */

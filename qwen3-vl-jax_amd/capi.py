@@ -56,6 +56,23 @@ class VisionWeights(C.Structure):
                 ("merger", MergerWeights), ("deepstack", C.POINTER(MergerWeights))]
 
 
+class SplitDense(C.Structure):
+    _fields_ = [("w", _p), ("scale", _p), ("bound", _p)]
+
+
+class SplitBlock(C.Structure):
+    _fields_ = [("qkv", SplitDense), ("proj", SplitDense), ("fc1", SplitDense), ("fc2", SplitDense)]
+
+
+class SplitMerger(C.Structure):
+    _fields_ = [("fc1", SplitDense), ("fc2", SplitDense)]
+
+
+class VisionSplit(C.Structure):
+    _fields_ = [("patch", SplitDense), ("blocks", C.POINTER(SplitBlock)), ("merger", SplitMerger),
+                ("deepstack", C.POINTER(SplitMerger))]
+
+
 class VisionMetadataDev(C.Structure):
     _fields_ = [("n_tokens", _i64), ("n_tiles", _i64), ("pos_hw", _p), ("tap_idx", _p), ("tap_w", _p),
                 ("tiles", _p), ("n_window_tiles", _i64), ("window_tiles", _p), ("window_index", _p),
@@ -115,6 +132,9 @@ SIGNATURES = {
     "qvl_encode_vision_workspace_size": (C.c_int, [C.POINTER(VisionConfig), _i64, C.POINTER(_sz)]),
     "qvl_encode_vision": (C.c_int, [_p, C.POINTER(VisionConfig), C.POINTER(VisionWeights),
                                     C.POINTER(VisionMetadataDev), _p, _p, C.POINTER(_p), _p, _sz]),
+    "qvl_encode_vision_split": (C.c_int, [_p, C.POINTER(VisionConfig), C.POINTER(VisionWeights), C.POINTER(VisionSplit),
+                                          C.POINTER(VisionMetadataDev), _p, _p, C.POINTER(_p), _p, _sz]),
+    "qvl_split_dense_weight": (C.c_int, [_p, _p, _i64, _i64, _p, _p, _p, _i64, _i32, _p, _p, _p]),
     "qvl_window_metadata": (C.c_int, [_pi32, _i64, _i32, _i32, _i32, _pi32, _pi32, _i64, C.POINTER(_i64), _pi32]),
     "qvl_gather_rows": (C.c_int, [_p, _i32, _p, _i64, _i32, _p, _i64, _p, _i64, _i32, _i64]),
     "qvl_patchify": (C.c_int, [_p, _i32, _p, _i64, _i64, _i64, _i32, _i32, _i32, _i32, _p, _i64]),

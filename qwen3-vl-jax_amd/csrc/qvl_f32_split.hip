@@ -16,36 +16,39 @@
 
 #include <algorithm>
 
-#include "qvl_kernels.h"
+#include "qvl_split.h"
 
 namespace qvl {
 
-typedef _Float16 f16;
-typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
-typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
-
-// The power of two that takes values up to `mx` (finite, >= 0) into f16 range: mx * s in [2^14, 2^15).
-// Clamped to normal fp32 values of s and 1 / s; zero and non-finite maxima give 1.
-__device__ __forceinline__ float split_scale(float mx) {
-  const int ex = (int)(__float_as_uint(mx) >> 23);   // biased exponent (mx >= 0); 0: zero or denormal
-  if (ex == 0 || ex == 255) return mx > 0.f && ex == 0 ? 0x1p126f : 1.0f;
-  return __uint_as_float((uint32_t)min(127 + 14 - (ex - 127), 253) << 23);
-}
-
-__device__ __forceinline__ void split4(const f32x4& v, float s, f16x4& hi, f16x4& lo) {
+// The sum, or the maximum of the bits, over the threads of a row (T = 64: a wave; 256: the workgroup, through
+// 4 floats of LDS).
+template <int T>
+__device__ __forceinline__ float row_sum(float v, float* tmp) {
 #pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    const float t = v[e] * s;
-    hi[e] = (f16)t;
-    lo[e] = (f16)(t - (float)hi[e]);
+  for (int o = 32; o >= 1; o >>= 1) v += __shfl_xor(v, o);
+  if constexpr (T > 64) {
+    __syncthreads();
+    if ((threadIdx.x & 63) == 0) tmp[threadIdx.x >> 6] = v;
+    __syncthreads();
+    v = (tmp[0] + tmp[1]) + (tmp[2] + tmp[3]);
   }
+  return v;
 }
 
-// Writes columns c..c+3 (c a multiple of 4) of a split row.
-__device__ __forceinline__ void store_split4(f16* row, int c, const f16x4& hi, const f16x4& lo) {
-  f16* g = row + (c >> 5) * 64 + (c & 31);
-  *reinterpret_cast<f16x4*>(g) = hi;
-  *reinterpret_cast<f16x4*>(g + 32) = lo;
+__device__ __forceinline__ uint32_t wave_max_bits(uint32_t m) {
+#pragma unroll
+  for (int o = 32; o >= 1; o >>= 1) m = max(m, (uint32_t)__shfl_xor((int)m, o));
+  return m;
+}
+
+__device__ __forceinline__ uint32_t block_max_bits(uint32_t m, float* tmp) {
+  m = wave_max_bits(m);
+  __syncthreads();
+  if ((threadIdx.x & 63) == 0) tmp[threadIdx.x >> 6] = __uint_as_float(m);
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < 4; ++i) m = max(m, __float_as_uint(tmp[i]));
+  return m;
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -66,7 +69,7 @@ struct SplitRowsParams {
 template <int T, int CH>
 __global__ __launch_bounds__(256) void split_rows_kernel(SplitRowsParams p) {
   constexpr int RPB = 256 / T;
-  __shared__ float wave_max[4];
+  __shared__ float tmp[4];
   const int first = (p.rows[0] + RPB - 1) / RPB, which = (int)blockIdx.x >= first;
   const int t = threadIdx.x % T;
   const int row = ((int)blockIdx.x - (which ? first : 0)) * RPB + threadIdx.x / T;
@@ -84,14 +87,8 @@ __global__ __launch_bounds__(256) void split_rows_kernel(SplitRowsParams p) {
   for (int i = 0; i < CH; ++i)
 #pragma unroll
     for (int e = 0; e < 4; ++e) mb = max(mb, __float_as_uint(v[i][e]) & 0x7fffffffu);
-#pragma unroll
-  for (int o = 32; o >= 1; o >>= 1) mb = max(mb, (uint32_t)__shfl_xor((int)mb, o));
-  if constexpr (T == 256) {
-    if ((threadIdx.x & 63) == 0) wave_max[threadIdx.x >> 6] = __uint_as_float(mb);
-    __syncthreads();
-#pragma unroll
-    for (int i = 0; i < 4; ++i) mb = max(mb, __float_as_uint(wave_max[i]));
-  }
+  if constexpr (T == 256) mb = block_max_bits(mb, tmp);
+  else mb = wave_max_bits(mb);
   const float s = split_scale(__uint_as_float(mb));
   f16* dst = p.dst[which] + (int64_t)row * 2 * p.K;
 #pragma unroll
@@ -105,8 +102,6 @@ __global__ __launch_bounds__(256) void split_rows_kernel(SplitRowsParams p) {
   if (t == 0) p.inv[which][row] = mb < 0x7f800000u ? 1.0f / s : __uint_as_float(0x7fc00000u);
 }
 
-constexpr int kSplitMaxK = 8192;   // the longest row split_rows takes
-
 static int split_rows(const SplitRowsParams& p, hipStream_t stream) {
   const int waves = (p.rows[0] + 3) / 4 + (p.rows[1] + 3) / 4, blocks = p.rows[0] + p.rows[1];
   if (p.K <= 1024) hipLaunchKernelGGL((split_rows_kernel<64, 4>), dim3(waves), dim3(256), 0, stream, p);
@@ -114,6 +109,169 @@ static int split_rows(const SplitRowsParams& p, hipStream_t stream) {
   else if (p.K <= 4096) hipLaunchKernelGGL((split_rows_kernel<256, 4>), dim3(blocks), dim3(256), 0, stream, p);
   else hipLaunchKernelGGL((split_rows_kernel<256, 8>), dim3(blocks), dim3(256), 0, stream, p);
   return check_launch("split_rows");
+}
+
+// ---------------------------------------------------------------------------------------------
+// Packed fp32 weights [n][k] -> split rows, once when a tower is bound, with a bound on |LN(x) . w + b|, the
+// Dense's output for any x: the normalised row has a norm of at most sqrt(k), so |.| <= sqrt(k) |gamma w| +
+// |beta . w| + |b| (one per row, to row_bound). It lets the outputs be split by one exponent that is known
+// before they are. Non-finite weights make it non-finite.
+// ---------------------------------------------------------------------------------------------
+template <int T, int CH>
+__global__ __launch_bounds__(256) void split_weight_kernel(const float* __restrict__ w, int k, int n,
+                                                           const float* __restrict__ bias,
+                                                           const float* __restrict__ gamma,
+                                                           const float* __restrict__ beta, int ln_cols,
+                                                           f16* __restrict__ out, float* __restrict__ inv,
+                                                           float* __restrict__ row_bound) {
+  __shared__ float tmp[4];
+  const int t = threadIdx.x % T, row = blockIdx.x * (256 / T) + threadIdx.x / T;
+  if (row >= n) return;                             // (a whole wave, or with T = 256 never)
+  const float* src = w + (int64_t)row * k;
+  f32x4 v[CH];
+  uint32_t mb = 0;
+  float norm = 0.f, dot = 0.f;
+#pragma unroll
+  for (int i = 0; i < CH; ++i) {
+    const int c = (t + i * T) * 4;
+    v[i] = c < k ? *reinterpret_cast<const f32x4*>(src + c) : f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+#pragma unroll
+  for (int i = 0; i < CH; ++i) {
+    const int c = (t + i * T) * 4;
+    if (c >= k) break;
+    const f32x4 one = {1.f, 1.f, 1.f, 1.f}, zero = {0.f, 0.f, 0.f, 0.f};
+    const f32x4 g = gamma ? *reinterpret_cast<const f32x4*>(gamma + c % ln_cols) : one;
+    const f32x4 b = beta ? *reinterpret_cast<const f32x4*>(beta + c % ln_cols) : zero;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      mb = max(mb, __float_as_uint(v[i][e]) & 0x7fffffffu);
+      norm = fmaf(g[e] * v[i][e], g[e] * v[i][e], norm);
+      dot = fmaf(b[e], v[i][e], dot);
+    }
+  }
+  if constexpr (T == 256) mb = block_max_bits(mb, tmp);
+  else mb = wave_max_bits(mb);
+  norm = row_sum<T>(norm, tmp);
+  dot = row_sum<T>(dot, tmp);
+  const float s = split_scale(__uint_as_float(mb));
+  f16* dst = out + (int64_t)row * 2 * k;
+#pragma unroll
+  for (int i = 0; i < CH; ++i) {
+    const int c = (t + i * T) * 4;
+    if (c >= k) break;
+    f16x4 hi, lo;
+    split4(v[i], s, hi, lo);
+    store_split4(dst, c, hi, lo);
+  }
+  if (t == 0) {
+    inv[row] = 1.0f / s;
+    const float b = 1.001f * sqrtf(norm * (float)k) + fabsf(dot) + fabsf(bias[row]);
+    row_bound[row] = b;
+  }
+}
+
+// out[g] = the largest of the values (>= 0 or NaN, which wins) of group g. (An atomic maximum per row on one
+// address took the launch above from 10 to 45 us.)
+__global__ __launch_bounds__(256) void group_max_kernel(const float* __restrict__ v, int n, float* __restrict__ out) {
+  __shared__ float tmp[4];
+  uint32_t mb = 0;
+  for (int i = threadIdx.x; i < n; i += 256) mb = max(mb, __float_as_uint(v[(int64_t)blockIdx.x * n + i]) & 0x7fffffffu);
+  mb = block_max_bits(mb, tmp);
+  if (threadIdx.x == 0) out[blockIdx.x] = __uint_as_float(mb);
+}
+
+int split_weight_f32(const float* w, int64_t k, int64_t n, const float* bias, const float* gamma, const float* beta,
+                     int ln_cols, int groups, void* out, float* inv, float* bound, hipStream_t stream) {
+#define QVL_SPLIT_WEIGHT(T, CH)                                                                                       \
+  hipLaunchKernelGGL((split_weight_kernel<T, CH>), dim3((unsigned)((n + 256 / T - 1) / (256 / T))), dim3(256), 0, stream, \
+                     w, (int)k, (int)n, bias, gamma, beta, ln_cols, (f16*)out, inv, bound + groups)
+  if (k <= 1024) QVL_SPLIT_WEIGHT(64, 4);
+  else if (k <= 2048) QVL_SPLIT_WEIGHT(64, 8);
+  else if (k <= 5120) QVL_SPLIT_WEIGHT(256, 5);
+  else QVL_SPLIT_WEIGHT(256, 8);
+#undef QVL_SPLIT_WEIGHT
+  QVL_TRY_RC(check_launch("split_weight"));
+  hipLaunchKernelGGL(group_max_kernel, dim3((unsigned)groups), dim3(256), 0, stream, bound + groups, (int)(n / groups), bound);
+  return check_launch("group_max");
+}
+
+// ---------------------------------------------------------------------------------------------
+// LayerNorm fp32 (the arithmetic of layernorm_f32_kernel) written as split rows for the Dense that reads it:
+// no fp32 copy of the normalised rows, and no pass to split them. T threads hold a row; MERGE: the 4 waves of a
+// workgroup normalise 4 consecutive rows that form one row of the output (the 2x2 merge), with one exponent.
+// ---------------------------------------------------------------------------------------------
+template <int T, int CH, bool MERGE>
+__global__ __launch_bounds__(256) void layernorm_split_kernel(const float* __restrict__ x, const float* __restrict__ gamma,
+                                                              const float* __restrict__ beta, f16* __restrict__ y,
+                                                              float* __restrict__ inv, int rows, int cols, float eps) {
+  static_assert(!MERGE || T == 64, "a wave per merged row");
+  __shared__ float tmp[4];
+  const int t = threadIdx.x % T, row = blockIdx.x * (256 / T) + threadIdx.x / T;
+  if (row >= rows) return;                            // (MERGE: rows % 4 == 0, all waves or none)
+  const float* xr = x + (int64_t)row * cols;
+  f32x4 v[CH];
+  float s = 0.f;
+#pragma unroll
+  for (int i = 0; i < CH; ++i) {
+    const int c = (t + T * i) * 4;
+    v[i] = c < cols ? *reinterpret_cast<const f32x4*>(xr + c) : f32x4{};
+    s += (v[i][0] + v[i][1]) + (v[i][2] + v[i][3]);
+  }
+  const float inv_n = 1.0f / (float)cols;
+  const float mean = row_sum<T>(s, tmp) * inv_n;
+  float q = 0.f;
+#pragma unroll
+  for (int i = 0; i < CH; ++i)
+    if ((t + T * i) * 4 < cols) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) { const float d = v[i][e] - mean; q += d * d; }
+    }
+  const float rstd = 1.0f / sqrtf(row_sum<T>(q, tmp) * inv_n + eps);
+  uint32_t mb = 0;
+#pragma unroll
+  for (int i = 0; i < CH; ++i) {
+    const int c = (t + T * i) * 4;
+    if (c >= cols) break;
+    const f32x4 g = *reinterpret_cast<const f32x4*>(gamma + c), b = *reinterpret_cast<const f32x4*>(beta + c);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      v[i][e] = (v[i][e] - mean) * rstd * g[e] + b[e];
+      mb = max(mb, __float_as_uint(v[i][e]) & 0x7fffffffu);
+    }
+  }
+  if constexpr (T > 64 || MERGE) mb = block_max_bits(mb, tmp);
+  else mb = wave_max_bits(mb);
+  const float sc = split_scale(__uint_as_float(mb));   // (a NaN row stays NaN in its hi terms)
+  const int orow = MERGE ? row / 4 : row, ocol = MERGE ? (row & 3) * cols : 0;
+  f16* dst = y + (int64_t)orow * 2 * (MERGE ? 4 * cols : cols);
+#pragma unroll
+  for (int i = 0; i < CH; ++i) {
+    const int c = (t + T * i) * 4;
+    if (c >= cols) break;
+    f16x4 hi, lo;
+    split4(v[i], sc, hi, lo);
+    store_split4(dst, ocol + c, hi, lo);
+  }
+  if (t == 0 && (!MERGE || (row & 3) == 0)) inv[orow] = 1.0f / sc;
+}
+
+// cols a multiple of 64 (32-column groups), at most kSplitMaxK; merge: rows % 4 == 0, cols <= 2048.
+int layer_norm_split(const float* x, const float* g, const float* b, void* y, float* inv, int rows, int cols, float eps,
+                     bool merge, hipStream_t stream) {
+  if (rows == 0) return QVL_OK;
+#define QVL_LN_SPLIT(T, CH, MERGE)                                                                              \
+  hipLaunchKernelGGL((layernorm_split_kernel<T, CH, MERGE>), dim3((rows + 256 / T - 1) / (256 / T)), dim3(256), 0, \
+                     stream, x, g, b, (f16*)y, inv, rows, cols, eps)
+  if (merge) {
+    if (cols <= 1024) QVL_LN_SPLIT(64, 4, true);
+    else QVL_LN_SPLIT(64, 8, true);
+  } else if (cols <= 1024) QVL_LN_SPLIT(64, 4, false);
+  else if (cols <= 2048) QVL_LN_SPLIT(64, 8, false);
+  else if (cols <= 5120) QVL_LN_SPLIT(256, 5, false);
+  else QVL_LN_SPLIT(256, 8, false);
+#undef QVL_LN_SPLIT
+  return check_launch("layernorm_split");
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -133,8 +291,8 @@ struct SplitShape {
 // one clock of a fragment read touches fall on 16 distinct bank groups.
 __device__ __forceinline__ int split_lds_off(int row, int chunk) { return row * 64 + ((chunk ^ ((row >> 1) & 7)) << 3); }
 
-// y[m, n..n+3] = epi(v + bias), v already scaled back.
-template <int EPI>
+// y[m, n..n+3] = epi(v + bias), v already scaled back; OUTS: as split rows, scaled by the exponent of p.ybound.
+template <int EPI, bool OUTS>
 __device__ __forceinline__ void split_store4(const GemmSplitParams& p, int m, int n, f32x4 v, const f32x4& bias) {
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
@@ -142,7 +300,18 @@ __device__ __forceinline__ void split_store4(const GemmSplitParams& p, int m, in
     if constexpr (EPI == kEpiBiasGelu) v[e] = gelu_tanh(v[e]);
   }
   if constexpr (EPI == kEpiBiasResidual) v += *reinterpret_cast<const f32x4*>(p.res + (int64_t)m * p.ldr + n);
-  *reinterpret_cast<f32x4*>(p.y + (int64_t)m * p.ldc + n) = v;
+  if constexpr (OUTS) {
+    f16x4 hi, lo;
+    split4(v, split_scale(*p.ybound), hi, lo);
+    store_split4(p.ys + (int64_t)m * 2 * p.N, n, hi, lo);
+  } else {
+    *reinterpret_cast<f32x4*>(p.y + (int64_t)m * p.ldc + n) = v;
+  }
+}
+
+// The factor of row m of x: its own, or one for every row from a bound on |x|.
+__device__ __forceinline__ float split_row_factor(const GemmSplitParams& p, int m) {
+  return p.sx ? p.sx[m] : 1.0f / split_scale(*p.xbound);
 }
 
 // acc 2^-(ex + ew): the smaller factor first, so that neither step leaves the range unless the result does
@@ -157,7 +326,7 @@ __device__ __forceinline__ bool any_nan(const f32x4& v) { return v[0] != v[0] ||
 
 // Outputs of a row or column that holds infinities or NaN (its scale is NaN), as the fp32 operands give them:
 // serial fp32 sums, left at the first NaN. Rare, so written small and not fast.
-template <int EPI>
+template <int EPI, bool OUTS>
 __device__ __forceinline__ void split_serial4(const GemmSplitParams& p, int m, int n, const f32x4& bias) {
   f32x4 v;
 #pragma unroll 1
@@ -168,10 +337,10 @@ __device__ __forceinline__ void split_serial4(const GemmSplitParams& p, int m, i
     for (int k = 0; k < p.K && a == a; ++k) a = fmaf(x[k], w[k], a);
     v[0] = e == 0 ? a : v[0]; v[1] = e == 1 ? a : v[1]; v[2] = e == 2 ? a : v[2]; v[3] = e == 3 ? a : v[3];
   }
-  split_store4<EPI>(p, m, n, v, bias);
+  split_store4<EPI, OUTS>(p, m, n, v, bias);
 }
 
-template <int BM, int BN, int WM, int WN, int NS, int EPI>
+template <int BM, int BN, int WM, int WN, int NS, int EPI, bool OUTS>
 __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_split_kernel(GemmSplitParams p) {
   using S = SplitShape<BM, BN, WM, WN>;
   extern __shared__ __attribute__((aligned(16))) f16 smem_h[];   // [NS][BM + BN][64]
@@ -326,22 +495,22 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_split_kernel(GemmSplitPa
       if (p.split > 1)
         *reinterpret_cast<f32x4*>(p.part + ((int64_t)part_i * p.M + m) * npad + n) = v;
       else if (nok) {
-        const float sx = p.sx[m];
-        if (sx == sx && !w_nan) split_store4<EPI>(p, m, n, split_unscale(v, sx, sw), bias);
+        const float sx = split_row_factor(p, m);
+        if (sx == sx && !w_nan) split_store4<EPI, OUTS>(p, m, n, split_unscale(v, sx, sw), bias);
       }
     }
   }
-  if (p.split > 1 || !nok) return;
+  if (p.split > 1 || !nok || !p.sx) return;
 #pragma unroll 1
   for (int r = lane / CH; r < S::TM; r += RPI) {
     const int m = m0 + wm * S::TM + r;
     if (m >= p.M) break;
-    if (w_nan || p.sx[m] != p.sx[m]) split_serial4<EPI>(p, m, n, bias);
+    if (w_nan || p.sx[m] != p.sx[m]) split_serial4<EPI, OUTS>(p, m, n, bias);
   }
 }
 
 // Sums the K parts in order and applies the epilogue, one thread per 4 consecutive outputs.
-template <int EPI>
+template <int EPI, bool OUTS>
 __global__ __launch_bounds__(256) void gemm_split_reduce_kernel(GemmSplitParams p, int64_t npad) {
   const int64_t q = (int64_t)blockIdx.x * 256 + threadIdx.x, quads = (int64_t)p.M * (p.N / 4);
   if (q >= quads) return;
@@ -351,28 +520,28 @@ __global__ __launch_bounds__(256) void gemm_split_reduce_kernel(GemmSplitParams 
   f32x4 v = *reinterpret_cast<const f32x4*>(src);
   for (int s = 1; s < p.split; ++s) v += *reinterpret_cast<const f32x4*>(src + s * stride);
   const f32x4 sw = *reinterpret_cast<const f32x4*>(p.sw + n), bias = *reinterpret_cast<const f32x4*>(p.bias + n);
-  const float sx = p.sx[m];
-  if (sx == sx && !any_nan(sw)) split_store4<EPI>(p, m, n, split_unscale(v, sx, sw), bias);
-  else split_serial4<EPI>(p, m, n, bias);
+  const float sx = split_row_factor(p, m);
+  if (sx == sx && !any_nan(sw)) split_store4<EPI, OUTS>(p, m, n, split_unscale(v, sx, sw), bias);
+  else split_serial4<EPI, OUTS>(p, m, n, bias);
 }
 
-template <int BM, int BN, int WM, int WN, int NS, int EPI>
+template <int BM, int BN, int WM, int WN, int NS, int EPI, bool OUTS>
 static int launch_gemm_split(GemmSplitParams p, int split, hipStream_t stream) {
   using S = SplitShape<BM, BN, WM, WN>;
   constexpr int lds = NS * S::STAGE * 2;
   static_assert(lds <= 163840, "LDS budget");
-  static const hipError_t attr = hipFuncSetAttribute((const void*)gemm_split_kernel<BM, BN, WM, WN, NS, EPI>,
+  static const hipError_t attr = hipFuncSetAttribute((const void*)gemm_split_kernel<BM, BN, WM, WN, NS, EPI, OUTS>,
                                                      hipFuncAttributeMaxDynamicSharedMemorySize, lds);
   if (attr != hipSuccess) return set_error(QVL_ERR_LAUNCH, "gemm_split: cannot reserve %d bytes of LDS", lds);
   const int tiles_n = (p.N + BN - 1) / BN, tiles = ((p.M + BM - 1) / BM) * tiles_n;
   const int64_t npad = (int64_t)tiles_n * BN;
   p.split = split;
   p.group_n = std::min(4, tiles_n);
-  hipLaunchKernelGGL((gemm_split_kernel<BM, BN, WM, WN, NS, EPI>), dim3(tiles * p.split), dim3(S::THREADS), lds, stream, p);
+  hipLaunchKernelGGL((gemm_split_kernel<BM, BN, WM, WN, NS, EPI, OUTS>), dim3(tiles * p.split), dim3(S::THREADS), lds, stream, p);
   int rc = check_launch("gemm_split");
   if (rc || p.split == 1) return rc;
   const int64_t blocks = ((int64_t)p.M * (p.N / 4) + 255) / 256;
-  hipLaunchKernelGGL(gemm_split_reduce_kernel<EPI>, dim3((unsigned)blocks), dim3(256), 0, stream, p, npad);
+  hipLaunchKernelGGL((gemm_split_reduce_kernel<EPI, OUTS>), dim3((unsigned)blocks), dim3(256), 0, stream, p, npad);
   return check_launch("gemm_split_reduce");
 }
 
@@ -410,7 +579,7 @@ static double split_cost(const SplitTile& t, const GemmSplitParams& p, int cus, 
          (split > 1 ? 8.0 * split * p.M * p.N / t.part_rate : 0.0);
 }
 
-template <int EPI>
+template <int EPI, bool OUTS = false>
 static int dispatch_gemm_split(const GemmSplitParams& p, hipStream_t stream) {
   const int cus = gemm_device_cus();
   int pick = 0, split = 1;
@@ -430,14 +599,18 @@ static int dispatch_gemm_split(const GemmSplitParams& p, hipStream_t stream) {
     }
   }
   switch (pick) {
-    case 0: return launch_gemm_split<64, 128, 2, 2, 2, EPI>(p, split, stream);
-    case 1: return launch_gemm_split<64, 128, 2, 2, 3, EPI>(p, split, stream);
-    case 2: return launch_gemm_split<128, 256, 2, 4, 3, EPI>(p, split, stream);
-    default: return launch_gemm_split<256, 256, 4, 2, 2, EPI>(p, split, stream);
+    case 0: return launch_gemm_split<64, 128, 2, 2, 2, EPI, OUTS>(p, split, stream);
+    case 1: return launch_gemm_split<64, 128, 2, 2, 3, EPI, OUTS>(p, split, stream);
+    case 2: return launch_gemm_split<128, 256, 2, 4, 3, EPI, OUTS>(p, split, stream);
+    default: return launch_gemm_split<256, 256, 4, 2, 2, EPI, OUTS>(p, split, stream);
   }
 }
 
 int gemm_split(const GemmSplitParams& p, int epi, hipStream_t stream) {
+  if (p.ys) {
+    if (epi != kEpiBiasGelu || p.N % 32) return set_error(QVL_ERR_INVALID_ARG, "gemm_split: split outputs need GELU, N %% 32 == 0");
+    return dispatch_gemm_split<kEpiBiasGelu, true>(p, stream);
+  }
   switch (epi) {
     case kEpiBias: return dispatch_gemm_split<kEpiBias>(p, stream);
     case kEpiBiasGelu: return dispatch_gemm_split<kEpiBiasGelu>(p, stream);
@@ -477,6 +650,13 @@ int gemm_f32_split(const GemmF32Params& g, int epi, hipStream_t stream) {
   p.part = g.part + used;          // (K is a multiple of 64: `used` is a multiple of 4)
   p.part_elems = g.part_elems - used;
   return gemm_split(p, epi, stream);
+}
+
+int split_rows_f32(const float* x, int64_t ldx, void* out, float* inv, int rows, int k, hipStream_t stream) {
+  SplitRowsParams r{};
+  r.src[0] = x; r.ld[0] = ldx; r.dst[0] = (f16*)out; r.inv[0] = inv; r.rows[0] = rows;
+  r.K = k;
+  return rows ? split_rows(r, stream) : QVL_OK;
 }
 
 }  // namespace qvl

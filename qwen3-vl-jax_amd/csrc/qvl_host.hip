@@ -485,7 +485,7 @@ struct TowerLayout {
   size_t esz;
   int64_t N, Np, D, I_pad, PV, PVp, hd, H;   // PVp: the pixel rows' width in the patch-embed GEMM
   int hdp, vrows;
-  size_t off_x, off_xn, off_q, off_k, off_vt, off_h, off_cs, off_part, part_bytes, off_apart, off_stats, apart_bytes, total;
+  size_t off_x, off_xn, off_q, off_k, off_vt, off_h, off_cs, off_part, part_bytes, off_apart, off_stats, off_sx, apart_bytes, total;
   int stat_groups;   // 128-column groups of a row's LayerNorm partials (hidden / 128; 0: hidden % 128 != 0)
 };
 
@@ -547,6 +547,8 @@ static int tower_layout(const qvl_vision_config* c, int64_t N, TowerLayout* L) {
   // (sum, squared deviations) of each row of x, or (mean, rstd) per row when hidden % 128 != 0
   L->stat_groups = c->hidden_size % 128 == 0 ? (int)(c->hidden_size / 128) : 0;
   L->off_stats = c->dtype == QVL_DTYPE_BF16 ? take((size_t)N * 8 * std::max(1, L->stat_groups)) : 0;
+  // row factors of the split-row operands (fp32 with split weights)
+  L->off_sx = c->dtype == QVL_DTYPE_F32 ? take((size_t)N * 4) : 0;
   L->total = o;
   return QVL_OK;
 }
@@ -560,6 +562,42 @@ int qvl_encode_vision_workspace_size(const qvl_vision_config* cfg, int64_t n_tok
   return QVL_OK;
 }
 
+
+// An fp32 Dense on split rows: x [M] split rows with the row factors sx, or one exponent for all from xbound;
+// the outputs fp32 (y) or, after GELU, split rows with the exponent of d.bound (ys). xf / wf: the fp32 operands,
+// where x may hold infinities or NaN (sx from split_rows).
+struct SplitDense {
+  const void* x; const float* sx; const float* xbound; const float* xf; int64_t ldx;
+  int64_t M, N, K;
+};
+
+static int split_dense(hipStream_t st, const qvl_split_dense& d, const SplitDense& a, const void* wf, const float* bias,
+                       int epi, const float* res, void* y, void* ys, void* part, size_t part_bytes) {
+  if (a.M * a.K * 4 >= (int64_t)UINT32_MAX) return set_error(QVL_ERR_UNSUPPORTED, "dense: operand larger than 4 GiB");
+  GemmSplitParams p{};
+  p.x = (const _Float16*)a.x; p.sx = a.sx; p.xbound = a.xbound; p.xf = a.xf; p.ldx = a.ldx;
+  p.w = (const _Float16*)d.w; p.sw = d.scale; p.wf = (const float*)wf; p.bias = bias;
+  p.res = res; p.ldr = a.N; p.y = (float*)y; p.ldc = a.N; p.ys = (_Float16*)ys; p.ybound = d.bound;
+  p.M = (int)a.M; p.N = (int)a.N; p.K = (int)a.K;
+  p.part = (float*)part; p.part_elems = (int64_t)(part_bytes / sizeof(float));
+  return gemm_split(p, epi, st);
+}
+
+// VisionPatchMerger.__call__ (model.py:648-656) in fp32 on split rows; h takes the hidden rows, xn the
+// normalised ones.
+static int run_merger_split(hipStream_t st, const qvl_vision_config* c, const TowerLayout& L, const qvl_merger_weights& mw,
+                            const qvl_split_merger& sm, bool postshuffle, const void* x, void* xn, void* h, void* out,
+                            float* sx, void* part) {
+  const int64_t N = L.N, D4 = 4 * L.D;
+  if (postshuffle)
+    QVL_TRY_RC(layer_norm_split((const float*)x, mw.norm_w, mw.norm_b, xn, sx, (int)(N / 4), (int)D4, c->ln_eps, false, st));
+  else
+    QVL_TRY_RC(layer_norm_split((const float*)x, mw.norm_w, mw.norm_b, xn, sx, (int)N, (int)L.D, c->ln_eps, true, st));
+  QVL_TRY_RC(split_dense(st, sm.fc1, {xn, sx, nullptr, nullptr, 0, N / 4, D4, D4}, mw.fc1_w, mw.fc1_b, QVL_EPI_BIAS_GELU,
+                         nullptr, nullptr, h, part, L.part_bytes));
+  return split_dense(st, sm.fc2, {h, nullptr, sm.fc1.bound, nullptr, 0, N / 4, c->out_hidden_size, D4}, mw.fc2_w, mw.fc2_b,
+                     QVL_EPI_BIAS, nullptr, out, nullptr, part, L.part_bytes);
+}
 
 // VisionPatchMerger.__call__ (model.py:648-656): main (LN over D then view [N/4, 4D]) or
 // deepstack (view [N/4, 4D] then LN over 4D); fc1 + GELU-tanh; fc2.
@@ -593,9 +631,9 @@ static int run_merger(hipStream_t st, const qvl_vision_config* c, const TowerLay
   return QVL_OK;
 }
 
-int qvl_encode_vision(void* stream, const qvl_vision_config* c, const qvl_vision_weights* W,
-                      const qvl_vision_metadata_dev* meta, const float* px, void* tokens, void* const* deepstack,
-                      void* ws, size_t ws_bytes) {
+static int encode_impl(void* stream, const qvl_vision_config* c, const qvl_vision_weights* W,
+                       const qvl_vision_split* split, const qvl_vision_metadata_dev* meta, const float* px, void* tokens,
+                       void* const* deepstack, void* ws, size_t ws_bytes) {
   if (!W || !meta) return set_error(QVL_ERR_INVALID_ARG, "encode_vision: NULL weights/metadata");
   TowerLayout L;
   QVL_TRY_RC(tower_layout(c, meta->n_tokens, &L));
@@ -621,6 +659,7 @@ int qvl_encode_vision(void* stream, const qvl_vision_config* c, const qvl_vision
   const int64_t N = L.N, D = L.D, I = L.I_pad;
   const size_t e = L.esz;
   const float qscale = (1.0f / sqrtf((float)L.hd)) * kLog2e;
+  float* sx = f32 ? (float*)(base + L.off_sx) : nullptr;
   const bool win = c->use_window != 0;
   const int64_t Dout = c->out_hidden_size;
   if (win) {
@@ -673,7 +712,16 @@ int qvl_encode_vision(void* stream, const qvl_vision_config* c, const qvl_vision
   for (int j = 0; j < c->n_deepstack && !f32; ++j) any_fold = any_fold || W->deepstack[j].fc1_ln.w;
   const int G = any_fold ? L.stat_groups : 0;
   bool have_parts = false;
-  if (c->num_position_embeddings > 0 && !f32 && D % 8 == 0) {
+  // (with split weights the pixel rows are split into the then idle q / k / v buffers)
+  const bool split_px = split && (size_t)N * L.PVp * 4 <= L.off_h - L.off_q;
+  if (split_px) {
+    if (c->num_position_embeddings > 0)
+      QVL_TRY_RC(qvl_pos_embed(st, dt, W->pos_table, meta->tap_idx, meta->tap_w, xn, N, D));
+    QVL_TRY_RC(split_rows_f32((const float*)px_in, L.PVp, Qb, sx, (int)N, (int)L.PVp, st));
+    QVL_TRY_RC(split_dense(st, split->patch, {Qb, sx, nullptr, (const float*)px_in, L.PVp, N, D, L.PVp}, W->patch_w,
+                           W->patch_b, c->num_position_embeddings > 0 ? QVL_EPI_BIAS_RESIDUAL : QVL_EPI_BIAS,
+                           (const float*)xn, x, nullptr, part, PB));
+  } else if (c->num_position_embeddings > 0 && !f32 && D % 8 == 0) {
     // bf16: the pos-embed gathered per row inside the patch embed's residual epilogue (no [N, D]
     // pos-embed buffer written and read back), with x's row partials when a fold reads them
     QVL_TRY_RC(qvl_dense_pos_embed_ws(st, dt, px_in, L.PVp, W->patch_w, W->patch_b, W->pos_table, meta->tap_idx,
@@ -700,9 +748,12 @@ int qvl_encode_vision(void* stream, const qvl_vision_config* c, const qvl_vision
     // bf16: norm1 / norm2 folded into the qkv / fc1 GEMMs (the Dense reads x itself; only the row
     // statistics run before it)
     const bool fold = !f32 && B.qkv_ln.w && B.qkv_ln.cd && B.fc1_ln.w && B.fc1_ln.cd;
+    const qvl_split_block* sb = split ? &split->blocks[i] : nullptr;
     // x += proj(attention(rotary(qkv(LN1 x))))   (model.py:628, 569-601)
     if (fold) {
       if (!have_parts) QVL_TRY_RC(qvl_row_stats(st, dt, x, D, N, D, c->ln_eps, stats));
+    } else if (sb) {
+      QVL_TRY_RC(layer_norm_split((const float*)x, B.norm1_w, B.norm1_b, xn, sx, (int)N, (int)D, c->ln_eps, false, st));
     } else {
       QVL_TRY_RC(qvl_layer_norm(st, dt, x, D, B.norm1_w, B.norm1_b, xn, D, N, D, c->ln_eps));
     }
@@ -726,7 +777,10 @@ int qvl_encode_vision(void* stream, const qvl_vision_config* c, const qvl_vision
         QVL_TRY_RC(qvl_dense_qkv_rotary(st, dt, xn, D, B.qkv_w, B.qkv_b, cs, Qb, Kb, Vb, N, D, (int)L.H, part, PB));
     } else {
       // qkv Dense into h, then rotary + head-major relayout.
-      if (fold && have_parts)
+      if (sb)
+        QVL_TRY_RC(split_dense(st, sb->qkv, {xn, sx, nullptr, nullptr, 0, N, 3 * D, D}, B.qkv_w, B.qkv_b, QVL_EPI_BIAS,
+                               nullptr, h, nullptr, part, PB));
+      else if (fold && have_parts)
         QVL_TRY_RC(qvl_dense_ln_parts_ws(st, dt, QVL_EPI_BIAS, x, D, B.qkv_ln.w, B.qkv_ln.cd, stats, G, c->ln_eps,
                                          B.qkv_b, h, 3 * D, N, 3 * D, D, part, PB));
       else if (fold)
@@ -756,43 +810,105 @@ int qvl_encode_vision(void* stream, const qvl_vision_config* c, const qvl_vision
                                          full ? meta->n_tiles : meta->n_window_tiles, N, (int)L.H, (int)L.hd, xn, D));
     }
     have_parts = fold && G;
-    if (have_parts)
-      QVL_TRY_RC(qvl_dense_rowstats_ws(st, dt, xn, D, B.proj_w, B.proj_b, x, D, x, D, N, D, D, stats, part, PB));
-    else
-      QVL_TRY_RC(qvl_dense_ws(st, dt, QVL_EPI_BIAS_RESIDUAL, xn, D, B.proj_w, B.proj_b, x, D, x, D, N, D, D, part, PB));
-    // x += fc2(gelu(fc1(LN2 x)))   (model.py:629, 610-614)
-    if (fold && have_parts) {
-      QVL_TRY_RC(qvl_dense_ln_parts_ws(st, dt, QVL_EPI_BIAS_GELU, x, D, B.fc1_ln.w, B.fc1_ln.cd, stats, G, c->ln_eps,
-                                       B.fc1_b, h, I, N, I, D, part, PB));
-    } else if (fold) {
-      QVL_TRY_RC(qvl_row_stats(st, dt, x, D, N, D, c->ln_eps, stats));
-      QVL_TRY_RC(qvl_dense_ln_ws(st, dt, QVL_EPI_BIAS_GELU, x, D, B.fc1_ln.w, B.fc1_ln.cd, stats, B.fc1_b, h, I, N, I,
-                                 D, part, PB));
+    if (sb) {
+      // the attention's output split into the then idle q buffer, proj, norm2 to split rows, fc1's GELU output
+      // written as split rows, fc2
+      QVL_TRY_RC(split_rows_f32((const float*)xn, D, Qb, sx, (int)N, (int)D, st));
+      QVL_TRY_RC(split_dense(st, sb->proj, {Qb, sx, nullptr, (const float*)xn, D, N, D, D}, B.proj_w, B.proj_b,
+                             QVL_EPI_BIAS_RESIDUAL, (const float*)x, x, nullptr, part, PB));
+      QVL_TRY_RC(layer_norm_split((const float*)x, B.norm2_w, B.norm2_b, xn, sx, (int)N, (int)D, c->ln_eps, false, st));
+      QVL_TRY_RC(split_dense(st, sb->fc1, {xn, sx, nullptr, nullptr, 0, N, I, D}, B.fc1_w, B.fc1_b, QVL_EPI_BIAS_GELU,
+                             nullptr, nullptr, h, part, PB));
+      QVL_TRY_RC(split_dense(st, sb->fc2, {h, nullptr, sb->fc1.bound, nullptr, 0, N, D, I}, B.fc2_w, B.fc2_b,
+                             QVL_EPI_BIAS_RESIDUAL, (const float*)x, x, nullptr, part, PB));
     } else {
-      QVL_TRY_RC(qvl_layer_norm(st, dt, x, D, B.norm2_w, B.norm2_b, xn, D, N, D, c->ln_eps));
-      QVL_TRY_RC(qvl_dense_ws(st, dt, QVL_EPI_BIAS_GELU, xn, D, B.fc1_w, B.fc1_b, nullptr, 0, h, I, N, I, D, part, PB));
+      if (have_parts)
+        QVL_TRY_RC(qvl_dense_rowstats_ws(st, dt, xn, D, B.proj_w, B.proj_b, x, D, x, D, N, D, D, stats, part, PB));
+      else
+        QVL_TRY_RC(qvl_dense_ws(st, dt, QVL_EPI_BIAS_RESIDUAL, xn, D, B.proj_w, B.proj_b, x, D, x, D, N, D, D, part, PB));
+      // x += fc2(gelu(fc1(LN2 x)))   (model.py:629, 610-614)
+      if (fold && have_parts) {
+        QVL_TRY_RC(qvl_dense_ln_parts_ws(st, dt, QVL_EPI_BIAS_GELU, x, D, B.fc1_ln.w, B.fc1_ln.cd, stats, G, c->ln_eps,
+                                         B.fc1_b, h, I, N, I, D, part, PB));
+      } else if (fold) {
+        QVL_TRY_RC(qvl_row_stats(st, dt, x, D, N, D, c->ln_eps, stats));
+        QVL_TRY_RC(qvl_dense_ln_ws(st, dt, QVL_EPI_BIAS_GELU, x, D, B.fc1_ln.w, B.fc1_ln.cd, stats, B.fc1_b, h, I, N, I,
+                                   D, part, PB));
+      } else {
+        QVL_TRY_RC(qvl_layer_norm(st, dt, x, D, B.norm2_w, B.norm2_b, xn, D, N, D, c->ln_eps));
+        QVL_TRY_RC(qvl_dense_ws(st, dt, QVL_EPI_BIAS_GELU, xn, D, B.fc1_w, B.fc1_b, nullptr, 0, h, I, N, I, D, part, PB));
+      }
+      // partials of the new x for the next block's folded norm1 or a folded deepstack merger
+      have_parts = G != 0;
+      if (have_parts)
+        QVL_TRY_RC(qvl_dense_rowstats_ws(st, dt, h, I, B.fc2_w, B.fc2_b, x, D, x, D, N, D, I, stats, part, PB));
+      else
+        QVL_TRY_RC(qvl_dense_ws(st, dt, QVL_EPI_BIAS_RESIDUAL, h, I, B.fc2_w, B.fc2_b, x, D, x, D, N, D, I, part, PB));
     }
-    // partials of the new x for the next block's folded norm1 or a folded deepstack merger
-    have_parts = G != 0;
-    if (have_parts)
-      QVL_TRY_RC(qvl_dense_rowstats_ws(st, dt, h, I, B.fc2_w, B.fc2_b, x, D, x, D, N, D, I, stats, part, PB));
-    else
-      QVL_TRY_RC(qvl_dense_ws(st, dt, QVL_EPI_BIAS_RESIDUAL, h, I, B.fc2_w, B.fc2_b, x, D, x, D, N, D, I, part, PB));
     // deepstack tap (model.py:841-843)
     for (int j = 0; j < c->n_deepstack; ++j)
       if (c->deepstack_indexes[j] == i) {
         void* out = win ? (void*)Qb : deepstack[ds_next];
-        QVL_TRY_RC(run_merger(st, c, L, W->deepstack[ds_next], true, x, xn, h, out, part, stats,
-                              have_parts ? G : 0));
+        if (split)
+          QVL_TRY_RC(run_merger_split(st, c, L, W->deepstack[ds_next], split->deepstack[ds_next], true, x, xn, h, out, sx,
+                                      part));
+        else
+          QVL_TRY_RC(run_merger(st, c, L, W->deepstack[ds_next], true, x, xn, h, out, part, stats,
+                                have_parts ? G : 0));
         if (win)   // unshuffle (model.py:845-848)
           QVL_TRY_RC(qvl_gather_rows(st, dt, Qb, Dout, dt, deepstack[ds_next], Dout, meta->window_reverse, N / 4, 1, Dout));
         ++ds_next;
       }
   }
   (void)e;
-  QVL_TRY_RC(run_merger(st, c, L, W->merger, false, x, xn, h, win ? (void*)Qb : tokens, part, stats, 0));
+  if (split)
+    QVL_TRY_RC(run_merger_split(st, c, L, W->merger, split->merger, false, x, xn, h, win ? (void*)Qb : tokens, sx, part));
+  else
+    QVL_TRY_RC(run_merger(st, c, L, W->merger, false, x, xn, h, win ? (void*)Qb : tokens, part, stats, 0));
   if (win) QVL_TRY_RC(qvl_gather_rows(st, dt, Qb, Dout, dt, tokens, Dout, meta->window_reverse, N / 4, 1, Dout));
   return QVL_OK;
+}
+
+int qvl_encode_vision(void* stream, const qvl_vision_config* c, const qvl_vision_weights* W,
+                      const qvl_vision_metadata_dev* meta, const float* px, void* tokens, void* const* deepstack,
+                      void* ws, size_t ws_bytes) {
+  return encode_impl(stream, c, W, nullptr, meta, px, tokens, deepstack, ws, ws_bytes);
+}
+
+int qvl_encode_vision_split(void* stream, const qvl_vision_config* c, const qvl_vision_weights* W,
+                            const qvl_vision_split* split, const qvl_vision_metadata_dev* meta, const float* px,
+                            void* tokens, void* const* deepstack, void* ws, size_t ws_bytes) {
+  if (!c || !split || !split->blocks || (c->n_deepstack > 0 && !split->deepstack))
+    return set_error(QVL_ERR_INVALID_ARG, "encode_vision_split: NULL config / split weights");
+  if (c->dtype != QVL_DTYPE_F32) return set_error(QVL_ERR_UNSUPPORTED, "encode_vision_split: dtype %d (fp32 only)", c->dtype);
+  if (round_up(c->patch_volume, 64) > kSplitMaxK || round_up(c->intermediate_size, 64) > kSplitMaxK ||
+      4 * (int64_t)c->hidden_size > kSplitMaxK)
+    return set_error(QVL_ERR_UNSUPPORTED, "encode_vision_split: rows longer than %d", kSplitMaxK);
+  const auto whole = [](const qvl_split_dense& d, bool bound) { return d.w && d.scale && (!bound || d.bound); };
+  bool ok = whole(split->patch, false) && whole(split->merger.fc1, true) && whole(split->merger.fc2, false);
+  for (int i = 0; i < c->depth; ++i) {
+    const qvl_split_block& b = split->blocks[i];
+    ok = ok && whole(b.qkv, true) && whole(b.proj, false) && whole(b.fc1, true) && whole(b.fc2, false);
+  }
+  for (int j = 0; j < c->n_deepstack; ++j)
+    ok = ok && whole(split->deepstack[j].fc1, true) && whole(split->deepstack[j].fc2, false);
+  if (!ok) return set_error(QVL_ERR_INVALID_ARG, "encode_vision_split: NULL split weight");
+  return encode_impl(stream, c, W, split, meta, px, tokens, deepstack, ws, ws_bytes);
+}
+
+int qvl_split_dense_weight(void* stream, const float* w, int64_t k_in, int64_t n_out, const float* bias,
+                           const float* gamma, const float* beta, int64_t ln_cols, int32_t groups, void* out_w,
+                           float* out_scale, float* out_bound) {
+  if (k_in <= 0 || k_in % 64 || k_in > kSplitMaxK || n_out <= 0 || n_out > INT32_MAX || groups <= 0 || n_out % groups ||
+      ((gamma || beta) && (ln_cols <= 0 || ln_cols % 4)))
+    return set_error(QVL_ERR_INVALID_ARG, "split_dense_weight: k_in=%lld (a multiple of 64, at most %d) n_out=%lld groups=%d",
+                     (long long)k_in, kSplitMaxK, (long long)n_out, groups);
+  if (!w || !bias || !out_w || !out_scale || !out_bound)
+    return set_error(QVL_ERR_INVALID_ARG, "split_dense_weight: NULL operand");
+  if (!aligned16(w) || !aligned16(out_w) || !aligned16(out_scale) || !aligned16(gamma) || !aligned16(beta))
+    return set_error(QVL_ERR_MISALIGNED, "split_dense_weight: operands must be 16-byte aligned");
+  return split_weight_f32(w, k_in, n_out, bias, gamma, beta, (int)ln_cols, groups, out_w, out_scale, out_bound,
+                          (hipStream_t)stream);
 }
 
 }  // extern "C"

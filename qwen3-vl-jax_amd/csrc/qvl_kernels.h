@@ -90,6 +90,9 @@ struct GemmSplitParams {
   float* y; int64_t ldc;
   int M, N, K;
   const float* xf; int64_t ldx; const float* wf;
+  const float* xbound;             // sx NULL: every row of x carries the exponent of *xbound >= max |x|
+  _Float16* ys;                    // GELU only, instead of y: the outputs [M, N] as split rows with the
+  const float* ybound;             // exponent of *ybound >= max |y|
   float* part; int64_t part_elems; // split-K partials (set up by the launcher, as in GemmF32Params)
   int split, group_n;
 };
@@ -145,6 +148,13 @@ int gemm_f32(GemmF32Params p, int epi, hipStream_t stream);
 bool gemm_f32_use_split(const GemmF32Params& g);
 int gemm_f32_split(const GemmF32Params& g, int epi, hipStream_t stream);
 int gemm_f32_set_plan(int tile);
+constexpr int kSplitMaxK = 8192;   // the longest row the split kernels hold
+int gemm_split(const GemmSplitParams& p, int epi, hipStream_t stream);
+int split_rows_f32(const float* x, int64_t ldx, void* out, float* inv, int rows, int k, hipStream_t stream);
+int split_weight_f32(const float* w, int64_t k, int64_t n, const float* bias, const float* gamma, const float* beta,
+                     int ln_cols, int groups, void* out, float* inv, float* bound, hipStream_t stream);
+int layer_norm_split(const float* x, const float* g, const float* b, void* y, float* inv, int rows, int cols, float eps,
+                     bool merge, hipStream_t stream);
 int layer_norm_f32(const float* x, int64_t ldx, const float* g, const float* b, float* y, int64_t ldy, int rows,
                    int cols, float eps, hipStream_t stream);
 int pos_embed_f32(const float* table, const int* idx, const float* wts, float* y, int n_tok, int dim,

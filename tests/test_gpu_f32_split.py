@@ -104,3 +104,68 @@ def test_split_dense_infinities_and_nan(dense, K):
             assert torch.equal(got[inf_at], want[inf_at]) and torch.equal(torch.isinf(got), inf_at)
             fine = torch.isfinite(want)
             assert torch.allclose(got[fine], want[fine], rtol=1e-4, atol=1e-4)
+
+
+# ---------------------------------------------------------------------------------------------
+# the fp32 tower on weights split when it is bound
+# ---------------------------------------------------------------------------------------------
+@pytest.mark.parametrize("K,N,groups", [(64, 64, 1), (1024, 192, 3), (1152, 128, 1), (4096, 64, 1), (8192, 128, 2)])
+def test_split_weight_values_and_bound(pkg, lib, K, N, groups):
+    """hi + lo is the weight to 2^-22 of it (or 2^-39 of the row's largest), and no normalised row's output passes
+    the bound: sqrt(K) |gamma w| + |beta . w| + |b|, reached within a factor by the row that points along gamma w."""
+    cp = pkg.capi
+    g = torch.Generator(device=DEV).manual_seed(K + N)
+    w = torch.randn((N, K), generator=g, device=DEV) * 10.0 ** torch.linspace(-20, 5, K, device=DEV)
+    w[1] = 0.0
+    gamma, beta = (torch.randn(K // 4, generator=g, device=DEV) for _ in range(2))     # repeated 4 times along a row
+    b = torch.randn(N, generator=g, device=DEV)
+    out = torch.empty((N, K // 32, 2, 32), dtype=torch.float16, device=DEV)
+    scale = torch.empty(N, device=DEV)
+    bound = torch.empty(groups + N, device=DEV)
+    cp.check(lib.qvl_split_dense_weight(torch.cuda.current_stream().cuda_stream, w.data_ptr(), K, N, b.data_ptr(),
+                                        gamma.data_ptr(), beta.data_ptr(), K // 4, groups, out.data_ptr(),
+                                        scale.data_ptr(), bound.data_ptr()))
+    got = (out.double().sum(2) * scale[:, None, None].double()).reshape(N, K)
+    big = w.abs().amax(1, keepdim=True).double()
+    assert torch.all((got - w.double()).abs() <= w.abs().double() * 2.0 ** -22 + big * 2.0 ** -39)
+    ga, be = gamma.double().repeat(4), beta.double().repeat(4)
+    gw = ga * w.double()
+    want = K ** 0.5 * gw.norm(dim=1) + (w.double() @ be).abs() + b.double().abs()
+    assert torch.all(bound[groups:] >= want * 0.9999) and torch.all(bound[groups:] <= want * 1.002)
+    assert torch.equal(bound[:groups], bound[groups:].view(groups, -1).amax(1))
+
+
+def tower_pair(pkg, spec, params):
+    """The fp32 tower with its split weights, and without them."""
+    a = pkg.Qwen3VisionTransformer(spec).bind(params)
+    b = pkg.Qwen3VisionTransformer(spec).bind_packed(a.packed_state())
+    assert a._split is not None
+    b._split = None
+    return a, b
+
+
+def test_split_tower_nan_stays_in_its_segment(pkg):
+    spec = pkg.spec_2b()
+    spec.depth, spec.deepstack_visual_indexes = 2, (0,)
+    a, b = tower_pair(pkg, spec, pkg.random_params(spec, seed=2))
+    grids = np.array([[1, 6, 10], [1, 8, 12]], np.int32)
+    px = np.random.default_rng(3).standard_normal((156, spec.patch_volume), dtype=np.float32)
+    clean = a(px, grids)
+    for bad in (np.nan, np.inf):
+        px[7, 100] = bad
+        (tok, ds), (tok_b, ds_b) = a(px, grids), b(px, grids)
+        for x, y, z in ((tok, tok_b, clean[0]), (ds[0], ds_b[0], clean[1][0])):
+            assert torch.equal(torch.isnan(x), torch.isnan(y)) and torch.equal(x[15:], z[15:])
+
+
+def test_weights_that_cannot_be_split_leave_the_tower_unsplit(pkg):
+    spec = pkg.spec_2b()
+    spec.depth, spec.deepstack_visual_indexes = 1, ()
+    params = pkg.random_params(spec, seed=2)
+    grids = np.array([[1, 4, 6]], np.int32)
+    px = np.random.default_rng(3).standard_normal((24, spec.patch_volume), dtype=np.float32)
+    params["visual"]["merger"]["linear_fc2"]["kernel"][3, 5] = np.inf
+    t = pkg.Qwen3VisionTransformer(spec).bind(params)
+    assert t._split is None
+    tokens, _ = t(px, grids)
+    assert not torch.isfinite(tokens[:, 5]).any() and torch.isfinite(tokens[:, :5]).all()
