@@ -32,7 +32,7 @@
 // within the 128-register budget of 4 waves/SIMD.
 #include <math.h>
 #include <type_traits>
-#include "qvl_kernels.h"
+#include "qvl_split.h"
 
 namespace qvl {
 
@@ -634,10 +634,11 @@ __global__ __launch_bounds__(256, 3) void attn_fwd_qk88_kernel(
 // (query, 4 dims) pairs of it: out = sum_i O_i 2^(m_i - M) / sum_i l_i 2^(m_i - M),
 // M = max_i m_i (scores in log2 units). All parts' loads issue before any use.
 // ---------------------------------------------------------------------------------------------
+// OutT bf16 or float rows, or f16: split rows (ldo = their width in fp32 values) with the exponent of *bound.
 template <int HD, typename OutT>
 __global__ __launch_bounds__(256) void attn_combine_kernel(const int* __restrict__ tiles, int n_whole, int n_slots,
                                                            const float* __restrict__ part, OutT* __restrict__ O,
-                                                           int64_t ldo) {
+                                                           int64_t ldo, const float* __restrict__ bound) {
   constexpr int kChunks = (kAttnBM * (HD / 4) + 255) / 256;
   const int slot = blockIdx.x / kChunks, chunk = blockIdx.x % kChunks;
   const int item = n_whole + slot;
@@ -676,7 +677,11 @@ __global__ __launch_bounds__(256) void attn_combine_kernel(const int* __restrict
     }
   }
   const float inv = 1.0f / L;
-  if constexpr (sizeof(OutT) == 4)
+  if constexpr (std::is_same<OutT, f16>::value) {
+    f16x4 hi, lo;
+    split4(acc * inv, split_scale(*bound), hi, lo);
+    store_split4(O + (int64_t)(q0 + ql) * 2 * ldo, head * HD + d, hi, lo);
+  } else if constexpr (sizeof(OutT) == 4)
     *reinterpret_cast<f32x4*>(O + (int64_t)(q0 + ql) * ldo + head * HD + d) =
         f32x4{acc[0] * inv, acc[1] * inv, acc[2] * inv, acc[3] * inv};
   else
@@ -686,11 +691,11 @@ __global__ __launch_bounds__(256) void attn_combine_kernel(const int* __restrict
 
 template <int HD, typename OutT = bf16>
 static int launch_combine(const int* d_tiles, int64_t n_tiles, int64_t n_whole, const float* part, OutT* out,
-                          int64_t ldo, hipStream_t stream) {
+                          int64_t ldo, hipStream_t stream, const float* bound = nullptr) {
   constexpr int kChunks = (kAttnBM * (HD / 4) + 255) / 256;
   const int64_t n_slots = n_tiles - n_whole;
   hipLaunchKernelGGL((attn_combine_kernel<HD, OutT>), dim3((unsigned)(n_slots * kChunks)), dim3(256), 0, stream,
-                     d_tiles, (int)n_whole, (int)n_slots, part, out, ldo);
+                     d_tiles, (int)n_whole, (int)n_slots, part, out, ldo, bound);
   return check_launch("attn_combine");
 }
 
@@ -700,6 +705,13 @@ int attention_combine_f32(const int* d_tiles, int64_t n_tiles, int64_t n_whole, 
   if (hd == 64) return launch_combine<64, float>(d_tiles, n_tiles, n_whole, part, out, ldo, stream);
   if (hd == 72) return launch_combine<72, float>(d_tiles, n_tiles, n_whole, part, out, ldo, stream);
   return launch_combine<80, float>(d_tiles, n_tiles, n_whole, part, out, ldo, stream);
+}
+
+int attention_combine_split(const int* d_tiles, int64_t n_tiles, int64_t n_whole, const float* part, const float* bound,
+                            void* out, int64_t ldo, int hd, hipStream_t stream) {
+  if (hd == 64) return launch_combine<64, f16>(d_tiles, n_tiles, n_whole, part, (f16*)out, ldo, stream, bound);
+  if (hd == 72) return launch_combine<72, f16>(d_tiles, n_tiles, n_whole, part, (f16*)out, ldo, stream, bound);
+  return launch_combine<80, f16>(d_tiles, n_tiles, n_whole, part, (f16*)out, ldo, stream, bound);
 }
 
 // One rotary output x*cos + rotate_half(x)*sin in the reference's bf16 arithmetic (model.py:579-582):

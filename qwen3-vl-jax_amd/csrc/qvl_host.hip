@@ -533,8 +533,10 @@ static int tower_layout(const qvl_vision_config* c, int64_t N, TowerLayout* L) {
   auto take = [&](size_t bytes) { size_t r = o; o += round_up((int64_t)bytes, 256); return r; };
   L->off_x = take((size_t)N * L->D * e);
   L->off_xn = take((size_t)N * L->D * e);
-  L->off_q = take((size_t)L->H * L->Np * hdp * e);
-  L->off_k = take((size_t)L->H * L->Np * hdp * e);
+  // (fp32: rows of the fp32 kernels, or the slightly longer ones of the split attention)
+  const size_t qk_row = c->dtype == QVL_DTYPE_F32 ? std::max<size_t>(hdp * 4, attn_split_row_halfs((int)hd) * 2) : hdp * e;
+  L->off_q = take((size_t)L->H * L->Np * qk_row);
+  L->off_k = take((size_t)L->H * L->Np * qk_row);
   L->off_vt = take((size_t)L->H * L->Np * vrows * e);
   L->off_h = take((size_t)N * hcols * e);
   L->off_cs = take((size_t)N * (hd / 2) * 8);
@@ -789,7 +791,10 @@ static int encode_impl(void* stream, const qvl_vision_config* c, const qvl_visio
       else
         QVL_TRY_RC(qvl_dense_ws(st, dt, QVL_EPI_BIAS, xn, D, B.qkv_w, B.qkv_b, nullptr, 0, h, 3 * D, N, 3 * D, D, part,
                                 PB));
-      if (f32)
+      if (sb)
+        QVL_TRY_RC(attention_relayout_split((const float*)h, 3 * D, cs, sb->qkv.bound, (int)N, (int)L.Np, (int)L.H,
+                                            (int)L.hd, Qb, Kb, Vb, st));
+      else if (f32)
         QVL_TRY_RC(attention_relayout_f32((const float*)h, (const float*)h + D, (const float*)h + 2 * D, 3 * D, cs,
                                           (int)N, (int)L.Np, (int)L.H, (int)L.hd, L.vrows, qscale, (float*)Qb,
                                           (float*)Kb, (float*)Vb, st));
@@ -800,7 +805,16 @@ static int encode_impl(void* stream, const qvl_vision_config* c, const qvl_visio
     }
     // window mode: blocks outside fullatt_block_indexes attend within windows (model.py:838-839)
     const bool full = !win || ((c->fullatt_mask >> i) & 1ull);
-    if (full && meta->split_tiles) {
+    if (sb) {
+      const bool parts = full && meta->split_tiles;
+      const int64_t n_items = parts ? meta->n_split_tiles : full ? meta->n_tiles : meta->n_window_tiles;
+      const int64_t n_whole = parts ? meta->n_split_whole : n_items;
+      if ((size_t)(n_items - n_whole) * attn_partial_floats((int)L.hd) * sizeof(float) > L.apart_bytes)
+        return set_error(QVL_ERR_WORKSPACE, "encode_vision: %lld key parts", (long long)(n_items - n_whole));
+      QVL_TRY_RC(attention_split(Qb, Kb, Vb, parts ? meta->split_tiles : full ? meta->tiles : meta->window_tiles, n_items,
+                                 n_whole, sb->qkv.bound, (int)L.Np, (int)L.H, (int)L.hd, qscale, xn,
+                                 (float*)(base + L.off_apart), st));
+    } else if (full && meta->split_tiles) {
       void* apart = base + L.off_apart;
       QVL_TRY_RC(qvl_attention_headmajor_split(st, dt, Qb, Kb, Vb, meta->split_tiles, meta->n_split_tiles,
                                                meta->n_split_whole, N, (int)L.H, (int)L.hd, xn, D, apart,
@@ -811,10 +825,9 @@ static int encode_impl(void* stream, const qvl_vision_config* c, const qvl_visio
     }
     have_parts = fold && G;
     if (sb) {
-      // the attention's output split into the then idle q buffer, proj, norm2 to split rows, fc1's GELU output
-      // written as split rows, fc2
-      QVL_TRY_RC(split_rows_f32((const float*)xn, D, Qb, sx, (int)N, (int)D, st));
-      QVL_TRY_RC(split_dense(st, sb->proj, {Qb, sx, nullptr, (const float*)xn, D, N, D, D}, B.proj_w, B.proj_b,
+      // proj on the attention's split rows (v's exponent), norm2 to split rows, fc1's GELU output written as
+      // split rows, fc2
+      QVL_TRY_RC(split_dense(st, sb->proj, {xn, nullptr, sb->qkv.bound + 2, nullptr, 0, N, D, D}, B.proj_w, B.proj_b,
                              QVL_EPI_BIAS_RESIDUAL, (const float*)x, x, nullptr, part, PB));
       QVL_TRY_RC(layer_norm_split((const float*)x, B.norm2_w, B.norm2_b, xn, sx, (int)N, (int)D, c->ln_eps, false, st));
       QVL_TRY_RC(split_dense(st, sb->fc1, {xn, sx, nullptr, nullptr, 0, N, I, D}, B.fc1_w, B.fc1_b, QVL_EPI_BIAS_GELU,

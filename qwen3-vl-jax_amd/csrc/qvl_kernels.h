@@ -169,6 +169,16 @@ int attention_f32(const float* Qb, const float* Kb, const float* Vtb, const int*
                   int hd, float* out, int64_t ldo, hipStream_t stream, int64_t n_whole = -1, float* part = nullptr);
 int attention_combine_f32(const int* d_tiles, int64_t n_tiles, int64_t n_whole, const float* part, float* out,
                           int64_t ldo, int hd, hipStream_t stream);
+// fp32 attention on f16-split operands (qvl_f32_attn.hip): the qkv Dense's rows [N, 3 H hd] to its operands, and
+// the attention itself, whose output is [N] split rows with the exponent of bound[2] (bound: on |q|, |k|, |v|
+// before the rotary).
+int64_t attn_split_row_halfs(int hd);
+int attention_relayout_split(const float* qkv, int64_t ld, const f32x2* cs, const float* bound, int N, int Np, int H,
+                             int hd, void* Qo, void* Ko, void* Vo, hipStream_t stream);
+int attention_split(const void* Q, const void* K, const void* Vt, const int* items, int64_t n_items, int64_t n_whole,
+                    const float* bound, int Np, int H, int hd, float qscale, void* out, float* part, hipStream_t stream);
+int attention_combine_split(const int* d_tiles, int64_t n_tiles, int64_t n_whole, const float* part, const float* bound,
+                            void* out, int64_t ldo, int hd, hipStream_t stream);
 int pack_weight_bf16(const float* w, int64_t k_in, int64_t n_out, bf16* out, hipStream_t stream);
 // qvl_gather_rows with the identity order when idx is NULL and out columns [width, pad_to) zeroed.
 int gather_rows_pad(void* stream, int32_t src_dtype, const void* src, int64_t ld_src, int32_t dst_dtype, void* dst,

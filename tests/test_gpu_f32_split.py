@@ -144,6 +144,28 @@ def tower_pair(pkg, spec, params):
     return a, b
 
 
+@pytest.mark.parametrize("head_dim", [64, 72, 80])
+@pytest.mark.parametrize("grids", [[(1, 2, 2), (1, 6, 4), (2, 10, 14)], [(1, 28, 28)]])
+def test_split_tower_large_scores(pkg, head_dim, grids):
+    """Scores of some tens (the qkv weights 10 times the usual ones), segments of 4 to 784 keys, whole lists and key
+    parts: no further from the fp64 oracle than the fp32 MFMA kernels."""
+    from oracle import vision_tower as vt
+    spec = pkg.VisionBackboneSpec(hidden_size=16 * head_dim, out_hidden_size=128, depth=1, num_heads=16,
+                                  intermediate_size=256)
+    params = pkg.random_params(spec, seed=head_dim)
+    params["visual"]["blocks_0"]["attn"]["qkv"]["kernel"] *= 10
+    n = sum(t * h * w for t, h, w in grids)
+    px = np.random.default_rng(1).standard_normal((n, spec.patch_volume), dtype=np.float32)
+    ospec = vt.VisionSpec(hidden_size=16 * head_dim, out_hidden_size=128, depth=1, num_heads=16, intermediate_size=256,
+                          deepstack_visual_indexes=())
+    ref = torch.from_numpy(np.asarray(vt.encode_vision(params, px, grids, ospec, "fp64").tokens, np.float64))
+    err = []
+    for t in tower_pair(pkg, spec, params):
+        tokens, _ = t(px, np.array(grids, np.int32))
+        err.append(((tokens.double().cpu() - ref).norm() / ref.norm()).item())
+    assert err[0] <= max(err[1], 2e-7), err
+
+
 def test_split_tower_nan_stays_in_its_segment(pkg):
     spec = pkg.spec_2b()
     spec.depth, spec.deepstack_visual_indexes = 2, (0,)
