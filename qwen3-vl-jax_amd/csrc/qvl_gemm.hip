@@ -807,17 +807,22 @@ __global__ __launch_bounds__(64 * WM * WN, 1) void gemm_bf16_kernel(GemmParams p
     else
       wait_vmcnt_upto<S::XPT + S::WPT>(dma_per_stage);
   };
-  auto dma_stage = [&](int k0, int stage) {
+  // (part of parts: every parts-th instruction of the stage)
+  auto dma_part = [&](int k0, int stage, int part, int parts) {
     const uint32_t xa = lds_base + stage * S::LDS_ELEMS * 2, wa = xa + BM * kBK * 2;
 #pragma unroll
     for (int i = 0; i < S::XPT; ++i)
-      if (BM % S::ROWS_PER_PASS == 0 || i * S::ROWS_PER_PASS + wave * 8 < BM)   // wave-uniform
+      if (i % parts != part) continue;
+      else if (BM % S::ROWS_PER_PASS == 0 || i * S::ROWS_PER_PASS + wave * 8 < BM)   // wave-uniform
         dma16(rxw, xv, (uint32_t)((i * S::ROWS_PER_PASS * p.lda + k0) * 2), xa + (i * S::ROWS_PER_PASS + wave * 8) * kBK * 2);
 #pragma unroll
     for (int i = 0; i < S::WPT; ++i)
-      if (BN % S::ROWS_PER_PASS == 0 || i * S::ROWS_PER_PASS + wave * 8 < BN)
+      if ((S::XPT + i) % parts != part) continue;
+      else if (BN % S::ROWS_PER_PASS == 0 || i * S::ROWS_PER_PASS + wave * 8 < BN)
         dma16(rww, wv, (uint32_t)((i * S::ROWS_PER_PASS * p.K + k0) * 2), wa + (i * S::ROWS_PER_PASS + wave * 8) * kBK * 2);
   };
+
+  auto dma_stage = [&](int k0, int stage) { dma_part(k0, stage, 0, 1); };
 
   // The first k-step's operands (and with three stages the second's) are on their way while the
   // prologue below copies its tables.
@@ -911,13 +916,16 @@ __global__ __launch_bounds__(64 * WM * WN, 1) void gemm_bf16_kernel(GemmParams p
     const bf16* xs = smem + cur * S::LDS_ELEMS;
     const bool more = kt + 1 < kt1;
     const int nxt = NS == 3 ? (cur == 2 ? 0 : cur + 1) : (cur ^ 1);
-    if constexpr (NS == 3) {
-      if (kt + 2 < kt1) dma_stage((kt + 2) * kBK, cur == 0 ? 2 : cur - 1);
-    } else {
-      if (more) dma_stage((kt + 1) * kBK, nxt);
-    }
+    // Tiles of one wave a SIMD issue a quarter of the next stage's DMA beside each 16-deep k-step instead of all of it
+    // ahead of the first (the issue stalls the wave, and no other wave's MFMAs fill in): 64x128 tiles 0.56 -> 0.48 us per
+    // k-step.
+    constexpr bool SPREAD = WM * WN <= 6;
+    const bool fetch = NS == 3 ? kt + 2 < kt1 : more;
+    const int fetch_k = (NS == 3 ? kt + 2 : kt + 1) * kBK, fetch_to = NS == 3 ? (cur == 0 ? 2 : cur - 1) : nxt;
+    if (!SPREAD && fetch) dma_stage(fetch_k, fetch_to);
 #pragma unroll
     for (int ks = 0; ks < kBK / 16; ++ks) {
+      if (SPREAD && fetch) dma_part(fetch_k, fetch_to, ks, kBK / 16);
       if (ks + 1 < kBK / 16) read_frags(xs, ks + 1, (ks + 1) & 1);
       mfmas(ks & 1);
       if (ks + 1 < kBK / 16) {
@@ -1180,7 +1188,8 @@ static GemmPlan plan_gemm(const GemmParams& p, int cus, double macs_per_us_per_c
 
 // Tile-plan override of the calling thread (qvl_set_gemm_plan): tile 0 = the cost model's
 // choice, 1..4 = 288x256 | 256x256 | 256x128 | 288x128, 5 = the row split (whole rounds of 288x256,
-// the rest 256x128), 6 = 128x128, 7 = 64x192 (the head_dim-64 rotary qkv GEMM only), 8 = 64x128;
+// the rest 256x128), 6 = 128x128, 7 = 64x192 (the head_dim-64 rotary qkv GEMM only), 8 = 64x128,
+// 9 = the few-rows kernel (32x128, never split);
 // split_mode -1 forbids, 1 forces, 0 lets the cost model decide the tail split;
 // group_n 0 = the default panel width. Thread-local, so a test pinning a plan on one thread does
 // not change another thread's launches.
@@ -1233,6 +1242,210 @@ static int launch_gemm(GemmParams p, const GemmPlan& g, hipStream_t stream) {
   }
 }
 
+// ---------------------------------------------------------------------------------------------
+// GEMM for launches of few rows (one round of 32x128 tiles): what such a launch costs is not arithmetic or bytes but
+// the serial chain of each workgroup's K loop, so the loop is made as short as it can be. 8 waves share one 32x128
+// tile by K: of the 128-wide K step (two blocks of 64) wave w takes the 16 columns [16 (w % 4), +16) of block w / 4,
+// so every LDS fragment is read by one wave only (40 KB a step; a 64x128 tile of 2x2 waves reads 96 KB for the same
+// K), two waves a SIMD overlap DMA issue, LDS reads and MFMAs, and there is one barrier per 128 of K. The waves'
+// sums meet in LDS at the end, in wave order. MI355X, beyond a start of 4.5 us, per 64 of K: 0.19 us (0.28 with weights
+// from HBM), against 0.56 us on 64x128 tiles and 0.75 us on 128x128 (0.48 and 0.70 with the DMA spread over the step).
+// A fourth ring stage changed 1 % of a forward.
+// ---------------------------------------------------------------------------------------------
+constexpr int kFewBM = 32, kFewBN = 128;
+constexpr int kFewBlock = (kFewBM + kFewBN) * kBK;            // elements of one 64-wide K block of a stage
+constexpr int kFewRed = 8 * kFewBM * kFewBN * 4;              // bytes of the waves' sums (more than the ring)
+static_assert(3 * 2 * kFewBlock * 2 <= kFewRed, "the three-stage ring lies within the reduction buffer");
+
+// Above it: a folded LayerNorm's (c, d) and row statistics, the rotary epilogue's positions, the pos-embed's taps.
+template <int EPI, bool LN>
+__host__ __device__ constexpr int few_rows_lds_bytes() {
+  return kFewRed + (LN ? (kFewBM + kFewBN) * 8 : 0) + (EPI == kEpiQkvRope ? rope_table_lds_bytes(64, LN) : 0) +
+         (EPI == kEpiBiasPosEmbed ? kFewBM * 4 * 8 : 0);
+}
+
+template <int EPI, bool LN>
+__global__ __launch_bounds__(512, 2) void gemm_few_rows_kernel(GemmParams p) {
+  extern __shared__ __attribute__((aligned(16))) bf16 smem[];
+  constexpr int BM = kFewBM, BN = kFewBN;
+  const int tiles_n = (p.N + BN - 1) / BN, tiles_m = (max(p.M, p.Np) + BM - 1) / BM;
+  int tm, tn;
+  tile_coords(xcd_remap(blockIdx.x, gridDim.x), tiles_m, tiles_n, p.group_n, tm, tn);
+  const int m0 = tm * BM, n0 = tn * BN;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l32 = lane & 31, hh = lane >> 5, blk = wave >> 2, wq = wave & 3;
+  const int KB = p.K / kBK, steps = (KB + 1) / 2;             // 64-wide blocks; an odd count leaves the last step half
+
+  // Operand DMA (as in gemm_bf16_kernel): wave (blk, wq) fetches rows [8 wq, +8) of x and rows 32 i + [8 wq, +8) of w
+  // of its block.
+  const int r8 = wq * 8 + (lane >> 3), ch = (lane & 7) ^ ((r8 >> 1) & 7);
+  const uint32_t xv = (uint32_t)(((int64_t)(m0 + r8) * p.lda + ch * 8) * 2);
+  const uint32_t wv = (uint32_t)(((int64_t)(n0 + r8) * p.K + ch * 8) * 2);
+  const u32x4 rxw = rsrc_words(p.x, (uint32_t)((int64_t)p.M * p.lda * 2));
+  const u32x4 rww = rsrc_words(p.w, (uint32_t)((int64_t)p.N * p.K * 2));
+  const uint32_t lds_base = lds_addr_of(smem) + blk * kFewBlock * 2 + wq * 8 * kBK * 2;
+  auto has = [&](int s) { return 2 * s + blk < KB; };          // this wave's block of step s exists
+  auto dma_step = [&](int s, int slot) {
+    const uint32_t k2 = (uint32_t)(2 * s + blk) * kBK * 2, at = lds_base + slot * 2 * kFewBlock * 2;
+    dma16(rxw, xv, k2, at);
+#pragma unroll
+    for (int i = 0; i < BN / 32; ++i) dma16(rww, wv, (uint32_t)(32 * i * p.K * 2) + k2, at + (BM + 32 * i) * kBK * 2);
+  };
+  if (has(0)) dma_step(0, 0);
+  if (has(1)) dma_step(1, 1);
+
+  // tables for the epilogue, above the reduction buffer (published by the barriers below)
+  char* extra = reinterpret_cast<char*>(smem) + kFewRed;
+  f32x2* lcd = reinterpret_cast<f32x2*>(extra);
+  if constexpr (LN) {
+    for (int i = tid; i < BN + BM; i += 512) {
+      if (i < BN) {
+        lcd[i] = n0 + i < p.N ? p.ln_cd[n0 + i] : f32x2{0.f, 0.f};
+      } else {
+        const f32x2 st = ln_row(p, m0 + i - BN);
+        lcd[i] = f32x2{st.y, -st.x * st.y};
+      }
+    }
+    extra += (BM + BN) * 8;
+  }
+  const uint32_t* ltab = nullptr;
+  if constexpr (EPI == kEpiQkvRope) {
+    if (p.rtab) {
+      uint32_t* t = reinterpret_cast<uint32_t*>(extra);
+      for (int i = tid; i < p.rtab_pos * (p.cs_half / 2); i += 512) t[i] = p.rtab[i];
+      ltab = t;
+    }
+  }
+  int2* ltaps = reinterpret_cast<int2*>(extra);
+  if constexpr (EPI == kEpiBiasPosEmbed) {
+    if (tid < BM * 4) {
+      const int m = m0 + (tid >> 2), j = tid & 3;
+      ltaps[tid] = m < p.M ? int2{p.pe_idx[(int64_t)j * p.M + m], __float_as_int(p.pe_w[(int64_t)j * p.M + m])} : int2{0, 0};
+    }
+  }
+
+  f32x16 acc[BN / 32];
+#pragma unroll
+  for (int a = 0; a < BN / 32; ++a) acc[a] = f32x16{};
+  int slot = 0;
+  for (int s = 0; s < steps; ++s) {
+    if (has(s + 1)) wait_vmcnt<1 + BN / 32>();                    // only the next step's DMA may be in flight
+    else wait_dma();
+    __syncthreads();                                              // step s is in LDS; step s - 1's slot is free
+    bf16x8 xf, wf[BN / 32];
+    const bool mine = has(s);
+    if (mine) {
+      const bf16* xs = smem + slot * 2 * kFewBlock + blk * kFewBlock;
+      xf = *reinterpret_cast<const bf16x8*>(xs + lds_off(l32, wq * 2 + hh));
+#pragma unroll
+      for (int a = 0; a < BN / 32; ++a)
+        wf[a] = *reinterpret_cast<const bf16x8*>(xs + BM * kBK + lds_off(a * 32 + l32, wq * 2 + hh));
+    }
+    if (has(s + 2)) dma_step(s + 2, slot == 0 ? 2 : slot - 1);
+    if (mine) {
+#pragma unroll
+      for (int a = 0; a < BN / 32; ++a) acc[a] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf[a], xf, acc[a], 0, 0, 0);
+    }
+    slot = slot == 2 ? 0 : slot + 1;
+  }
+
+  // The waves' sums, [wave][row][feature] fp32 with 16-byte chunks XOR-swizzled by row; then every thread adds its
+  // outputs' 8 terms in wave order.
+  float* red = reinterpret_cast<float*>(smem);
+  __syncthreads();
+#pragma unroll
+  for (int a = 0; a < BN / 32; ++a)
+#pragma unroll
+    for (int g = 0; g < 4; ++g)
+      *reinterpret_cast<f32x4*>(red + (wave * BM + l32) * BN + (((8 * a + 2 * g + hh) ^ l32) << 2)) =
+          f32x4{acc[a][4 * g], acc[a][4 * g + 1], acc[a][4 * g + 2], acc[a][4 * g + 3]};
+  __syncthreads();
+  const int r = tid >> 4, m = m0 + r;
+  auto sum4 = [&](int chunk, float (&v)[4]) {
+    f32x4 t = *reinterpret_cast<const f32x4*>(red + r * BN + ((chunk ^ r) << 2));
+#pragma unroll
+    for (int w = 1; w < 8; ++w) t += *reinterpret_cast<const f32x4*>(red + (w * BM + r) * BN + ((chunk ^ r) << 2));
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = t[e];
+    if constexpr (LN) {
+      const f32x2 rs = lcd[BN + r];
+      ln_fold_group(lcd, rs.x, rs.y, chunk * 4, v);
+    }
+  };
+  if constexpr (EPI == kEpiQkvRope) {
+    // thread: token r, head h2 of the tile's two, dims d..d+3 and d+32..d+35 (a tile lies in one of q, k, v)
+    const int h2 = (tid >> 3) & 1, d = (tid & 7) * 4, n = n0 + h2 * 64 + d;
+    const int which = n0 / p.D, head = (n0 % p.D) / 64 + h2;
+    float lo[4], hi[4];
+    sum4(h2 * 16 + d / 4, lo);
+    sum4(h2 * 16 + d / 4 + 8, hi);
+    const f32x4 blo = *reinterpret_cast<const f32x4*>(p.bias + n), bhi = *reinterpret_cast<const f32x4*>(p.bias + n + 32);
+    f32x4 c01 = {}, c23 = {};
+    if (which < 2) {
+      if (ltab) {
+        int ph, pw;
+        token_pos(p, m, ph, pw);
+        const u32x4 q = *reinterpret_cast<const u32x4*>(ltab + (d < 16 ? ph : pw) * 16 + (d & 15));
+        const uint32_t w[4] = {q.x, q.y, q.z, q.w};
+        unpack_cs4(w, c01, c23);
+      } else {
+        rope_cs_global(p, m, d, c01, c23);
+      }
+    }
+    u32x2 o1, o2;
+    rope_values(p, which, m, d, blo, bhi, lo, hi, c01, c23, o1, o2);
+    if (which < 2) {
+      if (m >= p.Np) return;
+      bf16* dst = (which == 0 ? p.q : p.k) + ((int64_t)head * p.Np + m) * 64;
+      *reinterpret_cast<u32x2*>(dst + d) = o1;
+      *reinterpret_cast<u32x2*>(dst + d + 32) = o2;
+      return;
+    }
+    // v: turned through LDS into 16-byte runs of 8 key positions
+    constexpr int VS = BM + 8;
+    bf16* vb = smem;
+    __syncthreads();
+    const uint32_t w[4] = {o1.x, o1.y, o2.x, o2.y};
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      vb[(h2 * 64 + d + e) * VS + vt_pos(r)] = __builtin_bit_cast(bf16, (uint16_t)(w[e >> 1] >> (16 * (e & 1))));
+      vb[(h2 * 64 + d + e + 32) * VS + vt_pos(r)] = __builtin_bit_cast(bf16, (uint16_t)(w[2 + (e >> 1)] >> (16 * (e & 1))));
+    }
+    __syncthreads();
+    const int f = tid >> 2, run = (tid & 3) * 8;
+    if (m0 + run < p.Np)
+      *reinterpret_cast<u32x4*>(p.vt + ((int64_t)((n0 % p.D) / 64 + (f >> 6)) * 64 + (f & 63)) * p.Np + m0 + run) =
+          *reinterpret_cast<const u32x4*>(vb + f * VS + run);
+  } else {
+    // thread: row r, features n..n+7; 16 consecutive threads hold a row's 128 columns
+    const int n = n0 + (tid & 15) * 8;
+    if (m >= p.M || n >= p.N) return;
+    float lo[4], hi[4];
+    sum4((tid & 15) * 2, lo);
+    sum4((tid & 15) * 2 + 1, hi);
+    const bool full = n + 8 <= p.N, vec16 = ((p.ldc | (EPI == kEpiBiasResidual ? p.ldr : 0)) & 7) == 0;
+    const f32x4 b0 = *reinterpret_cast<const f32x4*>(p.bias + n);
+    const f32x4 b1 = full ? *reinterpret_cast<const f32x4*>(p.bias + n + 4) : f32x4{};
+    const u32x4 raw = {pack_bf16x2(lo[0], lo[1]), pack_bf16x2(lo[2], lo[3]), pack_bf16x2(hi[0], hi[1]), pack_bf16x2(hi[2], hi[3])};
+    const u32x4 out = epi_store_oct<EPI>(p, m, n, raw, b0, b1, full, vec16, ltaps + 4 * r);
+    if constexpr (EPI == kEpiBiasResidual || EPI == kEpiBiasPosEmbed)
+      if (p.rs_part) row_group_stats(p, m, n, out);
+  }
+}
+
+template <int EPI, bool LN>
+static int launch_few_rows(GemmParams p, hipStream_t stream) {
+  constexpr int lds_max = few_rows_lds_bytes<EPI, LN>();
+  static_assert(lds_max <= 163840, "LDS budget");
+  static const hipError_t attr_rc = hipFuncSetAttribute((const void*)gemm_few_rows_kernel<EPI, LN>,
+                                                        hipFuncAttributeMaxDynamicSharedMemorySize, lds_max);
+  if (attr_rc != hipSuccess) return set_error(QVL_ERR_LAUNCH, "gemm_few_rows: cannot reserve %d bytes of LDS", lds_max);
+  const int tiles_n = (p.N + kFewBN - 1) / kFewBN, tiles = ((std::max(p.M, p.Np) + kFewBM - 1) / kFewBM) * tiles_n;
+  p.group_n = gemm_group_n(tiles_n);
+  hipLaunchKernelGGL((gemm_few_rows_kernel<EPI, LN>), dim3(tiles), dim3(512), lds_max, stream, p);
+  return check_launch("gemm_few_rows");
+}
+
 // Tile choice by the cost model above. Shapes (per-CU MAC rates measured on the tower's GEMMs):
 //   288x256 on 12 waves (three per SIMD, 96x64 each): 64 row tiles cover 18432 tokens, so the
 //     N = 1024 / 3072 / 4096 GEMMs fill exactly 1 / 3 / 4 rounds of 256 CUs;
@@ -1272,59 +1485,48 @@ static int dispatch_gemm(const GemmParams& p, hipStream_t stream) {
   const GemmPlan r_b = plan_gemm<256, 128>(rb, cus, kRate256x128, -1);
   const double r_cost = can_split && r_b.full <= cus ? r_a.cost_us + r_b.cost_us : 1e30;
   int pick = f.tile;
+  if (pick == 9) return launch_few_rows<EPI, LN>(p, stream);
   if (EPI == kEpiQkvRope && pick == 4) pick = 3;     // 64-feature heads need TN % 64 == 0 (288x128: 32)
   if (pick == 5 && !can_split) pick = 1;
-  // Small grids, K <= 1536: where one round of 128x128 tiles would cover half to all of the CUs,
-  // 64x128 tiles unsplit (4 waves of 32x64); where fewer 128x128 tiles split along K in up to 8
-  // parts fill at least 7/8 of the CUs, those (4 waves of 64x64). The larger tiles there leave most
-  // CUs idle or need long split-K tails. One 784-token image's forward: fc1 16.1 us on 128x128
-  // against 21.3 on 256x128 (64x128: below); proj, 56 tiles in 4 parts, 15.4 against 18.9 us for
-  // 288x128 tiles in 8 parts. Cases the rules leave to the cost model were measured slower on
-  // 128x128: 1568 rows' proj unsplit (104 tiles) 22.9 against 20.4 us; the mergers' K = 4096 GEMMs
-  // at 196 rows 25.2 / 26.8 against 20.3 / 24.2 us.
+  // One round of 32x128 tiles: the few-rows kernel (gemm_few_rows_kernel). Alone, cold weights: 784 x 1024 x 1024 7.8 us
+  // against 19.9 for 128x128 tiles split along K and their reduction, 784 x 1024 x 4096 17.8 against 26.0, 196 x 4096 x
+  // 1024 7.6 against 23.1, 196 x 4096 x 4096 23.3 against 25.4, 256 x 4096 x 1024 8.2 against 22.8; two rounds of it lose
+  // to 64x128 tiles (400 x 3072 x 1024 13.1 against 12.2, 784 x 4096 x 1024 23.3 against 13.4). Weights past 4096 x 4352
+  // on few rows stay with the split plans (49 x 4608 x 4608 28.4 against 26.1; at 196 rows 27.6 against 30.2).
+  const bool whole = pick == 0 && !p.row0 && !p.row1;
+  if (whole && f.split_mode <= 0 && ((rows + kFewBM - 1) / kFewBM) * ((p.N + kFewBN - 1) / kFewBN) <= cus &&
+      (rows > 128 || (int64_t)p.N * p.K <= 4096 * 4352))
+    return launch_few_rows<EPI, LN>(p, stream);
   // The head_dim-64 rotary qkv GEMM takes 64x192 tiles (6 waves of 32x64, whole heads; tiles may
   // straddle the q | k | v boundary, the epilogue picks the target per head) wherever one round of
-  // them fits the CUs: alone on MI355X (1024 x 3072 x 1024 with norm1 folded), 196 / 400 / 576 /
-  // 784 / 1024 tokens 14.3 / 14.5 / 14.7 / 15.3 / 15.4 us against 19.8 / 20.2 / 20.2 / 17.0 / 17.5
-  // for the plans below; at 1568 tokens and more (two rounds) the plans below stay ahead.
+  // them fits the CUs: alone on MI355X (K = 1024 with norm1 folded), 400 / 784 / 1024 tokens 14.5 /
+  // 15.3 / 15.4 us against 20.2 / 17.0 / 17.5 for the plans below; at 1568 tokens and more (two
+  // rounds) the plans below stay ahead.
   GemmPlan e{};
   if (pick == 6) e = plan_gemm<128, 128>(p, cus, kRate128x128, f.split_mode);
   if constexpr (EPI == kEpiQkvRope) {
     const int tiles64 = ((rows + 63) / 64) * ((p.N + 191) / 192);
-    if (pick == 0 && p.K <= kSmallTileMaxK && tiles64 <= cus && !p.row0 && !p.row1) pick = 7;
+    if (whole && p.K <= kSmallTileMaxK && tiles64 <= cus) pick = 7;
   }
+  // Short K, up to one full round of 128x128 tiles: 64x128 tiles unsplit (4 waves of 32x64, two workgroups per CU). Alone:
+  // 400 x 3072 x 1024 12.2 us against 22.5 for 256x128 tiles split along K, 1404 x 1024 x 1024 11.5 against 22.7, fc1 at
+  // 784 rows 13.4 against 15.8 on 128x128. A full round of 128x128 tiles stays on them (fc1 at 1024 rows: two full
+  // rounds of 64x128 made the forward 0.9 % slower), and so does the rotary qkv (64x128: 24-26 against 17.7 us).
   const int tiles128 = ((rows + 127) / 128) * ((p.N + 127) / 128);
-  if (pick == 0 && p.K <= kSmallTileMaxK && !p.row0 && !p.row1) {
-    if (2 * tiles128 >= cus && tiles128 <= cus) {
-      // below a full round of 128x128 tiles, one to two rounds of 64x128 run ahead (alone: fc1 at
-      // 784 rows 14.8 against 15.8 us, the 8B fc1 16.3 against 17.2, proj at 2304 rows 16.1 against
-      // 20.6; in the forward a 2304-patch image 4.013 -> 3.889 ms); a full round stays on 128x128
-      // (fc1 at 1024 rows: two full rounds of 64x128 made the forward 0.9 % slower); the head_dim-64
-      // rotary qkv stays on 128x128 (64x128: 24-26 against 17.7 us at 784 tokens)
-      if (tiles128 < cus && EPI != kEpiQkvRope) {
-        pick = 8;
-        e = plan_gemm<64, 128>(p, cus, kRate128x128, -1);
-      } else {
-        pick = 6;
-        e = plan_gemm<128, 128>(p, cus, kRate128x128, -1);
-      }
-    } else if (f.split_mode >= 0 && 2 * tiles128 < cus) {
-      const GemmPlan sp = plan_gemm<128, 128>(p, cus, kRate128x128, 1);
-      if (8 * sp.tail * sp.split >= 7 * cus) {
-        pick = 6;
-        e = sp;
-      }
-    } else if (EPI == kEpiBiasPosEmbed && ((rows + 63) / 64) * ((p.N + 127) / 128) <= cus) {
-      // the patch embed cannot split K: its small grids take 64x128 tiles (4 waves of 32x64) that
-      // fit one round (one 784-token image: 104 tiles, 23.5 against 37.9 us for 32 of 256x128)
+  if (pick == 0 && whole && p.K <= kSmallTileMaxK && tiles128 <= cus) {
+    if (tiles128 < cus && EPI != kEpiQkvRope && f.split_mode <= 0) {
       pick = 8;
+      e = plan_gemm<64, 128>(p, cus, kRate128x128, -1);
+    } else if (2 * tiles128 >= cus) {
+      pick = 6;
+      e = plan_gemm<128, 128>(p, cus, kRate128x128, -1);
     }
   }
   // Long K (fc2, K = 4096 / 4352) from 512 rows: 128x128 tiles split along K where up to 8 parts fill
   // at least 7/8 of the CUs (one 784-token image's fc2: 23.9 against 25.2 us for 288x128 tiles in 8
   // parts); at the mergers' 196 rows the cost model's plans stay ahead (25.2 / 26.8 against 20.3 /
   // 24.2 us on 128x128).
-  if (pick == 0 && p.K > kSmallTileMaxK && rows >= 512 && f.split_mode >= 0 && !p.row0 && !p.row1 &&
+  if (pick == 0 && whole && p.K > kSmallTileMaxK && rows >= 512 && f.split_mode >= 0 &&
       EPI != kEpiBiasPosEmbed && 2 * tiles128 < cus) {
     const GemmPlan sp = plan_gemm<128, 128>(p, cus, kRate128x128, 1);
     if (8 * sp.tail * sp.split >= 7 * cus) {
@@ -1336,7 +1538,7 @@ static int dispatch_gemm(const GemmParams& p, hipStream_t stream) {
   // combines each row's partials in the workgroup's prologue; on small grids 64-row tiles split
   // along K spread that over 4x the workgroups (one 784-token image's deepstack fc1, K = 4096:
   // 27.2 against 33.4 us for 256x128 tiles split 8 ways).
-  if (pick == 0 && LN && p.ln_part && p.ln_groups > 16 && f.split_mode >= 0 && !p.row0 && !p.row1 &&
+  if (pick == 0 && whole && LN && p.ln_part && p.ln_groups > 16 && f.split_mode >= 0 &&
       2 * ((rows + 63) / 64) * ((p.N + 127) / 128) <= cus) {
     const GemmPlan sp = plan_gemm<64, 128>(p, cus, kRate128x128, 1);
     if (8 * sp.tail * sp.split >= 7 * cus) {
@@ -1374,7 +1576,7 @@ static int dispatch_gemm(const GemmParams& p, hipStream_t stream) {
 }
 
 int gemm_set_plan(int tile, int split_mode, int group_n) {
-  if (tile < 0 || tile > 8 || split_mode < -1 || split_mode > 1 || group_n < 0)
+  if (tile < 0 || tile > 9 || split_mode < -1 || split_mode > 1 || group_n < 0)
     return set_error(QVL_ERR_INVALID_ARG, "gemm plan: tile=%d split_mode=%d group_n=%d", tile, split_mode, group_n);
   t_plan.tile = tile;
   t_plan.split_mode = split_mode;
