@@ -753,6 +753,30 @@ __device__ __forceinline__ void wait_vmcnt_upto(int n) {
   wait_vmcnt<MAX>();
 }
 
+// The next GEMM's weights, read once by n_wg workgroups that have no tile (wg: this one's number): the loads bring them
+// from HBM into the memory-side cache while the tiles compute. Without it a launch of few rows, bound by the latency of
+// its serial K loop, pays HBM's latency in every step: 784 x 1024 x 4096 24 us with its weights in HBM, 17.8 with them in
+// the cache.
+__device__ __forceinline__ void read_next_weights(const GemmParams& p, int wg, int n_wg) {
+  const u32x4* src = reinterpret_cast<const u32x4*>(p.next_w);
+  const int64_t n = p.next_bytes / 16, step = (int64_t)n_wg * blockDim.x;
+  int64_t i = (int64_t)wg * blockDim.x + threadIdx.x;
+  for (; i + 7 * step < n; i += 8 * step) {
+    u32x4 v[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[j] = src[i + j * step];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) asm volatile("" :: "v"(v[j]));   // (a use: the loads stay)
+  }
+  for (; i < n; i += step) {
+    const u32x4 v = src[i];
+    asm volatile("" :: "v"(v));
+  }
+}
+
+template <int BM, int BN>
+constexpr bool kReadsNext = BM * BN <= 64 * 288;   // the small tiles; the others' launches have no workgroup to spare
+
 template <int BM, int BN, int WM, int WN, int EPI, bool LN>
 __global__ __launch_bounds__(64 * WM * WN, 1) void gemm_bf16_kernel(GemmParams p) {
   using S = GemmShape<BM, BN, WM, WN>;
@@ -768,6 +792,8 @@ __global__ __launch_bounds__(64 * WM * WN, 1) void gemm_bf16_kernel(GemmParams p
     tile = xcd_remap(blockIdx.x, p.full_tiles);
   } else {
     unit = blockIdx.x - p.full_tiles;
+    if constexpr (kReadsNext<BM, BN>)
+      if (p.next_w) return read_next_weights(p, unit, gridDim.x - p.full_tiles);
     tile = p.full_tiles + unit / p.split;
     const int s = unit % p.split;
     kt0 = s * KT / p.split;
@@ -1202,6 +1228,22 @@ static int gemm_group_n(int tiles_n) {
   return std::max(1, std::min(g, tiles_n));
 }
 
+// Workgroups past a launch's tiles for read_next_weights: as many as the first round leaves free, of 256 KB at most each,
+// so that they end before the tiles do. Forwards of three 2B blocks and two mergers, weights in HBM: 196 patches 314 ->
+// 291 us, 400 339 -> 317, 784 358 -> 346 (8B 424 -> 412); with more rows the weights' latency no longer shows (1024 379.6
+// -> 381, 1440 496.5 -> 499.6), so none there.
+constexpr int kNextMaxRows = 896, kNextMaxGroups = 192, kNextBytes = 256 * 1024;
+
+static int next_weight_groups(GemmParams& p, int tiles, int slots) {
+  const int n = std::min<int64_t>(std::min(slots - tiles, kNextMaxGroups), (p.next_bytes + 32767) / 32768);
+  if (!p.next_w || n <= 0 || std::max(p.M, p.Np) > kNextMaxRows) {
+    p.next_w = nullptr;
+    return 0;
+  }
+  p.next_bytes = std::min<int64_t>(p.next_bytes, (int64_t)n * kNextBytes);
+  return n;
+}
+
 template <int BM, int BN, int WM, int WN, int EPI, bool LN>
 static int launch_gemm(GemmParams p, const GemmPlan& g, hipStream_t stream) {
   using S = GemmShape<BM, BN, WM, WN>;
@@ -1223,7 +1265,9 @@ static int launch_gemm(GemmParams p, const GemmPlan& g, hipStream_t stream) {
   p.full_tiles = g.full;
   p.split = g.split;
   p.group_n = gemm_group_n((p.N + BN - 1) / BN);
-  const int grid = g.full + g.tail * g.split;
+  if (g.tail || !kReadsNext<BM, BN>) p.next_w = nullptr;
+  const int slots = gemm_device_cus() * (2 * lds <= 163840 && S::THREADS <= 512 ? 2 : 1);
+  const int grid = g.full + (g.tail ? g.tail * g.split : next_weight_groups(p, g.full, slots));
   hipLaunchKernelGGL((gemm_bf16_kernel<BM, BN, WM, WN, EPI, LN>), dim3(grid), dim3(S::THREADS), lds, stream, p);
   int rc = check_launch("gemm_bf16");
   if (rc || g.tail == 0) return rc;
@@ -1270,7 +1314,8 @@ __global__ __launch_bounds__(512, 2) void gemm_few_rows_kernel(GemmParams p) {
   constexpr int BM = kFewBM, BN = kFewBN;
   const int tiles_n = (p.N + BN - 1) / BN, tiles_m = (max(p.M, p.Np) + BM - 1) / BM;
   int tm, tn;
-  tile_coords(xcd_remap(blockIdx.x, gridDim.x), tiles_m, tiles_n, p.group_n, tm, tn);
+  if ((int)blockIdx.x >= p.full_tiles) return read_next_weights(p, blockIdx.x - p.full_tiles, gridDim.x - p.full_tiles);
+  tile_coords(xcd_remap(blockIdx.x, p.full_tiles), tiles_m, tiles_n, p.group_n, tm, tn);
   const int m0 = tm * BM, n0 = tn * BN;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l32 = lane & 31, hh = lane >> 5, blk = wave >> 2, wq = wave & 3;
@@ -1442,7 +1487,9 @@ static int launch_few_rows(GemmParams p, hipStream_t stream) {
   if (attr_rc != hipSuccess) return set_error(QVL_ERR_LAUNCH, "gemm_few_rows: cannot reserve %d bytes of LDS", lds_max);
   const int tiles_n = (p.N + kFewBN - 1) / kFewBN, tiles = ((std::max(p.M, p.Np) + kFewBM - 1) / kFewBM) * tiles_n;
   p.group_n = gemm_group_n(tiles_n);
-  hipLaunchKernelGGL((gemm_few_rows_kernel<EPI, LN>), dim3(tiles), dim3(512), lds_max, stream, p);
+  p.full_tiles = tiles;
+  const int more = next_weight_groups(p, tiles, gemm_device_cus());
+  hipLaunchKernelGGL((gemm_few_rows_kernel<EPI, LN>), dim3(tiles + more), dim3(512), lds_max, stream, p);
   return check_launch("gemm_few_rows");
 }
 

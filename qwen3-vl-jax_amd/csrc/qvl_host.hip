@@ -44,11 +44,14 @@ int qvl_cast(void* stream, int32_t dtype, const float* x, void* y, int64_t n) {
   return cast_f32_bf16(x, (bf16*)y, n, (hipStream_t)stream);
 }
 
+// The weights the caller's next GEMM reads, where it knows them (GemmParams::next_w).
+struct NextWeights { const void* w = nullptr; int64_t bytes = 0; };
+
 static int dense_impl(void* stream, int32_t dtype, int32_t epi, const void* x, int64_t lda, const void* w,
                       const float* bias, const void* res, int64_t ldr, void* y, int64_t ldc, int64_t m, int64_t n,
                       int64_t k, void* ws, size_t ws_bytes, const float* ln_cd = nullptr,
                       const float* ln_stats = nullptr, const float* ln_part = nullptr, int ln_groups = 0,
-                      float ln_eps = 0.f, float* rs_part = nullptr) {
+                      float ln_eps = 0.f, float* rs_part = nullptr, NextWeights next = {}) {
   if (dtype != QVL_DTYPE_BF16 && dtype != QVL_DTYPE_F32) return set_error(QVL_ERR_UNSUPPORTED, "dense: dtype %d", dtype);
   if (epi < QVL_EPI_BIAS || epi > QVL_EPI_BIAS_RESIDUAL) return set_error(QVL_ERR_INVALID_ARG, "dense: epilogue %d", epi);
   if (m < 0 || n <= 0 || k <= 0) return set_error(QVL_ERR_INVALID_ARG, "dense: m=%lld n=%lld k=%lld", (long long)m, (long long)n, (long long)k);
@@ -90,6 +93,8 @@ static int dense_impl(void* stream, int32_t dtype, int32_t epi, const void* x, i
   p.ln_groups = ln_groups;
   p.ln_eps = ln_eps;
   p.rs_part = (f32x2*)rs_part;
+  p.next_w = next.w;
+  p.next_bytes = next.bytes;
   return gemm_bf16(p, epi, (hipStream_t)stream);
 }
 
@@ -270,7 +275,8 @@ static int qkv_rotary_impl(void* stream, int32_t dtype, const void* x, int64_t l
                            const void* cs, const int32_t* pos_hw, const uint32_t* rtab, int32_t n_pos, void* q,
                            void* k, void* vt, int64_t n_tokens, int64_t hidden, int32_t H, void* ws, size_t ws_bytes,
                            const float* ln_cd = nullptr, const float* ln_stats = nullptr,
-                           const float* ln_part = nullptr, int ln_groups = 0, float ln_eps = 0.f) {
+                           const float* ln_part = nullptr, int ln_groups = 0, float ln_eps = 0.f,
+                           NextWeights next = {}) {
   if (dtype != QVL_DTYPE_BF16) return set_error(QVL_ERR_UNSUPPORTED, "qkv_rotary: dtype %d", dtype);
   const bool ln = ln_stats || ln_part;
   if (H <= 0 || (hidden != (int64_t)H * 64 && hidden != (int64_t)H * 72))
@@ -307,6 +313,8 @@ static int qkv_rotary_impl(void* stream, int32_t dtype, const void* x, int64_t l
   p.ln_part = (const f32x2*)ln_part;
   p.ln_groups = ln_groups;
   p.ln_eps = ln_eps;
+  p.next_w = next.w;
+  p.next_bytes = next.bytes;
   return gemm_bf16(p, hd == 64 ? kEpiQkvRope : kEpiQkvRope72, (hipStream_t)stream);
 }
 
@@ -349,23 +357,28 @@ static int check_ln_parts(const char* what, int64_t rows, int64_t cols, const fl
   return QVL_OK;
 }
 
-int qvl_dense_rowstats_ws(void* stream, int32_t dtype, const void* x, int64_t lda, const void* w, const float* bias,
-                          const void* res, int64_t ldr, void* y, int64_t ldc, int64_t m, int64_t n, int64_t k,
-                          float* parts, void* ws, size_t ws_bytes) {
+static int dense_rowstats_ws_impl(void* stream, int32_t dtype, const void* x, int64_t lda, const void* w,
+                                  const float* bias, const void* res, int64_t ldr, void* y, int64_t ldc, int64_t m,
+                                  int64_t n, int64_t k, float* parts, void* ws, size_t ws_bytes, NextWeights next) {
   if (dtype != QVL_DTYPE_BF16) return set_error(QVL_ERR_UNSUPPORTED, "dense_rowstats: dtype %d (bf16 only)", dtype);
   if (n % 128) return set_error(QVL_ERR_UNSUPPORTED, "dense_rowstats: n=%lld not a multiple of 128", (long long)n);
   if (m > 0 && !parts) return set_error(QVL_ERR_INVALID_ARG, "dense_rowstats: NULL partials");
   if (((uintptr_t)parts & 7) || ldc % 8 || ldr % 8)
     return set_error(QVL_ERR_MISALIGNED, "dense_rowstats: partials 8-byte aligned, ldc and ldr multiples of 8");
   return dense_impl(stream, dtype, QVL_EPI_BIAS_RESIDUAL, x, lda, w, bias, res, ldr, y, ldc, m, n, k, ws, ws_bytes,
-                    nullptr, nullptr, nullptr, 0, 0.f, parts);
+                    nullptr, nullptr, nullptr, 0, 0.f, parts, next);
 }
 
-int qvl_dense_pos_embed_ws(void* stream, int32_t dtype, const void* x, int64_t lda, const void* w, const float* bias,
-                           const void* table, const int32_t* tap_idx, const float* tap_w, void* y, int64_t ldc,
-                           int64_t m, int64_t n, int64_t k, float* parts, void* ws, size_t ws_bytes) {
-  (void)ws;
-  (void)ws_bytes;
+int qvl_dense_rowstats_ws(void* stream, int32_t dtype, const void* x, int64_t lda, const void* w, const float* bias,
+                          const void* res, int64_t ldr, void* y, int64_t ldc, int64_t m, int64_t n, int64_t k,
+                          float* parts, void* ws, size_t ws_bytes) {
+  return dense_rowstats_ws_impl(stream, dtype, x, lda, w, bias, res, ldr, y, ldc, m, n, k, parts, ws, ws_bytes, {});
+}
+
+static int dense_pos_embed_ws_impl(void* stream, int32_t dtype, const void* x, int64_t lda, const void* w,
+                                   const float* bias, const void* table, const int32_t* tap_idx, const float* tap_w,
+                                   void* y, int64_t ldc, int64_t m, int64_t n, int64_t k, float* parts,
+                                   NextWeights next) {
   if (dtype != QVL_DTYPE_BF16) return set_error(QVL_ERR_UNSUPPORTED, "dense_pos_embed: dtype %d (bf16 only)", dtype);
   if (m < 0 || n <= 0 || k <= 0 || k % 64 || n % 8)
     return set_error(QVL_ERR_INVALID_ARG, "dense_pos_embed: m=%lld n=%lld (multiple of 8) k=%lld (multiple of 64)",
@@ -389,18 +402,50 @@ int qvl_dense_pos_embed_ws(void* stream, int32_t dtype, const void* x, int64_t l
   p.pe_table = (const bf16*)table;
   p.pe_idx = tap_idx;
   p.pe_w = tap_w;
+  p.next_w = next.w;
+  p.next_bytes = next.bytes;
   return gemm_bf16(p, kEpiBiasPosEmbed, (hipStream_t)stream);
 }
 
-int qvl_dense_ln_parts_ws(void* stream, int32_t dtype, int32_t epi, const void* x, int64_t lda, const void* w,
-                          const float* cd, const float* parts, int32_t groups, float eps, const float* bias, void* y,
-                          int64_t ldc, int64_t m, int64_t n, int64_t k, void* ws, size_t ws_bytes) {
+int qvl_dense_pos_embed_ws(void* stream, int32_t dtype, const void* x, int64_t lda, const void* w, const float* bias,
+                           const void* table, const int32_t* tap_idx, const float* tap_w, void* y, int64_t ldc,
+                           int64_t m, int64_t n, int64_t k, float* parts, void* ws, size_t ws_bytes) {
+  (void)ws;
+  (void)ws_bytes;
+  return dense_pos_embed_ws_impl(stream, dtype, x, lda, w, bias, table, tap_idx, tap_w, y, ldc, m, n, k, parts, {});
+}
+
+static int dense_ln_parts_ws_impl(void* stream, int32_t dtype, int32_t epi, const void* x, int64_t lda, const void* w,
+                                  const float* cd, const float* parts, int32_t groups, float eps, const float* bias,
+                                  void* y, int64_t ldc, int64_t m, int64_t n, int64_t k, void* ws, size_t ws_bytes,
+                                  NextWeights next) {
   if (dtype != QVL_DTYPE_BF16) return set_error(QVL_ERR_UNSUPPORTED, "dense_ln_parts: dtype %d (bf16 only)", dtype);
   if (epi != QVL_EPI_BIAS && epi != QVL_EPI_BIAS_GELU)
     return set_error(QVL_ERR_INVALID_ARG, "dense_ln_parts: epilogue %d (bias or bias+GELU)", epi);
   QVL_TRY_RC(check_ln_parts("dense_ln_parts", m, k, cd, parts, groups, eps));
   return dense_impl(stream, dtype, epi, x, lda, w, bias, nullptr, 0, y, ldc, m, n, k, ws, ws_bytes, cd, nullptr,
-                    parts, groups, eps);
+                    parts, groups, eps, nullptr, next);
+}
+
+int qvl_dense_ln_parts_ws(void* stream, int32_t dtype, int32_t epi, const void* x, int64_t lda, const void* w,
+                          const float* cd, const float* parts, int32_t groups, float eps, const float* bias, void* y,
+                          int64_t ldc, int64_t m, int64_t n, int64_t k, void* ws, size_t ws_bytes) {
+  return dense_ln_parts_ws_impl(stream, dtype, epi, x, lda, w, cd, parts, groups, eps, bias, y, ldc, m, n, k, ws, ws_bytes,
+                                {});
+}
+
+static int dense_qkv_rotary_ln_parts_impl(void* stream, int32_t dtype, const void* x, int64_t lda, const void* w,
+                                          const float* cd, const float* parts, int32_t groups, float eps,
+                                          const float* bias, const void* cs, const int32_t* pos_hw,
+                                          const uint32_t* table, int32_t n_positions, void* q, void* k, void* vt,
+                                          int64_t n_tokens, int64_t hidden, int32_t H, void* ws, size_t ws_bytes,
+                                          NextWeights next) {
+  QVL_TRY_RC(check_ln_parts("qkv_rotary_ln_parts", n_tokens, hidden, cd, parts, groups, eps));
+  if (n_tokens > 0 && (cs ? (pos_hw || table) : (!pos_hw || !table)))
+    return set_error(QVL_ERR_INVALID_ARG, "qkv_rotary_ln_parts: give either the per-token cos/sin table or positions + table");
+  return qkv_rotary_impl(stream, dtype, x, lda, w, bias, cs, cs ? nullptr : pos_hw, cs ? nullptr : table,
+                         cs ? 0 : n_positions, q, k, vt, n_tokens, hidden, H, ws, ws_bytes, cd, nullptr, parts, groups,
+                         eps, next);
 }
 
 int qvl_dense_qkv_rotary_ln_parts(void* stream, int32_t dtype, const void* x, int64_t lda, const void* w,
@@ -408,12 +453,8 @@ int qvl_dense_qkv_rotary_ln_parts(void* stream, int32_t dtype, const void* x, in
                                   const void* cs, const int32_t* pos_hw, const uint32_t* table, int32_t n_positions,
                                   void* q, void* k, void* vt, int64_t n_tokens, int64_t hidden, int32_t H, void* ws,
                                   size_t ws_bytes) {
-  QVL_TRY_RC(check_ln_parts("qkv_rotary_ln_parts", n_tokens, hidden, cd, parts, groups, eps));
-  if (n_tokens > 0 && (cs ? (pos_hw || table) : (!pos_hw || !table)))
-    return set_error(QVL_ERR_INVALID_ARG, "qkv_rotary_ln_parts: give either the per-token cos/sin table or positions + table");
-  return qkv_rotary_impl(stream, dtype, x, lda, w, bias, cs, cs ? nullptr : pos_hw, cs ? nullptr : table,
-                         cs ? 0 : n_positions, q, k, vt, n_tokens, hidden, H, ws, ws_bytes, cd, nullptr, parts, groups,
-                         eps);
+  return dense_qkv_rotary_ln_parts_impl(stream, dtype, x, lda, w, cd, parts, groups, eps, bias, cs, pos_hw, table,
+                                        n_positions, q, k, vt, n_tokens, hidden, H, ws, ws_bytes, {});
 }
 
 int qvl_attention_headmajor(void* stream, int32_t dtype, const void* q, const void* k, const void* vt,
@@ -608,13 +649,15 @@ static int run_merger_split(hipStream_t st, const qvl_vision_config* c, const To
 // 128-column groups per token row, 0: none), or a qvl_row_stats launch.
 static int run_merger(hipStream_t st, const qvl_vision_config* c, const TowerLayout& L, const qvl_merger_weights& mw,
                       bool postshuffle, const void* x, void* xn, void* h, void* out, void* part, float* stats,
-                      int parts_groups) {
+                      int parts_groups, NextWeights next) {
   const int64_t N = L.N, D = L.D, D4 = 4 * L.D;
   const int dt = L.dtype;
+  const NextWeights fc2 = {mw.fc2_w, c->out_hidden_size * D4 * 2};
   if (postshuffle && dt == QVL_DTYPE_BF16 && mw.fc1_ln.w && mw.fc1_ln.cd && stats) {
     if (parts_groups > 0 && 4 * parts_groups <= 64) {   // (hidden <= 2048: the merger LayerNorm's width bound)
-      QVL_TRY_RC(qvl_dense_ln_parts_ws(st, dt, QVL_EPI_BIAS_GELU, x, D4, mw.fc1_ln.w, mw.fc1_ln.cd, stats,
-                                       4 * parts_groups, c->ln_eps, mw.fc1_b, h, D4, N / 4, D4, D4, part, L.part_bytes));
+      QVL_TRY_RC(dense_ln_parts_ws_impl(st, dt, QVL_EPI_BIAS_GELU, x, D4, mw.fc1_ln.w, mw.fc1_ln.cd, stats,
+                                        4 * parts_groups, c->ln_eps, mw.fc1_b, h, D4, N / 4, D4, D4, part, L.part_bytes,
+                                        fc2));
     } else {
       QVL_TRY_RC(qvl_row_stats(st, dt, x, D4, N / 4, D4, c->ln_eps, stats));
       QVL_TRY_RC(qvl_dense_ln_ws(st, dt, QVL_EPI_BIAS_GELU, x, D4, mw.fc1_ln.w, mw.fc1_ln.cd, stats, mw.fc1_b, h, D4,
@@ -625,11 +668,11 @@ static int run_merger(hipStream_t st, const qvl_vision_config* c, const TowerLay
       QVL_TRY_RC(qvl_layer_norm(st, dt, x, D4, mw.norm_w, mw.norm_b, xn, D4, N / 4, D4, c->ln_eps));
     else
       QVL_TRY_RC(qvl_layer_norm(st, dt, x, D, mw.norm_w, mw.norm_b, xn, D, N, D, c->ln_eps));
-    QVL_TRY_RC(qvl_dense_ws(st, dt, QVL_EPI_BIAS_GELU, xn, D4, mw.fc1_w, mw.fc1_b, nullptr, 0, h, D4, N / 4, D4, D4,
-                            part, L.part_bytes));
+    QVL_TRY_RC(dense_impl(st, dt, QVL_EPI_BIAS_GELU, xn, D4, mw.fc1_w, mw.fc1_b, nullptr, 0, h, D4, N / 4, D4, D4, part,
+                          L.part_bytes, nullptr, nullptr, nullptr, 0, 0.f, nullptr, fc2));
   }
-  QVL_TRY_RC(qvl_dense_ws(st, dt, QVL_EPI_BIAS, h, D4, mw.fc2_w, mw.fc2_b, nullptr, 0, out, c->out_hidden_size, N / 4,
-                          c->out_hidden_size, D4, part, L.part_bytes));
+  QVL_TRY_RC(dense_impl(st, dt, QVL_EPI_BIAS, h, D4, mw.fc2_w, mw.fc2_b, nullptr, 0, out, c->out_hidden_size, N / 4,
+                        c->out_hidden_size, D4, part, L.part_bytes, nullptr, nullptr, nullptr, 0, 0.f, nullptr, next));
   return QVL_OK;
 }
 
@@ -714,6 +757,21 @@ static int encode_impl(void* stream, const qvl_vision_config* c, const qvl_visio
   for (int j = 0; j < c->n_deepstack && !f32; ++j) any_fold = any_fold || W->deepstack[j].fc1_ln.w;
   const int G = any_fold ? L.stat_groups : 0;
   bool have_parts = false;
+  // What a GEMM's successor reads (NextWeights): block i's qkv or, past the last block, the main merger's fc1; the tap
+  // merger of block i where there is one.
+  const auto qkv_of = [&](int i) {
+    const bool folded = i < c->depth && W->blocks[i].qkv_ln.w && W->blocks[i].qkv_ln.cd;
+    return i < c->depth ? NextWeights{folded ? W->blocks[i].qkv_ln.w : W->blocks[i].qkv_w, 3 * D * D * 2}
+                        : NextWeights{W->merger.fc1_w, 16 * D * D * 2};
+  };
+  const auto after_block = [&](int i, int tap) {
+    for (int j = 0; j < c->n_deepstack; ++j)
+      if (c->deepstack_indexes[j] == i && tap < c->n_deepstack) {
+        const qvl_merger_weights& m = W->deepstack[tap];
+        return NextWeights{m.fc1_ln.w && m.fc1_ln.cd ? m.fc1_ln.w : m.fc1_w, 16 * D * D * 2};
+      }
+    return qkv_of(i + 1);
+  };
   // (with split weights the pixel rows are split into the then idle q / k / v buffers)
   const bool split_px = split && (size_t)N * L.PVp * 4 <= L.off_h - L.off_q;
   if (split_px) {
@@ -726,8 +784,8 @@ static int encode_impl(void* stream, const qvl_vision_config* c, const qvl_visio
   } else if (c->num_position_embeddings > 0 && !f32 && D % 8 == 0) {
     // bf16: the pos-embed gathered per row inside the patch embed's residual epilogue (no [N, D]
     // pos-embed buffer written and read back), with x's row partials when a fold reads them
-    QVL_TRY_RC(qvl_dense_pos_embed_ws(st, dt, px_in, L.PVp, W->patch_w, W->patch_b, W->pos_table, meta->tap_idx,
-                                      meta->tap_w, x, D, N, D, L.PVp, G ? stats : nullptr, part, PB));
+    QVL_TRY_RC(dense_pos_embed_ws_impl(st, dt, px_in, L.PVp, W->patch_w, W->patch_b, W->pos_table, meta->tap_idx,
+                                       meta->tap_w, x, D, N, D, L.PVp, G ? stats : nullptr, qkv_of(0)));
     have_parts = G != 0;
   } else if (c->num_position_embeddings > 0) {
     QVL_TRY_RC(qvl_pos_embed(st, dt, W->pos_table, meta->tap_idx, meta->tap_w, xn, N, D));
@@ -765,8 +823,9 @@ static int encode_impl(void* stream, const qvl_vision_config* c, const qvl_visio
       const uint32_t* ttab = pos_tab ? (const uint32_t*)cs : nullptr;
       const int tnp = pos_tab ? (int)meta->n_positions : 0;
       if (have_parts)
-        QVL_TRY_RC(qvl_dense_qkv_rotary_ln_parts(st, dt, x, D, B.qkv_ln.w, B.qkv_ln.cd, stats, G, c->ln_eps, B.qkv_b,
-                                                 tcs, tpos, ttab, tnp, Qb, Kb, Vb, N, D, (int)L.H, part, PB));
+        QVL_TRY_RC(dense_qkv_rotary_ln_parts_impl(st, dt, x, D, B.qkv_ln.w, B.qkv_ln.cd, stats, G, c->ln_eps, B.qkv_b,
+                                                  tcs, tpos, ttab, tnp, Qb, Kb, Vb, N, D, (int)L.H, part, PB,
+                                                  {B.proj_w, D * D * 2}));
       else
         QVL_TRY_RC(qvl_dense_qkv_rotary_ln(st, dt, x, D, B.qkv_ln.w, B.qkv_ln.cd, stats, B.qkv_b, tcs, tpos, ttab, tnp,
                                            Qb, Kb, Vb, N, D, (int)L.H, part, PB));
@@ -836,13 +895,14 @@ static int encode_impl(void* stream, const qvl_vision_config* c, const qvl_visio
                              QVL_EPI_BIAS_RESIDUAL, (const float*)x, x, nullptr, part, PB));
     } else {
       if (have_parts)
-        QVL_TRY_RC(qvl_dense_rowstats_ws(st, dt, xn, D, B.proj_w, B.proj_b, x, D, x, D, N, D, D, stats, part, PB));
+        QVL_TRY_RC(dense_rowstats_ws_impl(st, dt, xn, D, B.proj_w, B.proj_b, x, D, x, D, N, D, D, stats, part, PB,
+                                          {B.fc1_ln.w, I * D * 2}));
       else
         QVL_TRY_RC(qvl_dense_ws(st, dt, QVL_EPI_BIAS_RESIDUAL, xn, D, B.proj_w, B.proj_b, x, D, x, D, N, D, D, part, PB));
       // x += fc2(gelu(fc1(LN2 x)))   (model.py:629, 610-614)
       if (fold && have_parts) {
-        QVL_TRY_RC(qvl_dense_ln_parts_ws(st, dt, QVL_EPI_BIAS_GELU, x, D, B.fc1_ln.w, B.fc1_ln.cd, stats, G, c->ln_eps,
-                                         B.fc1_b, h, I, N, I, D, part, PB));
+        QVL_TRY_RC(dense_ln_parts_ws_impl(st, dt, QVL_EPI_BIAS_GELU, x, D, B.fc1_ln.w, B.fc1_ln.cd, stats, G, c->ln_eps,
+                                          B.fc1_b, h, I, N, I, D, part, PB, {B.fc2_w, I * D * 2}));
       } else if (fold) {
         QVL_TRY_RC(qvl_row_stats(st, dt, x, D, N, D, c->ln_eps, stats));
         QVL_TRY_RC(qvl_dense_ln_ws(st, dt, QVL_EPI_BIAS_GELU, x, D, B.fc1_ln.w, B.fc1_ln.cd, stats, B.fc1_b, h, I, N, I,
@@ -854,7 +914,8 @@ static int encode_impl(void* stream, const qvl_vision_config* c, const qvl_visio
       // partials of the new x for the next block's folded norm1 or a folded deepstack merger
       have_parts = G != 0;
       if (have_parts)
-        QVL_TRY_RC(qvl_dense_rowstats_ws(st, dt, h, I, B.fc2_w, B.fc2_b, x, D, x, D, N, D, I, stats, part, PB));
+        QVL_TRY_RC(dense_rowstats_ws_impl(st, dt, h, I, B.fc2_w, B.fc2_b, x, D, x, D, N, D, I, stats, part, PB,
+                                          after_block(i, ds_next)));
       else
         QVL_TRY_RC(qvl_dense_ws(st, dt, QVL_EPI_BIAS_RESIDUAL, h, I, B.fc2_w, B.fc2_b, x, D, x, D, N, D, I, part, PB));
     }
@@ -866,8 +927,8 @@ static int encode_impl(void* stream, const qvl_vision_config* c, const qvl_visio
           QVL_TRY_RC(run_merger_split(st, c, L, W->deepstack[ds_next], split->deepstack[ds_next], true, x, xn, h, out, sx,
                                       part));
         else
-          QVL_TRY_RC(run_merger(st, c, L, W->deepstack[ds_next], true, x, xn, h, out, part, stats,
-                                have_parts ? G : 0));
+          QVL_TRY_RC(run_merger(st, c, L, W->deepstack[ds_next], true, x, xn, h, out, part, stats, have_parts ? G : 0,
+                                qkv_of(i + 1)));
         if (win)   // unshuffle (model.py:845-848)
           QVL_TRY_RC(qvl_gather_rows(st, dt, Qb, Dout, dt, deepstack[ds_next], Dout, meta->window_reverse, N / 4, 1, Dout));
         ++ds_next;
@@ -877,7 +938,7 @@ static int encode_impl(void* stream, const qvl_vision_config* c, const qvl_visio
   if (split)
     QVL_TRY_RC(run_merger_split(st, c, L, W->merger, split->merger, false, x, xn, h, win ? (void*)Qb : tokens, sx, part));
   else
-    QVL_TRY_RC(run_merger(st, c, L, W->merger, false, x, xn, h, win ? (void*)Qb : tokens, part, stats, 0));
+    QVL_TRY_RC(run_merger(st, c, L, W->merger, false, x, xn, h, win ? (void*)Qb : tokens, part, stats, 0, {}));
   if (win) QVL_TRY_RC(qvl_gather_rows(st, dt, Qb, Dout, dt, tokens, Dout, meta->window_reverse, N / 4, 1, Dout));
   return QVL_OK;
 }

@@ -61,6 +61,10 @@ struct GemmParams {
   const bf16* pe_table;
   const int* pe_idx;
   const float* pe_w;
+  // Weights that the caller's next GEMM reads (NULL: not known): a launch that leaves CUs idle has them read once by
+  // workgroups past its tiles. It changes no result.
+  const void* next_w;
+  int64_t next_bytes;
 };
 
 // fp32 GEMM (qvl_f32.hip): w packed [n_rows_w][ldw] fp32 (ldw = k padded to 64), Kp = ldw.

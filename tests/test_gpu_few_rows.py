@@ -167,3 +167,29 @@ def test_few_rows_pos_embed(pkg, lib, plans, grids):
     prod = x.double() @ w.double().t()
     assert close(y9, y3, prod, prod + b.double())
     assert torch.allclose(p9[..., 0].double(), y9.double().view(M, -1, 128).sum(2), rtol=0, atol=1e-5 * 128)
+
+
+# around the row count up to which a launch's idle workgroups read the next GEMM's weights, and the smallest grids
+@pytest.mark.parametrize("shape", ["2b", "8b"])
+@pytest.mark.parametrize("grids", [[(1, 2, 2)], [(1, 14, 14)], [(1, 28, 32)], [(1, 26, 34), (1, 2, 8)]])
+def test_tower_reading_next_weights(pkg, lib, grids, shape):
+    """64x128 tiles (whose launches read ahead) against 256x128 tiles (which do not), with a tap and both mergers: the
+    same k order, so the same bits (the head_dim-72 qkv GEMM keeps its own tiles on both)."""
+    from tests.test_gpu_parity_depth import ckpt_params, pixels, specs
+    spec, ospec = specs(pkg, shape, depth=2, ds=(0,))
+    tower = pkg.Qwen3VisionTransformer(spec, dtype="bfloat16").bind(ckpt_params(ospec, seed=5))
+    px, g = pixels(grids, 5), np.array(grids, np.int32)
+    out = []
+    for plan in (8, 3):
+        pkg.capi.check(lib.qvl_set_gemm_plan(plan, -1, 0))
+        try:
+            tok, ds = tower(px, g)
+            out.append([t.clone() for t in (tok, *ds)])
+        finally:
+            pkg.capi.check(lib.qvl_set_gemm_plan(0, 0, 0))
+    for a, b in zip(*out):
+        assert torch.isfinite(a.float()).all() and torch.equal(a, b)
+    tok, ds = tower(px, g)                            # the default plans: other K orders, so bf16 steps apart
+    for a, b in zip((tok, *ds), out[0]):
+        a, b = a.double(), b.double()
+        assert (a - b).norm() <= 1e-2 * b.norm()
