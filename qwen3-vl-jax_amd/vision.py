@@ -412,6 +412,7 @@ class Qwen3VisionTransformer:
         self.ln_fold = bool(ln_fold) and self.qdtype == capi.QVL_DTYPE_BF16
         self._folds: Dict[str, tuple] = {}
         self._split = None            # fp32: the Dense weights as f16-split rows (_split_weights)
+        self._split_of = None         # the write counts of the buffers those were made from
         self._lib = capi.load()
         self._w = None
         self._keep = []
@@ -532,6 +533,28 @@ class Qwen3VisionTransformer:
         if not bool(torch.isfinite(bounds).all()):
             return None
         return sp, (rows, scales, bounds, blocks, ds)
+
+    def _writes(self):
+        """torch's count of in-place writes to each bound buffer (inference tensors have none)."""
+        return [0 if t.is_inference() else t._version for t in self._state.values()]
+
+    def _current_split(self):
+        """The split weights, made anew where a bound buffer was written in place (packed_state, or the tensors
+        given to bind_packed, an optimizer's step on them): the forward follows such writes as it does without them.
+        During a stream capture, where they cannot be made (the check of their bounds waits for the GPU), a forward
+        after such a write reads the buffers themselves. The check costs 60 ns a buffer."""
+        if self._split is None:
+            return None
+        writes = self._writes()
+        if writes != self._split_of:
+            torch = _torch()
+            if torch.cuda.is_current_stream_capturing():
+                return None
+            split = self._split_weights(self._state)
+            if split is None:
+                return None           # no longer finite: looked at again on the next call
+            self._split, self._split_of = split, writes
+        return self._split
 
     def _vec(self, v):
         torch = _torch()
@@ -667,8 +690,10 @@ class Qwen3VisionTransformer:
         self._folds = folds
         self._keep = list(st.values()) + [t for f in folds.values() for t in f]
         self._blocks_arr, self._ds_arr = blocks, ds
-        self._split = self._split_weights(st) if self.qdtype == capi.QVL_DTYPE_F32 else None
         self._w = W
+        if self.qdtype == capi.QVL_DTYPE_F32:
+            self._split_of = self._writes()
+            self._split = self._split_weights(st)
         return self
 
     # -- per-grid metadata ----------------------------------------------------------------------
@@ -758,9 +783,10 @@ class Qwen3VisionTransformer:
               for _ in s.deepstack_visual_indexes]
         ds_ptrs = (C.c_void_p * max(len(ds), 1))(*[t.data_ptr() for t in ds])
         ws, nbytes = self.workspace(N)
-        if self._split is not None:
+        split = self._current_split()
+        if split is not None:
             capi.check(self._lib.qvl_encode_vision_split(self._stream(), C.byref(self._cfg), C.byref(self._w),
-                                                         C.byref(self._split[0]), C.byref(md), px.data_ptr(),
+                                                         C.byref(split[0]), C.byref(md), px.data_ptr(),
                                                          tokens.data_ptr(), ds_ptrs, ws.data_ptr(), nbytes),
                        "qvl_encode_vision_split")
         else:

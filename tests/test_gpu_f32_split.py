@@ -191,3 +191,27 @@ def test_weights_that_cannot_be_split_leave_the_tower_unsplit(pkg):
     assert t._split is None
     tokens, _ = t(px, grids)
     assert not torch.isfinite(tokens[:, 5]).any() and torch.isfinite(tokens[:, :5]).all()
+
+
+def test_split_weights_follow_writes_to_the_bound_buffers(pkg):
+    """A weight, a norm's parameter and a bias written in place between two forwards: the second one's outputs are those
+    of a tower bound to the written buffers."""
+    spec = pkg.spec_2b()
+    spec.depth, spec.deepstack_visual_indexes = 1, ()
+    grids = np.array([[1, 4, 6]], np.int32)
+    px = np.random.default_rng(3).standard_normal((24, spec.patch_volume), dtype=np.float32)
+    t = pkg.Qwen3VisionTransformer(spec).bind(pkg.random_params(spec, seed=2))
+    before = t(px, grids)[0].clone()
+    for name, by in (("blocks.0.fc1.w", 0.01), ("blocks.0.norm1.w", 50.0), ("merger.fc1.b", -2.0)):
+        t.packed_state()[name].add_(by)
+        got = t(px, grids)[0].clone()
+        want = pkg.Qwen3VisionTransformer(spec).bind_packed(t.packed_state())(px, grids)[0]
+        assert torch.equal(got, want) and not torch.equal(got, before)
+        before = got
+    w = t.packed_state()["merger.fc2.w"]
+    old = w[5, 3].item()
+    w[5, 3] = float("inf")                              # cannot be split: the buffers are read as they are
+    tokens = t(px, grids)[0]
+    assert not torch.isfinite(tokens[:, 5]).any() and torch.isfinite(tokens[:, :5]).all()
+    w[5, 3] = old
+    assert torch.equal(t(px, grids)[0], before)
