@@ -532,6 +532,17 @@ int qvl_scatter_vision_rows(void* stream, int32_t mode, int32_t hidden_dtype, vo
                             int64_t rows_batch_stride, int64_t n_rows, const int32_t* d_pos,
                             const int32_t* d_count);
 
+/* qvl_vision_positions and qvl_scatter_vision_rows in one launch, with the same results: rows[b][i] goes to the i-th
+ * flagged token of batch row b. `d_flags` [batch][seq_len]: flag_bytes 4, int32 tokens, flagged where == match;
+ * flag_bytes 1, a mask, flagged where not 0 (match unused). dim a multiple of 8; hidden, rows and every batch row of
+ * rows 16-byte aligned (else QVL_ERR_MISALIGNED); seq_len at most QVL_FLAGGED_MAX_SEQ (else QVL_ERR_UNSUPPORTED): the
+ * two entries above take the rest. */
+#define QVL_FLAGGED_MAX_SEQ 32768
+int qvl_scatter_flagged_rows(void* stream, int32_t mode, int32_t hidden_dtype, void* d_hidden, int64_t batch,
+                             int64_t seq_len, int64_t dim, int32_t rows_dtype, const void* d_rows,
+                             int64_t rows_batch_stride, int64_t n_rows, int32_t flag_bytes, const void* d_flags,
+                             int32_t match);
+
 #ifdef __cplusplus
 }
 #endif

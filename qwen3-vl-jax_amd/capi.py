@@ -15,6 +15,7 @@ QVL_DTYPE_BF16 = 1
 QVL_EPI_BIAS = 0
 QVL_EPI_BIAS_GELU = 1
 QVL_EPI_BIAS_RESIDUAL = 2
+QVL_FLAGGED_MAX_SEQ = 32768
 QVL_SCATTER_SET = 0
 QVL_SCATTER_ADD = 1
 
@@ -140,6 +141,7 @@ SIGNATURES = {
     "qvl_patchify": (C.c_int, [_p, _i32, _p, _i64, _i64, _i64, _i32, _i32, _i32, _i32, _p, _i64]),
     "qvl_vision_positions": (C.c_int, [_p, _p, _i64, _i64, _i32, _i64, _p, _p]),
     "qvl_scatter_vision_rows": (C.c_int, [_p, _i32, _i32, _p, _i64, _i64, _i64, _i32, _p, _i64, _i64, _p, _p]),
+    "qvl_scatter_flagged_rows": (C.c_int, [_p, _i32, _i32, _p, _i64, _i64, _i64, _i32, _p, _i64, _i64, _i32, _p, _i32]),
 }
 
 

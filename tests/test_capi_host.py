@@ -313,3 +313,22 @@ def test_metadata_packed_into_one_transfer(pkg):
         assert (t.data_ptr() - base) % 256 == 0, name
     with pytest.raises(TypeError):
         pkg.vision._to_device_packed({"x": np.zeros(3, np.int64)}, "cpu")
+
+
+def test_flagged_rows_argument_checks(pkg):
+    cp, lib = pkg.capi, pkg.capi.load()
+    BF, F32, SET, fake = cp.QVL_DTYPE_BF16, cp.QVL_DTYPE_F32, cp.QVL_SCATTER_SET, 4096
+    call = lib.qvl_scatter_flagged_rows
+    assert call(None, 2, BF, fake, 1, 8, 8, BF, fake, 0, 2, 1, fake, 1) == -1
+    assert call(None, SET, 3, fake, 1, 8, 8, BF, fake, 0, 2, 1, fake, 1) == -2
+    assert call(None, SET, BF, fake, 1, 8, 8, F32, fake, 0, 2, 2, fake, 1) == -1
+    assert call(None, SET, BF, fake, 1, -8, 8, F32, fake, 0, 2, 4, fake, 1) == -1
+    assert call(None, SET, BF, fake, 1, 8, 8, F32, None, 0, 2, 4, fake, 1) == -1
+    assert call(None, SET, BF, fake, 65536, 8, 8, F32, fake, 0, 2, 4, fake, 1) == -2
+    assert call(None, SET, BF, fake, 1, cp.QVL_FLAGGED_MAX_SEQ + 1, 8, F32, fake, 0, 2, 4, fake, 1) == -2
+    for hidden, rows, dim, stride, flags in ((fake + 8, fake, 8, 0, fake), (fake, fake + 8, 8, 0, fake),
+                                             (fake, fake, 12, 0, fake), (fake, fake, 8, 4, fake),
+                                             (fake, fake, 8, 0, fake + 2)):
+        assert call(None, SET, BF, hidden, 1, 8, dim, BF, rows, stride, 2, 4, flags, 1) == -3
+    for b, s, d, n in ((0, 8, 8, 2), (1, 0, 8, 2), (1, 8, 0, 2), (1, 8, 8, 0)):      # nothing to do
+        assert call(None, SET, BF, fake, b, s, d, BF, fake, 0, n, 1, fake, 1) == 0

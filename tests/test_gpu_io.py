@@ -229,3 +229,50 @@ def test_scatter_drops_out_of_range_positions(pkg, D):
                 if 0 <= pos[b, j] < S:
                     ref[b, pos[b, j]] = rows[b, j] if mode == cp.QVL_SCATTER_SET else ref[b, pos[b, j]] + rows[b, j]
         assert np.array_equal(bits(h.cpu().numpy()), bits(ref)), mode
+
+
+@pytest.mark.parametrize("hdt,rdt", [("bfloat16", "bfloat16"), ("bfloat16", "float32"), ("float32", "float32"),
+                                     ("float32", "bfloat16")])
+@pytest.mark.parametrize("B,S,D,V,share", [
+    (1, 1, 8, 3, 1.0),         # one token, fewer tokens than rows
+    (3, 9, 16, 4, 0.5),        # a workgroup's 8 tokens and one more
+    (2, 129, 520, 200, 0.7),   # never enough flags; rows one step of a wave long and a piece
+    (1, 20001, 8, 5000, 0.4),  # 16 tokens a workgroup, more flags than rows
+    (5, 2048, 24, 300, 0.01),  # most workgroups without a flag
+    (2, 100, 32, 8, 0.0),      # no flags
+])
+def test_flagged_rows_equal_positions_and_scatter(pkg, hdt, rdt, B, S, D, V, share):
+    """One launch against vision_positions + scatter_rows, bit for bit: masks and tokens, flag rows aligned to 16 bytes
+    and not, one set of rows and one per batch row, -0 and NaN in the hidden states."""
+    io, cp = pkg.decoder_io, pkg.capi
+    g = torch.Generator(device="cuda").manual_seed(S + D)
+    hidden = torch.randn((B, S, D), generator=g, device="cuda").to(getattr(torch, hdt))
+    hidden[:, 0, ::2] = -0.0
+    hidden[:, S // 2, 1] = float("nan")
+    for first in (True, False):
+        mask = torch.rand((B, S), generator=g, device="cuda") < share
+        mask[:, 0] = first and share > 0
+        tokens = torch.where(mask, 77, 5).to(torch.int32)
+        held = torch.empty(B * S + 1, dtype=torch.int32, device="cuda")[1:].view(B, S)
+        for flags, match in ((mask, 1), (tokens, 77), (held.copy_(tokens), 77), (tokens.long(), 77)):
+            for rb in (1, B):
+                rows = torch.randn((rb, V, D), generator=g, device="cuda").to(getattr(torch, rdt))
+                for mode in (cp.QVL_SCATTER_SET, cp.QVL_SCATTER_ADD):
+                    want, got = hidden.clone(), hidden.clone()
+                    io.scatter_rows(want, rows, *io.vision_positions(flags, V, match), mode)
+                    io._scatter_flagged(got, rows, flags, match, mode)
+                    view = torch.int16 if hdt == "bfloat16" else torch.int32
+                    assert torch.equal(got.view(view), want.view(view))
+
+
+def test_flagged_rows_forms_left_to_two_launches(pkg):
+    """Rows of 36 elements, hidden states off a 16-byte boundary, and the first length past the limit."""
+    io, cp = pkg.decoder_io, pkg.capi
+    for S, D, off in ((50, 36, 0), (50, 32, 1), (cp.QVL_FLAGGED_MAX_SEQ + 1, 8, 0)):
+        B, V = 2, 7
+        hidden = torch.randn(B * S * D + off, device="cuda")[off:].view(B, S, D)
+        want = hidden.clone()
+        mask = torch.rand((B, S), device="cuda") < 0.3
+        rows = torch.randn((V, D), device="cuda")
+        io.scatter_rows(want, rows, *io.vision_positions(mask, V), cp.QVL_SCATTER_ADD)
+        assert torch.equal(io.apply_deepstack(hidden, mask, rows), want)
