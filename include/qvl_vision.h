@@ -166,7 +166,7 @@ int qvl_set_attention_plan(int32_t key_groups);
 
 /* Tile override for the fp32 Dense with a workspace, FROM THE CALLING THREAD ONLY (thread-local), for tests
  * and tuning: 0 = the default rules, 1..4 = f16-split operands on 64x128 (two-stage ring), 64x128 (three
- * stages), 128x256 or 256x256 tiles, 5 = the fp32 MFMA kernel. No counterpart in the reference. */
+ * stages), 128x256 or 256x256 tiles, 5 = the fp32 MFMA kernel, 6 = f16-split operands on 128x128 tiles. No counterpart in the reference. */
 int qvl_set_f32_plan(int32_t tile);
 
 /* LayerNorm over the last axis: fp32 mean / biased variance / rsqrt(var + eps), affine, cast

@@ -546,11 +546,11 @@ static int launch_gemm_split(GemmSplitParams p, int split, hipStream_t stream) {
 }
 
 // Tile plan of the calling thread (qvl_set_f32_plan): 0 = the rules below, 1..4 = kSplitTiles[tile - 1],
-// 5 = the fp32 MFMA kernel.
+// 5 = the fp32 MFMA kernel, 6 = kSplitTiles[4].
 static thread_local int t_f32_plan = 0;
 
 int gemm_f32_set_plan(int tile) {
-  if (tile < 0 || tile > 5) return set_error(QVL_ERR_INVALID_ARG, "f32 plan: tile=%d (0..5)", tile);
+  if (tile < 0 || tile > 6) return set_error(QVL_ERR_INVALID_ARG, "f32 plan: tile=%d (0..6)", tile);
   t_f32_plan = tile;
   return QVL_OK;
 }
@@ -558,16 +558,23 @@ int gemm_f32_set_plan(int tile) {
 // Tile and K split by a cost model of the launch, in microseconds: start + rounds * (K / split * per_k +
 // per_tile), rounds = workgroups per CU, where a last partial round costs its share of the CUs but at least
 // `part` of a round, and a launch of less than one round at least `one`; split-K adds its partials' traffic at
-// part_rate bytes/us. Fitted to 45 shapes from 49 to 18432 rows (MI355X, cold weights, every tile): what it
-// picks is 2 % slower than the best measured choice on average, 17 % at worst. For instance
-// 784 x 3072 x 1024 runs in 34 us, 8192 x 4096 x 1024 in 189 us (1.09 PFLOP/s of f16 products; 609 us on
-// v_mfma_f32_32x32x2_f32), 8192 x 1024 x 4096 in 181 us (365 us).
+// part_rate bytes/us. Fitted to 68 shapes from 49 to 8192 rows with 1 to 8 K parts (MI355X, every tile and part count
+// that fits): what it picks is 1.2 % slower than the best measured choice on average, 13 % at worst. For instance
+// 8192 x 4096 x 1024 runs in 189 us (1.09 PFLOP/s of f16 products; 609 us on v_mfma_f32_32x32x2_f32), 8192 x 1024 x
+// 4096 in 181 us (365 us).
+// The small tiles are bound by the operands' way into LDS, not by the matrix units (64x128: 24 KB per 0.4 us and CU),
+// so 128x128 tiles, 2/3 of that traffic, win where one round of them covers most CUs; and eight waves a workgroup, each
+// with half the DMA to issue, beat four on the same tile. With the split pass: 784 x 3072 x 1024 44.8 -> 37.4 us, 784 x
+// 4096 x 1024 46.6 -> 38.9, 1024 x 1024 x 4096 51.3 -> 45.5 (128x128 on four waves: 43.6, 44.1, 47.2); 64x128 on eight
+// waves against four: 2048 x 1024 x 1024 29.1 against 32.6, 400 x 4096 x 1024 29.5 against 32.5, 4096 x 1024 x 1024
+// 39.8 against 42.4.
 struct SplitTile { int bm, bn, slots; double start, per_k, per_tile, part, one, part_rate; };   // slots: workgroups a CU holds
 constexpr SplitTile kSplitTiles[] = {
-    {64, 128, 3, 11.7, 14.1 / 1024, 0.0, 0.25, 1.20, 17.9e6},     // two-stage ring, 48 KB
-    {64, 128, 2, 5.1, 13.3 / 1024, 2.0, 0.81, 1.13, 6.9e6},       // three stages, 72 KB
-    {128, 256, 1, 0.2, 43.1 / 1024, 10.3, 0.88, 0.73, 8.0e6},     // three stages, 144 KB
-    {256, 256, 1, 0.0, 81.8 / 1024, 11.3, 0.86, 0.74, 7.9e6},     // two stages, 128 KB
+    {64, 128, 3, 13.2, 12.7 / 1024, 0.0, 0.57, 1.49, 34.1e6},     // 4 waves, two-stage ring, 48 KB
+    {64, 128, 2, 9.7, 11.8 / 1024, 1.6, 0.65, 0.96, 13.3e6},      // 8 waves, three stages, 72 KB
+    {128, 256, 1, 4.8, 38.9 / 1024, 11.3, 0.80, 0.06, 21.6e6},    // 8 waves, three stages, 144 KB
+    {256, 256, 1, 5.3, 80.1 / 1024, 11.8, 0.78, 0.22, 14.5e6},    // 8 waves, two stages, 128 KB
+    {128, 128, 1, 3.2, 19.9 / 1024, 9.5, 0.83, 0.89, 10.5e6},     // 8 waves, three stages, 96 KB
 };
 
 static double split_cost(const SplitTile& t, const GemmSplitParams& p, int cus, int split) {
@@ -584,11 +591,12 @@ static int dispatch_gemm_split(const GemmSplitParams& p, hipStream_t stream) {
   const int cus = gemm_device_cus();
   int pick = 0, split = 1;
   double best = 1e30;
-  for (int i = 0; i < 4; ++i) {
-    if (t_f32_plan >= 1 && t_f32_plan <= 4 && i != t_f32_plan - 1) continue;
+  const int only = t_f32_plan == 6 ? 4 : t_f32_plan >= 1 && t_f32_plan <= 4 ? t_f32_plan - 1 : -1;
+  for (int i = 0; i < 5; ++i) {
+    if (only >= 0 && i != only) continue;
     // (256x256 tiles add every product to one accumulator, 3 K / 16 roundings: nearer to float64 than the fp32
     // MFMA kernel where that does not split K, which is where its 128x128 tiles outnumber the CUs)
-    if (i == 3 && !t_f32_plan && ((p.M + 127) / 128) * ((p.N + 127) / 128) <= cus) continue;
+    if (i == 3 && only < 0 && ((p.M + 127) / 128) * ((p.N + 127) / 128) <= cus) continue;
     const SplitTile& t = kSplitTiles[i];
     const int tiles = ((p.M + t.bm - 1) / t.bm) * ((p.N + t.bn - 1) / t.bn);
     const int64_t npad = round_up(p.N, t.bn);
@@ -600,8 +608,9 @@ static int dispatch_gemm_split(const GemmSplitParams& p, hipStream_t stream) {
   }
   switch (pick) {
     case 0: return launch_gemm_split<64, 128, 2, 2, 2, EPI, OUTS>(p, split, stream);
-    case 1: return launch_gemm_split<64, 128, 2, 2, 3, EPI, OUTS>(p, split, stream);
+    case 1: return launch_gemm_split<64, 128, 2, 4, 3, EPI, OUTS>(p, split, stream);
     case 2: return launch_gemm_split<128, 256, 2, 4, 3, EPI, OUTS>(p, split, stream);
+    case 4: return launch_gemm_split<128, 128, 2, 4, 3, EPI, OUTS>(p, split, stream);
     default: return launch_gemm_split<256, 256, 4, 2, 2, EPI, OUTS>(p, split, stream);
   }
 }

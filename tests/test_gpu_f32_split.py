@@ -63,6 +63,23 @@ def test_split_dense_vs_fp64(dense, plan, M, N, K):
     assert torch.all((y.double() - gelu).abs() <= 1.13 * tol + 4e-6 * gelu.abs().clamp(min=1.0))
 
 
+# edges of the 128x128 tile, with and without K parts; (784, 3072, 1024): the default rule takes it
+@pytest.mark.parametrize("M,N,K", [(1, 4, 64), (127, 124, 192), (128, 128, 256), (129, 132, 1024), (300, 1152, 4352),
+                                   (784, 3072, 1024)])
+def test_split_dense_128x128_tiles(dense, M, N, K):
+    x, w, b, r = operands(M, N, K, M + N + K)
+    ref = x.double() @ w[:N].double().t() + b.double()
+    tol = bound(x, w, N, K) + ref.abs() * 2.0 ** -23
+    y = dense(6, x, w, b)
+    assert torch.all((y.double() - ref).abs() <= tol)
+    assert torch.all((dense(6, x, w, b, 2, r).double() - ref - r.double()).abs() <= tol + (ref.abs() + r.abs()) * 2.0 ** -23)
+    if M > 1:
+        assert (y.double() - ref).norm() <= (dense(5, x, w, b).double() - ref).norm()
+    x[0, 1], w[2, 3] = float("inf"), float("nan")
+    y, want = dense(6, x, w, b), dense(5, x, w, b)
+    assert torch.equal(torch.isnan(y), torch.isnan(want)) and torch.equal(torch.isinf(y), torch.isinf(want))
+
+
 @pytest.mark.parametrize("M,N,K", [(784, 1024, 1024), (300, 512, 4096), (2304, 3072, 1024)])
 def test_split_dense_is_nearer_to_fp64_than_fp32_mfma(dense, M, N, K):
     x, w, b, _ = operands(M, N, K, K)
