@@ -32,6 +32,13 @@ def _qdtype(t):
     raise TypeError(f"unsupported dtype {t.dtype} (bfloat16 or float32)")
 
 
+def _beside(t, hidden, what: str):
+    """t on hidden's GPU: the kernels read its memory there. Host memory is refused; another GPU's tensor is copied."""
+    if t.device.type != hidden.device.type:
+        raise ValueError(f"{what} on {t.device}, hidden on {hidden.device}")
+    return t.to(hidden.device)
+
+
 def _flags(mask_or_tokens, match: int):
     """([B, S] contiguous bool or int32 tensor, the value that counts): a bool mask counts True."""
     torch = _torch()
@@ -68,7 +75,7 @@ def _checked_rows(hidden, rows):
         raise ValueError("hidden must be a contiguous [B, S, D] tensor")
     B, S, D = (int(s) for s in hidden.shape)
     r = rows if rows.dim() == 3 else rows.unsqueeze(0)
-    r = r.contiguous()
+    r = _beside(r, hidden, "rows").contiguous()
     if int(r.shape[-1]) != D:
         raise ValueError(f"row width {int(r.shape[-1])} != hidden width {D}")
     if int(r.shape[0]) not in (1, B):
@@ -96,7 +103,7 @@ def _scatter_flagged(hidden, rows, mask_or_tokens, match: int, mode: int):
     counted by every workgroup), rows of a multiple of 8 elements, 16-byte aligned. 4 x 2048 tokens, 1152 rows of
     2048 bf16: 13.5 us against 27.8; one row of 400 tokens 10.2 against 24.4."""
     torch = _torch()
-    t, match = _flags(mask_or_tokens, match)
+    t, match = _flags(_beside(mask_or_tokens, hidden, "flags"), match)
     r, bstride = _checked_rows(hidden, rows)
     B, S, D = (int(s) for s in hidden.shape)
     if tuple(t.shape) != (B, S) or S > capi.QVL_FLAGGED_MAX_SEQ or D % 8 or hidden.data_ptr() % 16 or r.data_ptr() % 16:

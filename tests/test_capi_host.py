@@ -332,3 +332,28 @@ def test_flagged_rows_argument_checks(pkg):
         assert call(None, SET, BF, hidden, 1, 8, dim, BF, rows, stride, 2, 4, flags, 1) == -3
     for b, s, d, n in ((0, 8, 8, 2), (1, 0, 8, 2), (1, 8, 0, 2), (1, 8, 8, 0)):      # nothing to do
         assert call(None, SET, BF, fake, b, s, d, BF, fake, 0, n, 1, fake, 1) == 0
+
+
+@pytest.mark.parametrize("which", ["mask", "tokens", "rows"])
+def test_injection_refuses_host_memory(pkg, monkeypatch, which):
+    """A mask, tokens or rows in host memory, with hidden states elsewhere, are refused before anything is launched: a
+    kernel would read a host pointer. (Hidden states of the `meta` device stand in for a GPU's.)"""
+    torch = pytest.importorskip("torch")
+    io, cp = pkg.decoder_io, pkg.capi
+
+    class Lib:
+        def __getattr__(self, name):
+            return lambda *a: pytest.fail(f"{name} was called")
+
+    class Stream:
+        cuda_stream = 0
+    monkeypatch.setattr(cp, "load", lambda: Lib())
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda *a: Stream())
+    hidden = torch.empty((2, 16, 8), device="meta")
+    flags = {"mask": torch.zeros((2, 16), dtype=torch.bool), "tokens": torch.zeros((2, 16), dtype=torch.int32)}.get(
+        which, torch.zeros((2, 16), dtype=torch.bool, device="meta"))
+    rows = torch.zeros((4, 8), device="cpu" if which == "rows" else "meta")
+    with pytest.raises(ValueError, match="cpu"):
+        io._scatter_flagged(hidden, rows, flags, 1, cp.QVL_SCATTER_ADD)
+    with pytest.raises(ValueError, match="cpu"):
+        io.apply_deepstack(hidden, flags, rows)
