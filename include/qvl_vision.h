@@ -491,6 +491,24 @@ int qvl_encode_vision_split(void* stream, const qvl_vision_config* cfg, const qv
                             const float* d_pixel_values, void* d_tokens, void* const* d_deepstack,
                             void* d_workspace, size_t workspace_bytes);
 
+/* qvl_encode_vision for an fp32 tower of those widths, each layer's Dense weights split into `d_scratch` on the stream
+ * before the layer: nothing derived from the weights is kept between calls, so a forward, or a captured graph's
+ * replay, reads the weights as they are when it runs. Beside qvl_encode_vision_workspace_size it takes
+ * qvl_vision_split_scratch_size bytes of scratch (16-byte aligned; the largest layer's: 48 MB for a 1024-wide block).
+ * A weight row that holds infinities or NaN gets fp32 sums. */
+int qvl_vision_split_scratch_size(const qvl_vision_config* cfg, size_t* bytes);
+int qvl_encode_vision_split_scratch(void* stream, const qvl_vision_config* cfg, const qvl_vision_weights* weights,
+                                    const qvl_vision_metadata_dev* meta, const float* d_pixel_values, void* d_tokens,
+                                    void* const* d_deepstack, void* d_workspace, size_t workspace_bytes,
+                                    void* d_scratch, size_t scratch_bytes);
+
+/* The largest output bound (qvl_split_dense_weight) of every Dense of the tower: d_bounds [4 * depth + 2 * (1 +
+ * n_deepstack) + 1] fp32, qkv, proj, fc1, fc2 of each block, fc1, fc2 of the merger and of each deepstack merger, the
+ * patch embed. A non-finite one: that layer's weights hold infinities or NaN, or their norms overflow, and the tower
+ * is better run by qvl_encode_vision. */
+int qvl_vision_split_bounds(void* stream, const qvl_vision_config* cfg, const qvl_vision_weights* weights,
+                            void* d_scratch, size_t scratch_bytes, float* d_bounds);
+
 /* ------------------------------------------------------------------------------------------ */
 /* The steps either side of the tower: patchify before it, decoder-side injection after it.    */
 /* ------------------------------------------------------------------------------------------ */

@@ -135,6 +135,10 @@ SIGNATURES = {
                                     C.POINTER(VisionMetadataDev), _p, _p, C.POINTER(_p), _p, _sz]),
     "qvl_encode_vision_split": (C.c_int, [_p, C.POINTER(VisionConfig), C.POINTER(VisionWeights), C.POINTER(VisionSplit),
                                           C.POINTER(VisionMetadataDev), _p, _p, C.POINTER(_p), _p, _sz]),
+    "qvl_vision_split_scratch_size": (C.c_int, [C.POINTER(VisionConfig), C.POINTER(_sz)]),
+    "qvl_encode_vision_split_scratch": (C.c_int, [_p, C.POINTER(VisionConfig), C.POINTER(VisionWeights),
+                                                  C.POINTER(VisionMetadataDev), _p, _p, C.POINTER(_p), _p, _sz, _p, _sz]),
+    "qvl_vision_split_bounds": (C.c_int, [_p, C.POINTER(VisionConfig), C.POINTER(VisionWeights), _p, _sz, _p]),
     "qvl_split_dense_weight": (C.c_int, [_p, _p, _i64, _i64, _p, _p, _p, _i64, _i32, _p, _p, _p]),
     "qvl_window_metadata": (C.c_int, [_pi32, _i64, _i32, _i32, _i32, _pi32, _pi32, _i64, C.POINTER(_i64), _pi32]),
     "qvl_gather_rows": (C.c_int, [_p, _i32, _p, _i64, _i32, _p, _i64, _p, _i64, _i32, _i64]),

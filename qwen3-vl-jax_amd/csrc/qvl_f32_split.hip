@@ -112,87 +112,94 @@ static int split_rows(const SplitRowsParams& p, hipStream_t stream) {
 }
 
 // ---------------------------------------------------------------------------------------------
-// Packed fp32 weights [n][k] -> split rows, once when a tower is bound, with a bound on |LN(x) . w + b|, the
-// Dense's output for any x: the normalised row has a norm of at most sqrt(k), so |.| <= sqrt(k) |gamma w| +
-// |beta . w| + |b| (one per row, to row_bound). It lets the outputs be split by one exponent that is known
-// before they are. Non-finite weights make it non-finite.
+// Packed fp32 weights [n][k] -> split rows, with a bound on |LN(x) . w + b|, the Dense's output for any x: the
+// normalised row has a norm of at most sqrt(k), so |.| <= sqrt(k) |gamma w| + |beta . w| + |b| (one per row, to
+// row_bound). It lets the outputs be split by one exponent that is known before they are. Non-finite weights make
+// it non-finite, and their row's factor NaN.
+// A tower splits each layer's weights on the stream right before they are used, so that a forward (or a graph's
+// replay) reads the weights as they are then; all Dense weights of a layer share one launch, a wave holds a row.
+// Memory bound: a 1024-wide block's 48 MB are read and written. A 784-patch forward of 24 blocks takes 4.53 ms with
+// it, 3.85 with weights split beforehand, and 8.8 on the fp32 MFMA kernels.
 // ---------------------------------------------------------------------------------------------
-template <int T, int CH>
-__global__ __launch_bounds__(256) void split_weight_kernel(const float* __restrict__ w, int k, int n,
-                                                           const float* __restrict__ bias,
-                                                           const float* __restrict__ gamma,
-                                                           const float* __restrict__ beta, int ln_cols,
-                                                           f16* __restrict__ out, float* __restrict__ inv,
-                                                           float* __restrict__ row_bound) {
-  __shared__ float tmp[4];
-  const int t = threadIdx.x % T, row = blockIdx.x * (256 / T) + threadIdx.x / T;
-  if (row >= n) return;                             // (a whole wave, or with T = 256 never)
-  const float* src = w + (int64_t)row * k;
+template <int CH>
+__global__ __launch_bounds__(256) void split_weights_kernel(SplitWeights p) {
+  int which = 0;
+  while (which + 1 < p.count && (int)blockIdx.x >= p.e[which + 1].first) ++which;
+  const SplitWeight& e = p.e[which];
+  const int lane = threadIdx.x & 63, row = ((int)blockIdx.x - e.first) * 4 + (threadIdx.x >> 6), k = e.k;
+  if (row >= e.n) return;
+  const float* src = e.w + (int64_t)row * k;
   f32x4 v[CH];
   uint32_t mb = 0;
   float norm = 0.f, dot = 0.f;
 #pragma unroll
   for (int i = 0; i < CH; ++i) {
-    const int c = (t + i * T) * 4;
-    v[i] = c < k ? *reinterpret_cast<const f32x4*>(src + c) : f32x4{0.f, 0.f, 0.f, 0.f};
+    const int c = (lane + i * 64) * 4;
+    if (c < k) v[i] = *reinterpret_cast<const f32x4*>(src + c);
   }
 #pragma unroll
   for (int i = 0; i < CH; ++i) {
-    const int c = (t + i * T) * 4;
+    const int c = (lane + i * 64) * 4;
     if (c >= k) break;
     const f32x4 one = {1.f, 1.f, 1.f, 1.f}, zero = {0.f, 0.f, 0.f, 0.f};
-    const f32x4 g = gamma ? *reinterpret_cast<const f32x4*>(gamma + c % ln_cols) : one;
-    const f32x4 b = beta ? *reinterpret_cast<const f32x4*>(beta + c % ln_cols) : zero;
+    const f32x4 g = e.gamma ? *reinterpret_cast<const f32x4*>(e.gamma + c % e.ln_cols) : one;
+    const f32x4 b = e.beta ? *reinterpret_cast<const f32x4*>(e.beta + c % e.ln_cols) : zero;
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      mb = max(mb, __float_as_uint(v[i][e]) & 0x7fffffffu);
-      norm = fmaf(g[e] * v[i][e], g[e] * v[i][e], norm);
-      dot = fmaf(b[e], v[i][e], dot);
+    for (int j = 0; j < 4; ++j) {
+      mb = max(mb, __float_as_uint(v[i][j]) & 0x7fffffffu);
+      norm = fmaf(g[j] * v[i][j], g[j] * v[i][j], norm);
+      dot = fmaf(b[j], v[i][j], dot);
     }
   }
-  if constexpr (T == 256) mb = block_max_bits(mb, tmp);
-  else mb = wave_max_bits(mb);
-  norm = row_sum<T>(norm, tmp);
-  dot = row_sum<T>(dot, tmp);
+  mb = wave_max_bits(mb);
+  norm = row_sum<64>(norm, nullptr);
+  dot = row_sum<64>(dot, nullptr);
   const float s = split_scale(__uint_as_float(mb));
-  f16* dst = out + (int64_t)row * 2 * k;
+  f16* dst = e.out + (int64_t)row * 2 * k;
 #pragma unroll
   for (int i = 0; i < CH; ++i) {
-    const int c = (t + i * T) * 4;
+    const int c = (lane + i * 64) * 4;
     if (c >= k) break;
     f16x4 hi, lo;
     split4(v[i], s, hi, lo);
     store_split4(dst, c, hi, lo);
   }
-  if (t == 0) {
-    inv[row] = 1.0f / s;
-    const float b = 1.001f * sqrtf(norm * (float)k) + fabsf(dot) + fabsf(bias[row]);
-    row_bound[row] = b;
+  if (lane == 0) {
+    e.inv[row] = mb < 0x7f800000u ? 1.0f / s : __uint_as_float(0x7fc00000u);
+    e.row_bound[row] = 1.001f * sqrtf(norm * (float)k) + fabsf(dot) + fabsf(e.bias[row]);
   }
 }
 
-// out[g] = the largest of the values (>= 0 or NaN, which wins) of group g. (An atomic maximum per row on one
-// address took the launch above from 10 to 45 us.)
-__global__ __launch_bounds__(256) void group_max_kernel(const float* __restrict__ v, int n, float* __restrict__ out) {
-  __shared__ float tmp[4];
+// out = the largest of the n values of v (>= 0 or NaN, which wins). (An atomic maximum per row on one address took the
+// launch above from 10 to 45 us.)
+__device__ __forceinline__ void group_max(const float* __restrict__ v, int n, float* __restrict__ out, float* tmp) {
   uint32_t mb = 0;
-  for (int i = threadIdx.x; i < n; i += 256) mb = max(mb, __float_as_uint(v[(int64_t)blockIdx.x * n + i]) & 0x7fffffffu);
+  for (int i = threadIdx.x; i < n; i += 256) mb = max(mb, __float_as_uint(v[i]) & 0x7fffffffu);
   mb = block_max_bits(mb, tmp);
-  if (threadIdx.x == 0) out[blockIdx.x] = __uint_as_float(mb);
+  if (threadIdx.x == 0) *out = __uint_as_float(mb);
 }
 
-int split_weight_f32(const float* w, int64_t k, int64_t n, const float* bias, const float* gamma, const float* beta,
-                     int ln_cols, int groups, void* out, float* inv, float* bound, hipStream_t stream) {
-#define QVL_SPLIT_WEIGHT(T, CH)                                                                                       \
-  hipLaunchKernelGGL((split_weight_kernel<T, CH>), dim3((unsigned)((n + 256 / T - 1) / (256 / T))), dim3(256), 0, stream, \
-                     w, (int)k, (int)n, bias, gamma, beta, ln_cols, (f16*)out, inv, bound + groups)
-  if (k <= 1024) QVL_SPLIT_WEIGHT(64, 4);
-  else if (k <= 2048) QVL_SPLIT_WEIGHT(64, 8);
-  else if (k <= 5120) QVL_SPLIT_WEIGHT(256, 5);
-  else QVL_SPLIT_WEIGHT(256, 8);
-#undef QVL_SPLIT_WEIGHT
-  QVL_TRY_RC(check_launch("split_weight"));
-  hipLaunchKernelGGL(group_max_kernel, dim3((unsigned)groups), dim3(256), 0, stream, bound + groups, (int)(n / groups), bound);
+__global__ __launch_bounds__(256) void group_max_kernel(GroupMaxes g) {
+  __shared__ float tmp[4];
+  group_max(g.v[blockIdx.x], g.n[blockIdx.x], g.out[blockIdx.x], tmp);
+}
+
+int split_weights(SplitWeights p, hipStream_t stream) {
+  int k = 0, blocks = 0;
+  for (int i = 0; i < p.count; ++i) {
+    p.e[i].first = blocks;
+    blocks += (p.e[i].n + 3) / 4;
+    k = std::max(k, p.e[i].k);
+  }
+  if (k <= 1024) hipLaunchKernelGGL(split_weights_kernel<4>, dim3(blocks), dim3(256), 0, stream, p);
+  else if (k <= 4096) hipLaunchKernelGGL(split_weights_kernel<16>, dim3(blocks), dim3(256), 0, stream, p);
+  else if (k <= 5120) hipLaunchKernelGGL(split_weights_kernel<20>, dim3(blocks), dim3(256), 0, stream, p);
+  else hipLaunchKernelGGL(split_weights_kernel<32>, dim3(blocks), dim3(256), 0, stream, p);
+  return check_launch("split_weights");
+}
+
+int group_maxes(const GroupMaxes& g, hipStream_t stream) {
+  hipLaunchKernelGGL(group_max_kernel, dim3((unsigned)g.count), dim3(256), 0, stream, g);
   return check_launch("group_max");
 }
 
@@ -200,13 +207,20 @@ int split_weight_f32(const float* w, int64_t k, int64_t n, const float* bias, co
 // LayerNorm fp32 (the arithmetic of layernorm_f32_kernel) written as split rows for the Dense that reads it:
 // no fp32 copy of the normalised rows, and no pass to split them. T threads hold a row; MERGE: the 4 waves of a
 // workgroup normalise 4 consecutive rows that form one row of the output (the 2x2 merge), with one exponent.
+// Workgroups past the rows take the maxima of `gm` (a layer's output bounds, needed by the launches after this one).
 // ---------------------------------------------------------------------------------------------
 template <int T, int CH, bool MERGE>
 __global__ __launch_bounds__(256) void layernorm_split_kernel(const float* __restrict__ x, const float* __restrict__ gamma,
                                                               const float* __restrict__ beta, f16* __restrict__ y,
-                                                              float* __restrict__ inv, int rows, int cols, float eps) {
+                                                              float* __restrict__ inv, int rows, int cols, float eps,
+                                                              GroupMaxes gm) {
   static_assert(!MERGE || T == 64, "a wave per merged row");
   __shared__ float tmp[4];
+  const int first_max = gridDim.x - gm.count;         // the last workgroups: the layer's output bounds
+  if ((int)blockIdx.x >= first_max) {
+    const int g = blockIdx.x - first_max;
+    return group_max(gm.v[g], gm.n[g], gm.out[g], tmp);
+  }
   const int t = threadIdx.x % T, row = blockIdx.x * (256 / T) + threadIdx.x / T;
   if (row >= rows) return;                            // (MERGE: rows % 4 == 0, all waves or none)
   const float* xr = x + (int64_t)row * cols;
@@ -258,11 +272,11 @@ __global__ __launch_bounds__(256) void layernorm_split_kernel(const float* __res
 
 // cols a multiple of 64 (32-column groups), at most kSplitMaxK; merge: rows % 4 == 0, cols <= 2048.
 int layer_norm_split(const float* x, const float* g, const float* b, void* y, float* inv, int rows, int cols, float eps,
-                     bool merge, hipStream_t stream) {
+                     bool merge, const GroupMaxes& gm, hipStream_t stream) {
   if (rows == 0) return QVL_OK;
-#define QVL_LN_SPLIT(T, CH, MERGE)                                                                              \
-  hipLaunchKernelGGL((layernorm_split_kernel<T, CH, MERGE>), dim3((rows + 256 / T - 1) / (256 / T)), dim3(256), 0, \
-                     stream, x, g, b, (f16*)y, inv, rows, cols, eps)
+#define QVL_LN_SPLIT(T, CH, MERGE)                                                                                  \
+  hipLaunchKernelGGL((layernorm_split_kernel<T, CH, MERGE>), dim3((rows + 256 / T - 1) / (256 / T) + gm.count),     \
+                     dim3(256), 0, stream, x, g, b, (f16*)y, inv, rows, cols, eps, gm)
   if (merge) {
     if (cols <= 1024) QVL_LN_SPLIT(64, 4, true);
     else QVL_LN_SPLIT(64, 8, true);
@@ -324,17 +338,23 @@ __device__ __forceinline__ f32x4 split_unscale(f32x4 v, float sx, const f32x4& s
 
 __device__ __forceinline__ bool any_nan(const f32x4& v) { return v[0] != v[0] || v[1] != v[1] || v[2] != v[2] || v[3] != v[3]; }
 
-// Outputs of a row or column that holds infinities or NaN (its scale is NaN), as the fp32 operands give them:
-// serial fp32 sums, left at the first NaN. Rare, so written small and not fast.
+// Outputs of a row or column that holds infinities or NaN (its scale is NaN), as the fp32 operands give them (x from
+// its split rows where there is no other copy): serial fp32 sums, left at the first NaN. Rare, so written small and
+// not fast.
 template <int EPI, bool OUTS>
 __device__ __forceinline__ void split_serial4(const GemmSplitParams& p, int m, int n, const f32x4& bias) {
   f32x4 v;
 #pragma unroll 1
   for (int e = 0; e < 4; ++e) {
     const float *x = p.xf + (int64_t)m * p.ldx, *w = p.wf + (int64_t)(n + e) * p.K;
+    const f16* xs = p.x + (int64_t)m * 2 * p.K;
+    const float fx = split_row_factor(p, m);
     float a = 0.f;
 #pragma unroll 1
-    for (int k = 0; k < p.K && a == a; ++k) a = fmaf(x[k], w[k], a);
+    for (int k = 0; k < p.K && a == a; ++k) {
+      const int at = (k >> 5) * 64 + (k & 31);
+      a = fmaf(p.xf ? x[k] : ((float)xs[at] + (float)xs[at + 32]) * fx, w[k], a);
+    }
     v[0] = e == 0 ? a : v[0]; v[1] = e == 1 ? a : v[1]; v[2] = e == 2 ? a : v[2]; v[3] = e == 3 ? a : v[3];
   }
   split_store4<EPI, OUTS>(p, m, n, v, bias);
@@ -500,12 +520,13 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_split_kernel(GemmSplitPa
       }
     }
   }
-  if (p.split > 1 || !nok || !p.sx) return;
+  const bool rows_nan = p.sx && p.xf;          // (without the fp32 rows no factor is NaN)
+  if (p.split > 1 || !nok || !(w_nan || rows_nan)) return;
 #pragma unroll 1
   for (int r = lane / CH; r < S::TM; r += RPI) {
     const int m = m0 + wm * S::TM + r;
     if (m >= p.M) break;
-    if (w_nan || p.sx[m] != p.sx[m]) split_serial4<EPI, OUTS>(p, m, n, bias);
+    if (w_nan || p.sx[m] != p.sx[m]) split_serial4<EPI, OUTS>(p, m, n, bias);   // (w_nan first: sx may be NULL)
   }
 }
 
@@ -661,9 +682,11 @@ int gemm_f32_split(const GemmF32Params& g, int epi, hipStream_t stream) {
   return gemm_split(p, epi, stream);
 }
 
-int split_rows_f32(const float* x, int64_t ldx, void* out, float* inv, int rows, int k, hipStream_t stream) {
+int split_rows_f32(const float* x, int64_t ldx, void* out, float* inv, int rows, const float* w, void* w_out, float* w_inv,
+                   int w_rows, int k, hipStream_t stream) {
   SplitRowsParams r{};
   r.src[0] = x; r.ld[0] = ldx; r.dst[0] = (f16*)out; r.inv[0] = inv; r.rows[0] = rows;
+  r.src[1] = w; r.ld[1] = k; r.dst[1] = (f16*)w_out; r.inv[1] = w_inv; r.rows[1] = w_rows;
   r.K = k;
   return rows ? split_rows(r, stream) : QVL_OK;
 }

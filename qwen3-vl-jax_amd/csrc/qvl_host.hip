@@ -626,16 +626,79 @@ static int split_dense(hipStream_t st, const qvl_split_dense& d, const SplitDens
   return gemm_split(p, epi, st);
 }
 
+// One layer's Dense weights in split form, in scratch that the next layer uses again: rows, factors, bounds. The
+// bounds of the Dense layers after a LayerNorm (`groups` of rows each, 0: no LayerNorm) are left to `gm`.
+struct SplitScratch {
+  char *rows, *inv, *bound;
+  SplitWeights p{};
+  GroupMaxes gm{};
+
+  qvl_split_dense add(const void* w, const float* bias, const float* gamma, const float* beta, int64_t ln_cols,
+                      int64_t n, int64_t k, int groups) {
+    SplitWeight& e = p.e[p.count++];
+    e.w = (const float*)w; e.bias = bias; e.gamma = gamma; e.beta = beta; e.ln_cols = (int)ln_cols;
+    e.n = (int)n; e.k = (int)k;
+    e.out = (_Float16*)rows; e.inv = (float*)inv; e.row_bound = (float*)bound;
+    rows += n * k * 4;
+    inv += n * 4;
+    bound += n * 4;
+    const qvl_split_dense d = {e.out, e.inv, (float*)bound};
+    for (int g = 0; g < groups; ++g, bound += 4) {
+      gm.v[gm.count] = e.row_bound + n / groups * g;
+      gm.n[gm.count] = (int)(n / groups);
+      gm.out[gm.count++] = (float*)bound;
+    }
+    bound += 4 * ((4 - groups % 4) % 4);
+    return d;
+  }
+};
+
+// Bytes of scratch for the largest layer (widths are multiples of 64), and where its parts lie.
+struct SplitScratchLayout { int64_t rows, n, total; };
+
+static SplitScratchLayout split_scratch_layout(const qvl_vision_config* c) {
+  const int64_t D = c->hidden_size, I = round_up(c->intermediate_size, 64), PV = round_up(c->patch_volume, 64),
+                Dout = c->out_hidden_size, D4 = 4 * D;
+  SplitScratchLayout l;
+  l.rows = 4 * std::max<int64_t>({D * PV, 4 * D * D + 2 * D * I, D4 * (D4 + Dout)});
+  l.n = std::max<int64_t>(5 * D + I, D4 + Dout);
+  l.total = l.rows + 4 * (l.n + l.n + 16);
+  return l;
+}
+
+static SplitScratch split_scratch(const qvl_vision_config* c, void* base) {
+  const SplitScratchLayout l = split_scratch_layout(c);
+  char* b = (char*)base;
+  return SplitScratch{b, b + l.rows, b + l.rows + 4 * l.n};
+}
+
+static qvl_split_block add_block(SplitScratch& s, const TowerLayout& L, const qvl_block_weights& B) {
+  const int64_t D = L.D, I = L.I_pad;
+  return {s.add(B.qkv_w, B.qkv_b, B.norm1_w, B.norm1_b, D, 3 * D, D, 3),
+          s.add(B.proj_w, B.proj_b, nullptr, nullptr, 0, D, D, 0),
+          s.add(B.fc1_w, B.fc1_b, B.norm2_w, B.norm2_b, D, I, D, 1),
+          s.add(B.fc2_w, B.fc2_b, nullptr, nullptr, 0, D, I, 0)};
+}
+
+// norm: over D repeated 4 times along the row (the main merger), or over the row.
+static qvl_split_merger add_merger(SplitScratch& s, const qvl_vision_config* c, const TowerLayout& L,
+                                   const qvl_merger_weights& m, bool postshuffle) {
+  const int64_t D4 = 4 * L.D;
+  return {s.add(m.fc1_w, m.fc1_b, m.norm_w, m.norm_b, postshuffle ? D4 : L.D, D4, D4, 1),
+          s.add(m.fc2_w, m.fc2_b, nullptr, nullptr, 0, c->out_hidden_size, D4, 0)};
+}
+
 // VisionPatchMerger.__call__ (model.py:648-656) in fp32 on split rows; h takes the hidden rows, xn the
 // normalised ones.
 static int run_merger_split(hipStream_t st, const qvl_vision_config* c, const TowerLayout& L, const qvl_merger_weights& mw,
-                            const qvl_split_merger& sm, bool postshuffle, const void* x, void* xn, void* h, void* out,
-                            float* sx, void* part) {
+                            const qvl_split_merger& sm, const GroupMaxes& gm, bool postshuffle, const void* x, void* xn,
+                            void* h, void* out, float* sx, void* part) {
   const int64_t N = L.N, D4 = 4 * L.D;
   if (postshuffle)
-    QVL_TRY_RC(layer_norm_split((const float*)x, mw.norm_w, mw.norm_b, xn, sx, (int)(N / 4), (int)D4, c->ln_eps, false, st));
+    QVL_TRY_RC(layer_norm_split((const float*)x, mw.norm_w, mw.norm_b, xn, sx, (int)(N / 4), (int)D4, c->ln_eps, false, gm,
+                                st));
   else
-    QVL_TRY_RC(layer_norm_split((const float*)x, mw.norm_w, mw.norm_b, xn, sx, (int)N, (int)L.D, c->ln_eps, true, st));
+    QVL_TRY_RC(layer_norm_split((const float*)x, mw.norm_w, mw.norm_b, xn, sx, (int)N, (int)L.D, c->ln_eps, true, gm, st));
   QVL_TRY_RC(split_dense(st, sm.fc1, {xn, sx, nullptr, nullptr, 0, N / 4, D4, D4}, mw.fc1_w, mw.fc1_b, QVL_EPI_BIAS_GELU,
                          nullptr, nullptr, h, part, L.part_bytes));
   return split_dense(st, sm.fc2, {h, nullptr, sm.fc1.bound, nullptr, 0, N / 4, c->out_hidden_size, D4}, mw.fc2_w, mw.fc2_b,
@@ -676,9 +739,11 @@ static int run_merger(hipStream_t st, const qvl_vision_config* c, const TowerLay
   return QVL_OK;
 }
 
+// split: the fp32 Dense weights split beforehand; scratch: each layer's are split into it before they are used (at
+// most one of the two; neither: the entries' own choice per Dense).
 static int encode_impl(void* stream, const qvl_vision_config* c, const qvl_vision_weights* W,
-                       const qvl_vision_split* split, const qvl_vision_metadata_dev* meta, const float* px, void* tokens,
-                       void* const* deepstack, void* ws, size_t ws_bytes) {
+                       const qvl_vision_split* split, void* scratch, const qvl_vision_metadata_dev* meta, const float* px,
+                       void* tokens, void* const* deepstack, void* ws, size_t ws_bytes) {
   if (!W || !meta) return set_error(QVL_ERR_INVALID_ARG, "encode_vision: NULL weights/metadata");
   TowerLayout L;
   QVL_TRY_RC(tower_layout(c, meta->n_tokens, &L));
@@ -772,13 +837,34 @@ static int encode_impl(void* stream, const qvl_vision_config* c, const qvl_visio
       }
     return qkv_of(i + 1);
   };
-  // (with split weights the pixel rows are split into the then idle q / k / v buffers)
-  const bool split_px = split && (size_t)N * L.PVp * 4 <= L.off_h - L.off_q;
+  const auto merge_split = [&](const qvl_merger_weights& m, const qvl_split_merger* sm, bool postshuffle, void* out) {
+    qvl_split_merger made;
+    GroupMaxes gm{};
+    if (!sm) {
+      SplitScratch s = split_scratch(c, scratch);
+      made = add_merger(s, c, L, m, postshuffle);
+      gm = s.gm;
+      QVL_TRY_RC(split_weights(s.p, st));
+    }
+    return run_merger_split(st, c, L, m, sm ? *sm : made, gm, postshuffle, x, xn, h, out, sx, part);
+  };
+  // (with split weights the pixel rows are split into the then idle q / k / v buffers, in one launch with the patch
+  // weights where those are split here)
+  const bool split_px = (split || scratch) && (size_t)N * L.PVp * 4 <= L.off_h - L.off_q;
   if (split_px) {
     if (c->num_position_embeddings > 0)
       QVL_TRY_RC(qvl_pos_embed(st, dt, W->pos_table, meta->tap_idx, meta->tap_w, xn, N, D));
-    QVL_TRY_RC(split_rows_f32((const float*)px_in, L.PVp, Qb, sx, (int)N, (int)L.PVp, st));
-    QVL_TRY_RC(split_dense(st, split->patch, {Qb, sx, nullptr, (const float*)px_in, L.PVp, N, D, L.PVp}, W->patch_w,
+    qvl_split_dense patch{};
+    if (split) {
+      patch = split->patch;
+      QVL_TRY_RC(split_rows_f32((const float*)px_in, L.PVp, Qb, sx, (int)N, nullptr, nullptr, nullptr, 0, (int)L.PVp, st));
+    } else {
+      const SplitScratch s = split_scratch(c, scratch);
+      patch = {s.rows, (float*)s.inv, nullptr};
+      QVL_TRY_RC(split_rows_f32((const float*)px_in, L.PVp, Qb, sx, (int)N, (const float*)W->patch_w, s.rows,
+                                (float*)s.inv, (int)D, (int)L.PVp, st));
+    }
+    QVL_TRY_RC(split_dense(st, patch, {Qb, sx, nullptr, (const float*)px_in, L.PVp, N, D, L.PVp}, W->patch_w,
                            W->patch_b, c->num_position_embeddings > 0 ? QVL_EPI_BIAS_RESIDUAL : QVL_EPI_BIAS,
                            (const float*)xn, x, nullptr, part, PB));
   } else if (c->num_position_embeddings > 0 && !f32 && D % 8 == 0) {
@@ -809,11 +895,20 @@ static int encode_impl(void* stream, const qvl_vision_config* c, const qvl_visio
     // statistics run before it)
     const bool fold = !f32 && B.qkv_ln.w && B.qkv_ln.cd && B.fc1_ln.w && B.fc1_ln.cd;
     const qvl_split_block* sb = split ? &split->blocks[i] : nullptr;
+    qvl_split_block made;
+    GroupMaxes gm{};
+    if (scratch) {
+      SplitScratch s = split_scratch(c, scratch);
+      made = add_block(s, L, B);
+      sb = &made;
+      gm = s.gm;
+      QVL_TRY_RC(split_weights(s.p, st));
+    }
     // x += proj(attention(rotary(qkv(LN1 x))))   (model.py:628, 569-601)
     if (fold) {
       if (!have_parts) QVL_TRY_RC(qvl_row_stats(st, dt, x, D, N, D, c->ln_eps, stats));
     } else if (sb) {
-      QVL_TRY_RC(layer_norm_split((const float*)x, B.norm1_w, B.norm1_b, xn, sx, (int)N, (int)D, c->ln_eps, false, st));
+      QVL_TRY_RC(layer_norm_split((const float*)x, B.norm1_w, B.norm1_b, xn, sx, (int)N, (int)D, c->ln_eps, false, gm, st));
     } else {
       QVL_TRY_RC(qvl_layer_norm(st, dt, x, D, B.norm1_w, B.norm1_b, xn, D, N, D, c->ln_eps));
     }
@@ -888,7 +983,7 @@ static int encode_impl(void* stream, const qvl_vision_config* c, const qvl_visio
       // split rows, fc2
       QVL_TRY_RC(split_dense(st, sb->proj, {xn, nullptr, sb->qkv.bound + 2, nullptr, 0, N, D, D}, B.proj_w, B.proj_b,
                              QVL_EPI_BIAS_RESIDUAL, (const float*)x, x, nullptr, part, PB));
-      QVL_TRY_RC(layer_norm_split((const float*)x, B.norm2_w, B.norm2_b, xn, sx, (int)N, (int)D, c->ln_eps, false, st));
+      QVL_TRY_RC(layer_norm_split((const float*)x, B.norm2_w, B.norm2_b, xn, sx, (int)N, (int)D, c->ln_eps, false, {}, st));
       QVL_TRY_RC(split_dense(st, sb->fc1, {xn, sx, nullptr, nullptr, 0, N, I, D}, B.fc1_w, B.fc1_b, QVL_EPI_BIAS_GELU,
                              nullptr, nullptr, h, part, PB));
       QVL_TRY_RC(split_dense(st, sb->fc2, {h, nullptr, sb->fc1.bound, nullptr, 0, N, D, I}, B.fc2_w, B.fc2_b,
@@ -923,9 +1018,8 @@ static int encode_impl(void* stream, const qvl_vision_config* c, const qvl_visio
     for (int j = 0; j < c->n_deepstack; ++j)
       if (c->deepstack_indexes[j] == i) {
         void* out = win ? (void*)Qb : deepstack[ds_next];
-        if (split)
-          QVL_TRY_RC(run_merger_split(st, c, L, W->deepstack[ds_next], split->deepstack[ds_next], true, x, xn, h, out, sx,
-                                      part));
+        if (split || scratch)
+          QVL_TRY_RC(merge_split(W->deepstack[ds_next], split ? &split->deepstack[ds_next] : nullptr, true, out));
         else
           QVL_TRY_RC(run_merger(st, c, L, W->deepstack[ds_next], true, x, xn, h, out, part, stats, have_parts ? G : 0,
                                 qkv_of(i + 1)));
@@ -935,8 +1029,8 @@ static int encode_impl(void* stream, const qvl_vision_config* c, const qvl_visio
       }
   }
   (void)e;
-  if (split)
-    QVL_TRY_RC(run_merger_split(st, c, L, W->merger, split->merger, false, x, xn, h, win ? (void*)Qb : tokens, sx, part));
+  if (split || scratch)
+    QVL_TRY_RC(merge_split(W->merger, split ? &split->merger : nullptr, false, win ? (void*)Qb : tokens));
   else
     QVL_TRY_RC(run_merger(st, c, L, W->merger, false, x, xn, h, win ? (void*)Qb : tokens, part, stats, 0, {}));
   if (win) QVL_TRY_RC(qvl_gather_rows(st, dt, Qb, Dout, dt, tokens, Dout, meta->window_reverse, N / 4, 1, Dout));
@@ -946,7 +1040,16 @@ static int encode_impl(void* stream, const qvl_vision_config* c, const qvl_visio
 int qvl_encode_vision(void* stream, const qvl_vision_config* c, const qvl_vision_weights* W,
                       const qvl_vision_metadata_dev* meta, const float* px, void* tokens, void* const* deepstack,
                       void* ws, size_t ws_bytes) {
-  return encode_impl(stream, c, W, nullptr, meta, px, tokens, deepstack, ws, ws_bytes);
+  return encode_impl(stream, c, W, nullptr, nullptr, meta, px, tokens, deepstack, ws, ws_bytes);
+}
+
+static int check_split_config(const char* what, const qvl_vision_config* c) {
+  if (!c) return set_error(QVL_ERR_INVALID_ARG, "%s: NULL config", what);
+  if (c->dtype != QVL_DTYPE_F32) return set_error(QVL_ERR_UNSUPPORTED, "%s: dtype %d (fp32 only)", what, c->dtype);
+  if (round_up(c->patch_volume, 64) > kSplitMaxK || round_up(c->intermediate_size, 64) > kSplitMaxK ||
+      4 * (int64_t)c->hidden_size > kSplitMaxK)
+    return set_error(QVL_ERR_UNSUPPORTED, "%s: rows longer than %d", what, kSplitMaxK);
+  return QVL_OK;
 }
 
 int qvl_encode_vision_split(void* stream, const qvl_vision_config* c, const qvl_vision_weights* W,
@@ -954,10 +1057,7 @@ int qvl_encode_vision_split(void* stream, const qvl_vision_config* c, const qvl_
                             void* tokens, void* const* deepstack, void* ws, size_t ws_bytes) {
   if (!c || !split || !split->blocks || (c->n_deepstack > 0 && !split->deepstack))
     return set_error(QVL_ERR_INVALID_ARG, "encode_vision_split: NULL config / split weights");
-  if (c->dtype != QVL_DTYPE_F32) return set_error(QVL_ERR_UNSUPPORTED, "encode_vision_split: dtype %d (fp32 only)", c->dtype);
-  if (round_up(c->patch_volume, 64) > kSplitMaxK || round_up(c->intermediate_size, 64) > kSplitMaxK ||
-      4 * (int64_t)c->hidden_size > kSplitMaxK)
-    return set_error(QVL_ERR_UNSUPPORTED, "encode_vision_split: rows longer than %d", kSplitMaxK);
+  QVL_TRY_RC(check_split_config("encode_vision_split", c));
   const auto whole = [](const qvl_split_dense& d, bool bound) { return d.w && d.scale && (!bound || d.bound); };
   bool ok = whole(split->patch, false) && whole(split->merger.fc1, true) && whole(split->merger.fc2, false);
   for (int i = 0; i < c->depth; ++i) {
@@ -967,7 +1067,67 @@ int qvl_encode_vision_split(void* stream, const qvl_vision_config* c, const qvl_
   for (int j = 0; j < c->n_deepstack; ++j)
     ok = ok && whole(split->deepstack[j].fc1, true) && whole(split->deepstack[j].fc2, false);
   if (!ok) return set_error(QVL_ERR_INVALID_ARG, "encode_vision_split: NULL split weight");
-  return encode_impl(stream, c, W, split, meta, px, tokens, deepstack, ws, ws_bytes);
+  return encode_impl(stream, c, W, split, nullptr, meta, px, tokens, deepstack, ws, ws_bytes);
+}
+
+int qvl_vision_split_scratch_size(const qvl_vision_config* c, size_t* bytes) {
+  QVL_TRY_RC(check_split_config("vision_split_scratch", c));
+  TowerLayout L;
+  QVL_TRY_RC(tower_layout(c, 0, &L));
+  if (!bytes) return set_error(QVL_ERR_INVALID_ARG, "bytes is NULL");
+  *bytes = (size_t)split_scratch_layout(c).total;
+  return QVL_OK;
+}
+
+static int check_split_scratch(const char* what, const qvl_vision_config* c, const qvl_vision_weights* W,
+                               const void* scratch, size_t scratch_bytes) {
+  QVL_TRY_RC(check_split_config(what, c));
+  if (!W || !W->blocks || (c->n_deepstack > 0 && !W->deepstack)) return set_error(QVL_ERR_INVALID_ARG, "%s: NULL weights", what);
+  const size_t need = (size_t)split_scratch_layout(c).total;
+  if (!scratch || scratch_bytes < need) return set_error(QVL_ERR_WORKSPACE, "%s: scratch %zu < %zu", what, scratch_bytes, need);
+  if (!aligned16(scratch)) return set_error(QVL_ERR_MISALIGNED, "%s: scratch alignment", what);
+  return QVL_OK;
+}
+
+int qvl_encode_vision_split_scratch(void* stream, const qvl_vision_config* c, const qvl_vision_weights* W,
+                                    const qvl_vision_metadata_dev* meta, const float* px, void* tokens,
+                                    void* const* deepstack, void* ws, size_t ws_bytes, void* scratch,
+                                    size_t scratch_bytes) {
+  QVL_TRY_RC(check_split_scratch("encode_vision_split_scratch", c, W, scratch, scratch_bytes));
+  return encode_impl(stream, c, W, nullptr, scratch, meta, px, tokens, deepstack, ws, ws_bytes);
+}
+
+int qvl_vision_split_bounds(void* stream, const qvl_vision_config* c, const qvl_vision_weights* W, void* scratch,
+                            size_t scratch_bytes, float* bounds) {
+  QVL_TRY_RC(check_split_scratch("vision_split_bounds", c, W, scratch, scratch_bytes));
+  TowerLayout L;
+  QVL_TRY_RC(tower_layout(c, 0, &L));
+  if (!bounds) return set_error(QVL_ERR_INVALID_ARG, "vision_split_bounds: NULL bounds");
+  hipStream_t st = (hipStream_t)stream;
+  const auto layer = [&](const SplitScratch& s, float* out) {
+    QVL_TRY_RC(split_weights(s.p, st));
+    GroupMaxes g{};
+    for (int i = 0; i < s.p.count; ++i) {
+      g.v[i] = s.p.e[i].row_bound;
+      g.n[i] = s.p.e[i].n;
+      g.out[i] = out + i;
+    }
+    g.count = s.p.count;
+    return group_maxes(g, st);
+  };
+  for (int i = 0; i < c->depth; ++i, bounds += 4) {
+    SplitScratch s = split_scratch(c, scratch);
+    add_block(s, L, W->blocks[i]);
+    QVL_TRY_RC(layer(s, bounds));
+  }
+  for (int j = -1; j < c->n_deepstack; ++j, bounds += 2) {
+    SplitScratch s = split_scratch(c, scratch);
+    add_merger(s, c, L, j < 0 ? W->merger : W->deepstack[j], j >= 0);
+    QVL_TRY_RC(layer(s, bounds));
+  }
+  SplitScratch s = split_scratch(c, scratch);
+  s.add(W->patch_w, W->patch_b, nullptr, nullptr, 0, L.D, L.PVp, 0);
+  return layer(s, bounds);
 }
 
 int qvl_split_dense_weight(void* stream, const float* w, int64_t k_in, int64_t n_out, const float* bias,
@@ -981,8 +1141,20 @@ int qvl_split_dense_weight(void* stream, const float* w, int64_t k_in, int64_t n
     return set_error(QVL_ERR_INVALID_ARG, "split_dense_weight: NULL operand");
   if (!aligned16(w) || !aligned16(out_w) || !aligned16(out_scale) || !aligned16(gamma) || !aligned16(beta))
     return set_error(QVL_ERR_MISALIGNED, "split_dense_weight: operands must be 16-byte aligned");
-  return split_weight_f32(w, k_in, n_out, bias, gamma, beta, (int)ln_cols, groups, out_w, out_scale, out_bound,
-                          (hipStream_t)stream);
+  SplitWeights p{};
+  p.count = 1;
+  p.e[0] = {w, bias, gamma, beta, (_Float16*)out_w, out_scale, out_bound + groups, (int)n_out, (int)k_in, (int)ln_cols, 0};
+  QVL_TRY_RC(split_weights(p, (hipStream_t)stream));
+  for (int g = 0; g < groups; g += 4) {
+    GroupMaxes gm{};
+    for (; gm.count < 4 && g + gm.count < groups; ++gm.count) {
+      gm.v[gm.count] = out_bound + groups + (int64_t)(g + gm.count) * (n_out / groups);
+      gm.n[gm.count] = (int)(n_out / groups);
+      gm.out[gm.count] = out_bound + g + gm.count;
+    }
+    QVL_TRY_RC(group_maxes(gm, (hipStream_t)stream));
+  }
+  return QVL_OK;
 }
 
 }  // extern "C"

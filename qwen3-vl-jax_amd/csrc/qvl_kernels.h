@@ -101,6 +101,19 @@ struct GemmSplitParams {
   int split, group_n;
 };
 
+// The Dense weights of one layer that one launch writes as split rows (split_weights): w [n][k] packed fp32, gamma /
+// beta [ln_cols] of the LayerNorm before it repeat along the row (NULL: 1 / 0). first: set by the launcher.
+struct SplitWeight {
+  const float *w, *bias, *gamma, *beta;
+  _Float16* out;
+  float *inv, *row_bound;
+  int n, k, ln_cols, first;
+};
+struct SplitWeights { SplitWeight e[4]; int count; };
+
+// out[i] = the largest of the n[i] values v[i] (>= 0, or NaN, which wins).
+struct GroupMaxes { const float* v[4]; float* out[4]; int n[4]; int count; };
+
 // Floats of split-K partial workspace that lets every GEMM of up to 256x256 tiles split its tail
 // on a device with `cus` compute units (one tail unit per CU, at most one tile of partials each).
 inline int64_t gemm_partials_elems(int cus) { return (int64_t)cus * 256 * 256; }
@@ -154,11 +167,13 @@ int gemm_f32_split(const GemmF32Params& g, int epi, hipStream_t stream);
 int gemm_f32_set_plan(int tile);
 constexpr int kSplitMaxK = 8192;   // the longest row the split kernels hold
 int gemm_split(const GemmSplitParams& p, int epi, hipStream_t stream);
-int split_rows_f32(const float* x, int64_t ldx, void* out, float* inv, int rows, int k, hipStream_t stream);
-int split_weight_f32(const float* w, int64_t k, int64_t n, const float* bias, const float* gamma, const float* beta,
-                     int ln_cols, int groups, void* out, float* inv, float* bound, hipStream_t stream);
+// x [rows] (and, w_rows > 0, w) -> split rows; a row's factor is NaN where it holds an infinity or a NaN.
+int split_rows_f32(const float* x, int64_t ldx, void* out, float* inv, int rows, const float* w, void* w_out, float* w_inv,
+                   int w_rows, int k, hipStream_t stream);
+int split_weights(SplitWeights p, hipStream_t stream);
+int group_maxes(const GroupMaxes& g, hipStream_t stream);
 int layer_norm_split(const float* x, const float* g, const float* b, void* y, float* inv, int rows, int cols, float eps,
-                     bool merge, hipStream_t stream);
+                     bool merge, const GroupMaxes& gm, hipStream_t stream);
 int layer_norm_f32(const float* x, int64_t ldx, const float* g, const float* b, float* y, int64_t ldy, int rows,
                    int cols, float eps, hipStream_t stream);
 int pos_embed_f32(const float* table, const int* idx, const float* wts, float* y, int n_tok, int dim,

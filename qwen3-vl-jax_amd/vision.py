@@ -411,8 +411,7 @@ class Qwen3VisionTransformer:
         # tolerances). ln_fold=False runs the reference's LayerNorm launches.
         self.ln_fold = bool(ln_fold) and self.qdtype == capi.QVL_DTYPE_BF16
         self._folds: Dict[str, tuple] = {}
-        self._split = None            # fp32: the Dense weights as f16-split rows (_split_weights)
-        self._split_of = None         # the write counts of the buffers those were made from
+        self._split = None            # fp32: scratch for a layer's Dense weights as f16-split rows (_split_scratch)
         self._lib = capi.load()
         self._w = None
         self._keep = []
@@ -484,77 +483,23 @@ class Qwen3VisionTransformer:
                                                 beta.data_ptr(), out.data_ptr(), cd.data_ptr()), "qvl_fold_ln_weight")
         return out, cd
 
-    def _split_weights(self, st: Dict[str, object]):
-        """The fp32 tower's Dense weights once more as f16-split rows (qvl_split_dense_weight), so that its
-        forwards run on the f16 matrix cores: (qvl_vision_split struct, what it points to), or None
-        where the widths or the weights' values rule it out (non-finite weights, or norms that
-        overflow): the forward then splits or not per Dense, as qvl_dense_ws does."""
+    def _split_scratch(self):
+        """fp32: the device buffer each layer's Dense weights are split into, on the stream before the layer, so that
+        its Dense runs on the f16 matrix cores (qvl_encode_vision_split_scratch); or None where the widths or the
+        weights' values rule it out (non-finite weights, or norms that overflow): the forward then splits or not per
+        Dense, as qvl_dense_ws does. No forward keeps anything derived from the weights."""
         torch = _torch()
         s = self.spec
-        D, M4 = s.hidden_size, s.hidden_size * s.spatial_merge_size ** 2
-        if max(M4, st["patch_embed.w"].shape[1], st["blocks.0.fc2.w"].shape[1] if s.depth else 0) > 8192:
+        nb = C.c_size_t()
+        if self._lib.qvl_vision_split_scratch_size(C.byref(self._cfg), C.byref(nb)) != 0:
             return None
-        taps = len(s.deepstack_visual_indexes)
-        names = ["patch_embed"] + [f"{m}.{f}" for m in ["merger"] + [f"deepstack.{j}" for j in range(taps)]
-                                   for f in ("fc1", "fc2")]
-        names += [f"blocks.{i}.{d}" for i in range(s.depth) for d in ("qkv", "proj", "fc1", "fc2")]
-        # one allocation each: the split rows (2 f16 per value), the row factors, the output bounds
-        rows = torch.empty(sum(st[n + ".w"].numel() for n in names), dtype=torch.int32, device=self.device)
-        scales = torch.empty(sum(st[n + ".w"].shape[0] for n in names), dtype=torch.float32, device=self.device)
-        bounds = torch.empty(len(names) + 2 * s.depth + scales.numel(), dtype=torch.float32, device=self.device)
-        at = [rows.data_ptr(), scales.data_ptr(), bounds.data_ptr()]
-        stream = self._stream()
-
-        def split(name, norm=None, groups=1):
-            w = st[name + ".w"]
-            n, k = w.shape
-            g, b = (st[norm + ".w"], st[norm + ".b"]) if norm else (None, None)
-            capi.check(self._lib.qvl_split_dense_weight(stream, w.data_ptr(), k, n, st[name + ".b"].data_ptr(),
-                                                        _ptr(g) or None, _ptr(b) or None, g.numel() if norm else 0,
-                                                        groups, *at), "qvl_split_dense_weight")
-            d = capi.SplitDense(*at)
-            at[0] += 4 * n * k
-            at[1] += 4 * n
-            at[2] += 4 * (groups + n)
-            return d
-
-        def merger(name):
-            return capi.SplitMerger(split(name + ".fc1", name + ".norm"), split(name + ".fc2"))
-
-        blocks = (capi.SplitBlock * max(s.depth, 1))()
-        for i in range(s.depth):
-            p = f"blocks.{i}."
-            blocks[i] = capi.SplitBlock(split(p + "qkv", p + "norm1", 3), split(p + "proj"),
-                                        split(p + "fc1", p + "norm2"), split(p + "fc2"))
-        ds = (capi.SplitMerger * max(taps, 1))()
-        for j in range(taps):
-            ds[j] = merger(f"deepstack.{j}")
-        sp = capi.VisionSplit(split("patch_embed"), blocks, merger("merger"), ds)
-        if not bool(torch.isfinite(bounds).all()):
-            return None
-        return sp, (rows, scales, bounds, blocks, ds)
-
-    def _writes(self):
-        """torch's count of in-place writes to each bound buffer (inference tensors have none)."""
-        return [0 if t.is_inference() else t._version for t in self._state.values()]
-
-    def _current_split(self):
-        """The split weights, made anew where a bound buffer was written in place (packed_state, or the tensors
-        given to bind_packed, an optimizer's step on them): the forward follows such writes as it does without them.
-        During a stream capture, where they cannot be made (the check of their bounds waits for the GPU), a forward
-        after such a write reads the buffers themselves. The check costs 60 ns a buffer."""
-        if self._split is None:
-            return None
-        writes = self._writes()
-        if writes != self._split_of:
-            torch = _torch()
-            if torch.cuda.is_current_stream_capturing():
-                return None
-            split = self._split_weights(self._state)
-            if split is None:
-                return None           # no longer finite: looked at again on the next call
-            self._split, self._split_of = split, writes
-        return self._split
+        buf = torch.empty(nb.value, dtype=torch.uint8, device=self.device)
+        bounds = torch.empty(4 * s.depth + 2 * (1 + len(s.deepstack_visual_indexes)) + 1, dtype=torch.float32,
+                             device=self.device)
+        capi.check(self._lib.qvl_vision_split_bounds(self._stream(), C.byref(self._cfg), C.byref(self._w),
+                                                     buf.data_ptr(), nb.value, bounds.data_ptr()),
+                   "qvl_vision_split_bounds")
+        return buf if bool(torch.isfinite(bounds).all()) else None
 
     def _vec(self, v):
         torch = _torch()
@@ -692,8 +637,7 @@ class Qwen3VisionTransformer:
         self._blocks_arr, self._ds_arr = blocks, ds
         self._w = W
         if self.qdtype == capi.QVL_DTYPE_F32:
-            self._split_of = self._writes()
-            self._split = self._split_weights(st)
+            self._split = self._split_scratch()
         return self
 
     # -- per-grid metadata ----------------------------------------------------------------------
@@ -783,12 +727,11 @@ class Qwen3VisionTransformer:
               for _ in s.deepstack_visual_indexes]
         ds_ptrs = (C.c_void_p * max(len(ds), 1))(*[t.data_ptr() for t in ds])
         ws, nbytes = self.workspace(N)
-        split = self._current_split()
-        if split is not None:
-            capi.check(self._lib.qvl_encode_vision_split(self._stream(), C.byref(self._cfg), C.byref(self._w),
-                                                         C.byref(split[0]), C.byref(md), px.data_ptr(),
-                                                         tokens.data_ptr(), ds_ptrs, ws.data_ptr(), nbytes),
-                       "qvl_encode_vision_split")
+        if self._split is not None:
+            capi.check(self._lib.qvl_encode_vision_split_scratch(
+                self._stream(), C.byref(self._cfg), C.byref(self._w), C.byref(md), px.data_ptr(), tokens.data_ptr(),
+                ds_ptrs, ws.data_ptr(), nbytes, self._split.data_ptr(), self._split.numel()),
+                "qvl_encode_vision_split_scratch")
         else:
             capi.check(self._lib.qvl_encode_vision(self._stream(), C.byref(self._cfg), C.byref(self._w), C.byref(md),
                                                    px.data_ptr(), tokens.data_ptr(), ds_ptrs, ws.data_ptr(), nbytes),

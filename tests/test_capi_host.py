@@ -357,3 +357,30 @@ def test_injection_refuses_host_memory(pkg, monkeypatch, which):
         io._scatter_flagged(hidden, rows, flags, 1, cp.QVL_SCATTER_ADD)
     with pytest.raises(ValueError, match="cpu"):
         io.apply_deepstack(hidden, flags, rows)
+
+
+def test_split_scratch_argument_checks(pkg):
+    cp, lib = pkg.capi, pkg.capi.load()
+    t = pkg.Qwen3VisionTransformer
+    cfg = t(pkg.spec_2b())._cfg
+    nb = C.c_size_t()
+    assert lib.qvl_vision_split_scratch_size(C.byref(cfg), None) == -1
+    assert lib.qvl_vision_split_scratch_size(None, C.byref(nb)) == -1
+    assert lib.qvl_vision_split_scratch_size(C.byref(t(pkg.spec_2b(), dtype="bfloat16")._cfg), C.byref(nb)) == -2
+    assert lib.qvl_vision_split_scratch_size(C.byref(cfg), C.byref(nb)) == 0
+    # the largest layer: a merger's two weights, 4 bytes a value, with factors and bounds of its rows
+    assert 4 * 4096 * (4096 + 2048) < nb.value < 4 * 4096 * (4096 + 2048) + 16 * (4096 + 2048)
+    W, md, fake = cp.VisionWeights(), cp.VisionMetadataDev(), 4096
+    blocks = (cp.BlockWeights * 24)()
+    ds = (cp.MergerWeights * 3)()
+
+    def call(w, scratch, size):
+        return lib.qvl_encode_vision_split_scratch(None, C.byref(cfg), w, C.byref(md), fake, fake, None, fake, 1 << 40,
+                                                   scratch, size)
+    assert call(C.byref(W), fake, nb.value) == -1            # no blocks
+    W.blocks, W.deepstack = blocks, ds
+    assert call(None, fake, nb.value) == -1
+    assert call(C.byref(W), None, nb.value) == call(C.byref(W), fake, nb.value - 1) == -4
+    assert call(C.byref(W), fake + 8, nb.value) == -3
+    assert call(C.byref(W), fake, nb.value) == 0             # no tokens: nothing to do
+    assert lib.qvl_vision_split_bounds(None, C.byref(cfg), C.byref(W), fake, nb.value, None) == -1

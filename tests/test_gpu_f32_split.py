@@ -232,3 +232,121 @@ def test_split_weights_follow_writes_to_the_bound_buffers(pkg):
     assert not torch.isfinite(tokens[:, 5]).any() and torch.isfinite(tokens[:, :5]).all()
     w[5, 3] = old
     assert torch.equal(t(px, grids)[0], before)
+
+
+def one_block(pkg):
+    spec = pkg.spec_2b()
+    spec.depth, spec.deepstack_visual_indexes = 1, (0,)
+    grids = np.array([[1, 4, 6]], np.int32)
+    px = torch.from_numpy(np.random.default_rng(3).standard_normal((24, spec.patch_volume), dtype=np.float32)).to(DEV)
+    return spec, pkg.random_params(spec, seed=2), px, grids
+
+
+def outputs(tower, px, grids):
+    tokens, ds = tower(px, grids)
+    return [t.clone() for t in (tokens, *ds)]
+
+
+def fresh(pkg, tower, px, grids):
+    return outputs(pkg.Qwen3VisionTransformer(tower.spec).bind_packed(tower.packed_state()), px, grids)
+
+
+WRITES = (("blocks.0.fc1.w", 0.01), ("blocks.0.qkv.b", 3.0), ("blocks.0.norm1.w", 50.0), ("deepstack.0.fc1.w", 0.02),
+          ("patch_embed.w", 0.01), ("merger.fc2.w", 0.03))
+
+
+def same(got, want):
+    return all(torch.equal(a, b) for a, b in zip(got, want))
+
+
+@pytest.mark.parametrize("how", ["data", "inference", "dlpack"])
+def test_split_tower_follows_writes_that_torch_does_not_count(pkg, how):
+    """Writes through .data, to inference tensors and through DLPack leave torch's version counts as they were; the next
+    forward reads the written weights all the same."""
+    spec, params, px, grids = one_block(pkg)
+    with torch.inference_mode(how == "inference"):
+        t = pkg.Qwen3VisionTransformer(spec).bind(params)
+        assert t._split is not None
+        before = outputs(t, px, grids)
+        for name, by in WRITES:
+            w = t.packed_state()[name]
+            (w.data if how == "data" else torch.utils.dlpack.from_dlpack(w) if how == "dlpack" else w).add_(by)
+            got = outputs(t, px, grids)
+            assert same(got, fresh(pkg, t, px, grids)) and not same(got, before), name
+            before = got
+
+
+def test_captured_split_forward_follows_writes(pkg):
+    """A graph captured around a forward, weights written, other forwards and allocations in between: each replay gives
+    what a tower bound to the buffers as they are then gives."""
+    spec, params, px, grids = one_block(pkg)
+    t = pkg.Qwen3VisionTransformer(spec).bind(params)
+    before = outputs(t, px, grids)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        tokens, ds = t(px, grids)
+    graph.replay()
+    torch.cuda.synchronize()
+    assert same((tokens, *ds), before)
+    for name, by in WRITES:
+        t.packed_state()[name].add_(by)
+        graph.replay()                                   # no forward since the write
+        torch.cuda.synchronize()
+        want = fresh(pkg, t, px, grids)
+        assert same((tokens, *ds), want) and not same(want, before), name
+        assert same(outputs(t, px, grids), want)
+        junk = [torch.full((1 << 22,), float("nan"), device=DEV) for _ in range(8)]
+        graph.replay()
+        torch.cuda.synchronize()
+        assert same((tokens, *ds), want), name
+        before = want
+        del junk
+
+
+def split_beforehand(pkg, lib, t):
+    """qvl_vision_split of a bound tower, made by qvl_split_dense_weight: (struct, what it points to)."""
+    cp, st, keep = pkg.capi, t.packed_state(), []
+
+    def split(name, norm=None, groups=1):
+        w = st[name + ".w"]
+        n, k = w.shape
+        g, b = (st[norm + ".w"], st[norm + ".b"]) if norm else (None, None)
+        out = [torch.empty(m, device=DEV) for m in (n * k, n, groups + n)]
+        cp.check(lib.qvl_split_dense_weight(torch.cuda.current_stream().cuda_stream, w.data_ptr(), k, n,
+                                            st[name + ".b"].data_ptr(), g.data_ptr() if norm else None,
+                                            b.data_ptr() if norm else None, g.numel() if norm else 0, groups,
+                                            *(o.data_ptr() for o in out)))
+        keep.extend(out)
+        return cp.SplitDense(*(o.data_ptr() for o in out))
+
+    def merger(name):
+        return cp.SplitMerger(split(name + ".fc1", name + ".norm"), split(name + ".fc2"))
+    s = t.spec
+    blocks, ds = (cp.SplitBlock * s.depth)(), (cp.SplitMerger * max(1, len(s.deepstack_visual_indexes)))()
+    for i in range(s.depth):
+        p = f"blocks.{i}."
+        blocks[i] = cp.SplitBlock(split(p + "qkv", p + "norm1", 3), split(p + "proj"), split(p + "fc1", p + "norm2"),
+                                  split(p + "fc2"))
+    for j in range(len(s.deepstack_visual_indexes)):
+        ds[j] = merger(f"deepstack.{j}")
+    return cp.VisionSplit(split("patch_embed"), blocks, merger("merger"), ds), (keep, blocks, ds)
+
+
+@pytest.mark.parametrize("shape", ["spec_2b", "spec_8b"])
+def test_weights_split_beforehand_give_the_same_bits(pkg, lib, shape):
+    """qvl_encode_vision_split on weights that the caller split against the tower's own forward, two blocks and a tap."""
+    cp = pkg.capi
+    spec = getattr(pkg, shape)()
+    spec.depth, spec.deepstack_visual_indexes = 2, (0,)
+    t = pkg.Qwen3VisionTransformer(spec).bind(pkg.random_params(spec, seed=4))
+    grids = np.array([[1, 6, 10], [1, 14, 14]], np.int32)
+    px = torch.randn((256, spec.patch_volume), device=DEV)
+    want = outputs(t, px, grids)
+    split, _keep = split_beforehand(pkg, lib, t)
+    got = [torch.empty_like(o) for o in want]
+    ws, nb = t.workspace(256)
+    cp.check(lib.qvl_encode_vision_split(torch.cuda.current_stream().cuda_stream, C.byref(t._cfg), C.byref(t._w),
+                                         C.byref(split), C.byref(t.metadata(grids)[2]), px.data_ptr(), got[0].data_ptr(),
+                                         (C.c_void_p * 1)(got[1].data_ptr()), ws.data_ptr(), nb))
+    assert same(got, want)
