@@ -117,57 +117,74 @@ static int split_rows(const SplitRowsParams& p, hipStream_t stream) {
 // row_bound). It lets the outputs be split by one exponent that is known before they are. Non-finite weights make
 // it non-finite, and their row's factor NaN.
 // A tower splits each layer's weights on the stream right before they are used, so that a forward (or a graph's
-// replay) reads the weights as they are then; all Dense weights of a layer share one launch, a wave holds a row.
-// Memory bound: a 1024-wide block's 48 MB are read and written. A 784-patch forward of 24 blocks takes 4.53 ms with
-// it, 3.85 with weights split beforehand, and 8.8 on the fp32 MFMA kernels.
+// replay) reads the weights as they are then; all Dense weights of a layer share one launch, a wave or a workgroup
+// holds a row.
+// Memory bound: a 1024-wide block's 48 MB are read and written in 20 us, a copy's 4.7 TB/s (28 us with a wave on every
+// row: 16 chunks of a 4096-wide row are too many registers for the waves that keep the loads in flight). A 784-patch
+// forward of 24 blocks takes 4.37 ms with it, 3.85 with weights split beforehand, and 8.8 on the fp32 MFMA kernels.
 // ---------------------------------------------------------------------------------------------
 template <int CH>
 __global__ __launch_bounds__(256) void split_weights_kernel(SplitWeights p) {
+  __shared__ float tmp[4];
   int which = 0;
   while (which + 1 < p.count && (int)blockIdx.x >= p.e[which + 1].first) ++which;
   const SplitWeight& e = p.e[which];
-  const int lane = threadIdx.x & 63, row = ((int)blockIdx.x - e.first) * 4 + (threadIdx.x >> 6), k = e.k;
-  if (row >= e.n) return;
+  const int k = e.k, T = k <= 256 * CH ? 64 : 256;                 // (uniform over the workgroup)
+  const int t = threadIdx.x & (T - 1), row = ((int)blockIdx.x - e.first) * (256 / T) + threadIdx.x / T;
+  if (row >= e.n) return;                                          // (a whole wave, or with T = 256 never)
   const float* src = e.w + (int64_t)row * k;
   f32x4 v[CH];
+#pragma unroll
+  for (int i = 0; i < CH; ++i) {
+    const int c = (t + i * T) * 4;
+    v[i] = c < k ? *reinterpret_cast<const f32x4*>(src + c) : f32x4{};
+  }
+  const auto max_bits = [&](uint32_t m) { return T == 64 ? wave_max_bits(m) : block_max_bits(m, tmp); };
+  const auto sum = [&](float x) { return T == 64 ? row_sum<64>(x, tmp) : row_sum<256>(x, tmp); };
   uint32_t mb = 0;
-  float norm = 0.f, dot = 0.f;
 #pragma unroll
-  for (int i = 0; i < CH; ++i) {
-    const int c = (lane + i * 64) * 4;
-    if (c < k) v[i] = *reinterpret_cast<const f32x4*>(src + c);
-  }
+  for (int i = 0; i < CH; ++i)
 #pragma unroll
-  for (int i = 0; i < CH; ++i) {
-    const int c = (lane + i * 64) * 4;
-    if (c >= k) break;
-    const f32x4 one = {1.f, 1.f, 1.f, 1.f}, zero = {0.f, 0.f, 0.f, 0.f};
-    const f32x4 g = e.gamma ? *reinterpret_cast<const f32x4*>(e.gamma + c % e.ln_cols) : one;
-    const f32x4 b = e.beta ? *reinterpret_cast<const f32x4*>(e.beta + c % e.ln_cols) : zero;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      mb = max(mb, __float_as_uint(v[i][j]) & 0x7fffffffu);
-      norm = fmaf(g[j] * v[i][j], g[j] * v[i][j], norm);
-      dot = fmaf(b[j], v[i][j], dot);
-    }
-  }
-  mb = wave_max_bits(mb);
-  norm = row_sum<64>(norm, nullptr);
-  dot = row_sum<64>(dot, nullptr);
+    for (int j = 0; j < 4; ++j) mb = max(mb, __float_as_uint(v[i][j]) & 0x7fffffffu);
+  mb = max_bits(mb);
   const float s = split_scale(__uint_as_float(mb));
   f16* dst = e.out + (int64_t)row * 2 * k;
 #pragma unroll
   for (int i = 0; i < CH; ++i) {
-    const int c = (lane + i * 64) * 4;
+    const int c = (t + i * T) * 4;
     if (c >= k) break;
     f16x4 hi, lo;
     split4(v[i], s, hi, lo);
     store_split4(dst, c, hi, lo);
   }
-  if (lane == 0) {
-    e.inv[row] = mb < 0x7f800000u ? 1.0f / s : __uint_as_float(0x7fc00000u);
-    e.row_bound[row] = 1.001f * sqrtf(norm * (float)k) + fabsf(dot) + fabsf(e.bias[row]);
+  if (t == 0) e.inv[row] = mb < 0x7f800000u ? 1.0f / s : __uint_as_float(0x7fc00000u);
+  if (!e.row_bound) return;
+  uint32_t gb = 0;                                                 // the bits of max |gamma w|
+  float norm = 0.f, dot = 0.f;
+#pragma unroll
+  for (int i = 0; i < CH; ++i) {
+    const int c = (t + i * T) * 4;
+    if (c >= k) break;
+    int lc = c;
+    while (e.gamma && lc >= e.ln_cols) lc -= e.ln_cols;
+    const f32x4 g = e.gamma ? *reinterpret_cast<const f32x4*>(e.gamma + lc) : f32x4{1.f, 1.f, 1.f, 1.f};
+    const f32x4 b = e.beta ? *reinterpret_cast<const f32x4*>(e.beta + lc) : f32x4{};
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      dot = fmaf(b[j], v[i][j], dot);
+      v[i][j] *= g[j];
+      gb = max(gb, __float_as_uint(v[i][j]) & 0x7fffffffu);
+    }
   }
+  // (the squares are taken of multiples of up to 2^15: neither weights of 1e-25 nor of 1e25 leave the range)
+  const float gs = split_scale(__uint_as_float(max_bits(gb)));
+#pragma unroll
+  for (int i = 0; i < CH; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) norm = fmaf(v[i][j] * gs, v[i][j] * gs, norm);
+  norm = sum(norm);
+  dot = sum(dot);
+  if (t == 0) e.row_bound[row] = 1.001f * sqrtf(norm * (float)k) / gs + fabsf(dot) + fabsf(e.bias[row]);
 }
 
 // out = the largest of the n values of v (>= 0 or NaN, which wins). (An atomic maximum per row on one address took the
@@ -186,15 +203,15 @@ __global__ __launch_bounds__(256) void group_max_kernel(GroupMaxes g) {
 
 int split_weights(SplitWeights p, hipStream_t stream) {
   int k = 0, blocks = 0;
+  for (int i = 0; i < p.count; ++i) k = std::max(k, p.e[i].k);
+  const int ch = k <= 4096 ? 4 : k <= 5120 ? 5 : 8;
   for (int i = 0; i < p.count; ++i) {
     p.e[i].first = blocks;
-    blocks += (p.e[i].n + 3) / 4;
-    k = std::max(k, p.e[i].k);
+    blocks += p.e[i].k <= 256 * ch ? (p.e[i].n + 3) / 4 : p.e[i].n;
   }
-  if (k <= 1024) hipLaunchKernelGGL(split_weights_kernel<4>, dim3(blocks), dim3(256), 0, stream, p);
-  else if (k <= 4096) hipLaunchKernelGGL(split_weights_kernel<16>, dim3(blocks), dim3(256), 0, stream, p);
-  else if (k <= 5120) hipLaunchKernelGGL(split_weights_kernel<20>, dim3(blocks), dim3(256), 0, stream, p);
-  else hipLaunchKernelGGL(split_weights_kernel<32>, dim3(blocks), dim3(256), 0, stream, p);
+  if (ch == 4) hipLaunchKernelGGL(split_weights_kernel<4>, dim3(blocks), dim3(256), 0, stream, p);
+  else if (ch == 5) hipLaunchKernelGGL(split_weights_kernel<5>, dim3(blocks), dim3(256), 0, stream, p);
+  else hipLaunchKernelGGL(split_weights_kernel<8>, dim3(blocks), dim3(256), 0, stream, p);
   return check_launch("split_weights");
 }
 

@@ -630,6 +630,7 @@ static int split_dense(hipStream_t st, const qvl_split_dense& d, const SplitDens
 // bounds of the Dense layers after a LayerNorm (`groups` of rows each, 0: no LayerNorm) are left to `gm`.
 struct SplitScratch {
   char *rows, *inv, *bound;
+  bool all = false;                 // row bounds of the others too
   SplitWeights p{};
   GroupMaxes gm{};
 
@@ -638,11 +639,11 @@ struct SplitScratch {
     SplitWeight& e = p.e[p.count++];
     e.w = (const float*)w; e.bias = bias; e.gamma = gamma; e.beta = beta; e.ln_cols = (int)ln_cols;
     e.n = (int)n; e.k = (int)k;
-    e.out = (_Float16*)rows; e.inv = (float*)inv; e.row_bound = (float*)bound;
+    e.out = (_Float16*)rows; e.inv = (float*)inv; e.row_bound = groups || all ? (float*)bound : nullptr;
     rows += n * k * 4;
     inv += n * 4;
-    bound += n * 4;
-    const qvl_split_dense d = {e.out, e.inv, (float*)bound};
+    bound += groups || all ? n * 4 : 0;
+    const qvl_split_dense d = {e.out, e.inv, groups ? (float*)bound : nullptr};
     for (int g = 0; g < groups; ++g, bound += 4) {
       gm.v[gm.count] = e.row_bound + n / groups * g;
       gm.n[gm.count] = (int)(n / groups);
@@ -666,10 +667,10 @@ static SplitScratchLayout split_scratch_layout(const qvl_vision_config* c) {
   return l;
 }
 
-static SplitScratch split_scratch(const qvl_vision_config* c, void* base) {
+static SplitScratch split_scratch(const qvl_vision_config* c, void* base, bool all = false) {
   const SplitScratchLayout l = split_scratch_layout(c);
   char* b = (char*)base;
-  return SplitScratch{b, b + l.rows, b + l.rows + 4 * l.n};
+  return SplitScratch{b, b + l.rows, b + l.rows + 4 * l.n, all};
 }
 
 static qvl_split_block add_block(SplitScratch& s, const TowerLayout& L, const qvl_block_weights& B) {
@@ -1116,16 +1117,16 @@ int qvl_vision_split_bounds(void* stream, const qvl_vision_config* c, const qvl_
     return group_maxes(g, st);
   };
   for (int i = 0; i < c->depth; ++i, bounds += 4) {
-    SplitScratch s = split_scratch(c, scratch);
+    SplitScratch s = split_scratch(c, scratch, true);
     add_block(s, L, W->blocks[i]);
     QVL_TRY_RC(layer(s, bounds));
   }
   for (int j = -1; j < c->n_deepstack; ++j, bounds += 2) {
-    SplitScratch s = split_scratch(c, scratch);
+    SplitScratch s = split_scratch(c, scratch, true);
     add_merger(s, c, L, j < 0 ? W->merger : W->deepstack[j], j >= 0);
     QVL_TRY_RC(layer(s, bounds));
   }
-  SplitScratch s = split_scratch(c, scratch);
+  SplitScratch s = split_scratch(c, scratch, true);
   s.add(W->patch_w, W->patch_b, nullptr, nullptr, 0, L.D, L.PVp, 0);
   return layer(s, bounds);
 }

@@ -350,3 +350,32 @@ def test_weights_split_beforehand_give_the_same_bits(pkg, lib, shape):
                                          C.byref(split), C.byref(t.metadata(grids)[2]), px.data_ptr(), got[0].data_ptr(),
                                          (C.c_void_p * 1)(got[1].data_ptr()), ws.data_ptr(), nb))
     assert same(got, want)
+
+
+@pytest.mark.parametrize("K", [64, 1024, 4352])
+def test_split_weight_bound_over_the_fp32_range(pkg, lib, K):
+    """Rows from 1e-36 to 1e33 (whose squares fp32 does not hold), no bias: the bound is the row's own."""
+    cp = pkg.capi
+    N = 128
+    g = torch.Generator(device=DEV).manual_seed(K)
+    w = torch.randn((N, K), generator=g, device=DEV).double() * 10.0 ** torch.linspace(-36, 33, N, device=DEV).double()[:, None]
+    w = w.float()
+    gamma, b = 1 + 0.1 * torch.randn(K, generator=g, device=DEV), torch.zeros(N, device=DEV)
+    beta = torch.zeros_like(gamma)
+    out, scale, bound = (torch.empty(n, device=DEV) for n in (N * K, N, 1 + N))
+    cp.check(lib.qvl_split_dense_weight(torch.cuda.current_stream().cuda_stream, w.data_ptr(), K, N, b.data_ptr(),
+                                        gamma.data_ptr(), beta.data_ptr(), K, 1, out.data_ptr(), scale.data_ptr(),
+                                        bound.data_ptr()))
+    want = K ** 0.5 * (gamma.double() * w.double()).norm(dim=1)
+    assert torch.all(bound[1:] >= want * 0.9999) and torch.all(bound[1:] <= want * 1.002)
+
+
+def test_split_tower_with_tiny_hidden_rows(pkg):
+    """fc1 weights of 1e-26 and fc2 weights of 1e25, no fc1 bias: the hidden rows keep their values."""
+    spec, params, px, grids = one_block(pkg)
+    mlp = params["visual"]["blocks_0"]["mlp"]
+    mlp["linear_fc1"]["kernel"] *= np.float32(1e-25)
+    mlp["linear_fc2"]["kernel"] *= np.float32(1e25)
+    a, b = tower_pair(pkg, spec, params)
+    for x, y in zip(outputs(a, px, grids), outputs(b, px, grids)):
+        assert torch.isfinite(x).all() and (x - y).norm() <= 1e-5 * y.norm()
