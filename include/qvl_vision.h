@@ -123,13 +123,19 @@ int qvl_dense(void* stream, int32_t dtype, int32_t epilogue, const void* d_x, in
 /* qvl_dense with a workspace for split-K: bf16, when the tiles do not fill whole rounds of the
  * GPU's compute units, the last round's tiles are split along K. The parts' fp32 partials go to
  * `d_workspace` and a second kernel sums them (in part order) before the epilogue: same results up
- * to fp32 summation order. fp32: where the workspace holds both operands again, each is written there
- * as two f16 terms per value with a power-of-two factor per row, and the Dense runs as three f16 MFMA
- * products into fp32 accumulators (nearer to float64 than the fp32 MFMA; rows or weights that hold
- * infinities or NaN get fp32 sums); else, when the 128 x 128 tiles of the fp32 MFMA kernel fill at
- * most half of the workgroup slots (two per compute unit), every tile is split along K into up to 8
- * parts. Without enough workspace it behaves exactly like qvl_dense.
- * qvl_dense_workspace_size gives the bytes that always suffice on the current device. */
+ * to fp32 summation order. fp32: where the workspace holds both operands again, 4 (m + n) k bytes beside the rows'
+ * factors, each is written there as two f16 terms per value with a power-of-two factor per row, and the Dense runs as
+ * three f16 MFMA products into fp32 accumulators. Values down to 2^-17 of their row's largest keep 22 bits and smaller
+ * ones an absolute error of 2^-39 of it, so |error| <= 2^-39 (max |x_m| sum |w_n| + max |w_n| sum |x_m|) comes on top of
+ * the fp32 sums'; rows of x or w that hold infinities or NaN, or more than a quarter of whose nonzero entries are below
+ * that line, get fp32 sums of the fp32 operands on the fp32 MFMA. With the rest the result is nearer to float64 than
+ * the fp32 MFMA's, whose chain of roundings is longer. Without a workspace (or by qvl_dense) every row runs on the
+ * fp32 MFMA. Where the workspace is smaller than that, and the 128 x 128 tiles of the fp32 MFMA kernel fill at most half
+ * of the workgroup slots (two per compute unit), every tile is split along K into up to 8 parts. Without enough
+ * workspace it behaves exactly like qvl_dense.
+ * qvl_dense_workspace_size gives the bytes that always suffice for split-K on the current device (64 MiB on 256
+ * compute units); fp32 operands larger than that together run on the fp32 MFMA unless the caller's workspace holds
+ * them. */
 int qvl_dense_workspace_size(size_t* bytes);
 int qvl_dense_ws(void* stream, int32_t dtype, int32_t epilogue, const void* d_x, int64_t lda,
                  const void* d_w, const float* d_bias, const void* d_residual, int64_t ldr,
@@ -426,7 +432,8 @@ typedef struct qvl_vision_split {
  * d_out_scale [n_out] fp32. d_out_bound [groups + n_out] fp32: the largest sqrt(k_in) |gamma w_n| +
  * |beta . w_n| + |bias_n| of each of `groups` equal groups of rows, then every row's; gamma / beta
  * [ln_cols] (a multiple of 4) repeat along the row (NULL: 1 / 0). A non-finite bound (weights that hold infinities or NaN, or
- * whose norms overflow) means the split must not be used. */
+ * whose norms overflow) means the split must not be used. Entries below 2^-17 of their row's largest keep an absolute
+ * error of 2^-39 of it and no more (qvl_dense_ws tells such rows apart; this split does not). */
 int qvl_split_dense_weight(void* stream, const float* d_w, int64_t k_in, int64_t n_out, const float* d_bias,
                            const float* d_gamma, const float* d_beta, int64_t ln_cols, int32_t groups,
                            void* d_out_w, float* d_out_scale, float* d_out_bound);
@@ -495,7 +502,7 @@ int qvl_encode_vision_split(void* stream, const qvl_vision_config* cfg, const qv
  * before the layer: nothing derived from the weights is kept between calls, so a forward, or a captured graph's
  * replay, reads the weights as they are when it runs. Beside qvl_encode_vision_workspace_size it takes
  * qvl_vision_split_scratch_size bytes of scratch (16-byte aligned; the largest layer's: 48 MB for a 1024-wide block).
- * A weight row that holds infinities or NaN gets fp32 sums. */
+ * Weight rows that qvl_dense_ws would run on the fp32 MFMA (infinities, NaN, too wide a range) do so here. */
 int qvl_vision_split_scratch_size(const qvl_vision_config* cfg, size_t* bytes);
 int qvl_encode_vision_split_scratch(void* stream, const qvl_vision_config* cfg, const qvl_vision_weights* weights,
                                     const qvl_vision_metadata_dev* meta, const float* d_pixel_values, void* d_tokens,

@@ -51,6 +51,48 @@ __device__ __forceinline__ uint32_t block_max_bits(uint32_t m, float* tmp) {
   return m;
 }
 
+// Which rows the split does not serve as well as fp32 does. An entry below 2^-17 of its row's largest has fewer than 22
+// bits left (an absolute error of 2^-39 of the largest): nothing beside the others' rounding where such entries are few,
+// but all there is where most of the row is that small and what multiplies its few large entries is zero. So a row
+// is wide, and its outputs are computed from the fp32 operands, where more than a quarter of its entries (zeros, which
+// have no error, aside) are below that line, or where it holds an infinity or a NaN. Normal values: an entry in 40000
+// is below it; under one entry 2^16 above the rest of them a row is wide.
+__device__ __forceinline__ uint32_t count_small(const f32x4& v, float s) {
+  uint32_t n = 0;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) n += (__float_as_uint(v[e] * s) & 0x7fffffffu) - 1u < 0x3e7fffffu;   // 0 < |v s| < 0.25
+  return n;
+}
+
+template <int T>
+__device__ __forceinline__ uint32_t row_count(uint32_t n, float* tmp) {
+#pragma unroll
+  for (int o = 32; o >= 1; o >>= 1) n += (uint32_t)__shfl_xor((int)n, o);
+  if constexpr (T > 64) {
+    __syncthreads();
+    if ((threadIdx.x & 63) == 0) tmp[threadIdx.x >> 6] = __uint_as_float(n);
+    __syncthreads();
+    n = 0;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) n += __float_as_uint(tmp[i]);
+  }
+  return n;
+}
+
+// mb: the bits of the row's maximum; small: this thread's count; v[CH]: this thread's entries, zeros past the row.
+template <int T, int CH>
+__device__ __forceinline__ bool row_is_wide(uint32_t mb, uint32_t small, const f32x4 (&v)[CH], float* tmp) {
+  if (T == 64 && !__builtin_amdgcn_ballot_w64(small != 0)) return mb >= 0x7f800000u;
+  small = row_count<T>(small, tmp);
+  if (small == 0 || mb >= 0x7f800000u) return mb >= 0x7f800000u;
+  uint32_t some = 0;
+#pragma unroll
+  for (int i = 0; i < CH; ++i)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) some += v[i][e] != 0.f;
+  return 4 * small > row_count<T>(some, tmp);
+}
+
 // ---------------------------------------------------------------------------------------------
 // fp32 rows -> split rows: a row's maximum, then its values scaled and split. Memory bound (each row read
 // and written once): T = 64 or 256 threads hold a row in registers, CH chunks of 4 values each, so that
@@ -61,7 +103,7 @@ struct SplitRowsParams {
   const float* src[2];
   int64_t ld[2];
   f16* dst[2];
-  float* inv[2];      // 2^-e of each row; NaN for a row that holds an infinity or a NaN
+  float* inv[2];      // 2^-e of each row; NaN for a row that goes by fp32 (row_is_wide)
   int rows[2];
   int K;
 };
@@ -91,6 +133,7 @@ __global__ __launch_bounds__(256) void split_rows_kernel(SplitRowsParams p) {
   else mb = wave_max_bits(mb);
   const float s = split_scale(__uint_as_float(mb));
   f16* dst = p.dst[which] + (int64_t)row * 2 * p.K;
+  uint32_t small = 0;
 #pragma unroll
   for (int i = 0; i < CH; ++i) {
     const int c = (t + i * T) * 4;
@@ -98,8 +141,10 @@ __global__ __launch_bounds__(256) void split_rows_kernel(SplitRowsParams p) {
     f16x4 hi, lo;
     split4(v[i], s, hi, lo);
     store_split4(dst, c, hi, lo);
+    small += count_small(v[i], s);
   }
-  if (t == 0) p.inv[which][row] = mb < 0x7f800000u ? 1.0f / s : __uint_as_float(0x7fc00000u);
+  const bool wide = row_is_wide<T>(mb, small, v, tmp);
+  if (t == 0) p.inv[which][row] = wide ? __uint_as_float(0x7fc00000u) : 1.0f / s;
 }
 
 static int split_rows(const SplitRowsParams& p, hipStream_t stream) {
@@ -149,6 +194,7 @@ __global__ __launch_bounds__(256) void split_weights_kernel(SplitWeights p) {
   mb = max_bits(mb);
   const float s = split_scale(__uint_as_float(mb));
   f16* dst = e.out + (int64_t)row * 2 * k;
+  uint32_t small = 0;
 #pragma unroll
   for (int i = 0; i < CH; ++i) {
     const int c = (t + i * T) * 4;
@@ -156,8 +202,10 @@ __global__ __launch_bounds__(256) void split_weights_kernel(SplitWeights p) {
     f16x4 hi, lo;
     split4(v[i], s, hi, lo);
     store_split4(dst, c, hi, lo);
+    small += count_small(v[i], s);
   }
-  if (t == 0) e.inv[row] = mb < 0x7f800000u ? 1.0f / s : __uint_as_float(0x7fc00000u);
+  const bool wide = T == 64 ? row_is_wide<64>(mb, small, v, tmp) : row_is_wide<256>(mb, small, v, tmp);
+  if (t == 0) e.inv[row] = wide && (p.mark_wide || mb >= 0x7f800000u) ? __uint_as_float(0x7fc00000u) : 1.0f / s;
   if (!e.row_bound) return;
   uint32_t gb = 0;                                                 // the bits of max |gamma w|
   float norm = 0.f, dot = 0.f;
@@ -355,26 +403,50 @@ __device__ __forceinline__ f32x4 split_unscale(f32x4 v, float sx, const f32x4& s
 
 __device__ __forceinline__ bool any_nan(const f32x4& v) { return v[0] != v[0] || v[1] != v[1] || v[2] != v[2] || v[3] != v[3]; }
 
-// Outputs of a row or column that holds infinities or NaN (its scale is NaN), as the fp32 operands give them (x from
-// its split rows where there is no other copy): serial fp32 sums, left at the first NaN. Rare, so written small and
-// not fast.
-template <int EPI, bool OUTS>
-__device__ __forceinline__ void split_serial4(const GemmSplitParams& p, int m, int n, const f32x4& bias) {
-  f32x4 v;
-#pragma unroll 1
-  for (int e = 0; e < 4; ++e) {
-    const float *x = p.xf + (int64_t)m * p.ldx, *w = p.wf + (int64_t)(n + e) * p.K;
-    const f16* xs = p.x + (int64_t)m * 2 * p.K;
-    const float fx = split_row_factor(p, m);
-    float a = 0.f;
-#pragma unroll 1
-    for (int k = 0; k < p.K && a == a; ++k) {
-      const int at = (k >> 5) * 64 + (k & 31);
-      a = fmaf(p.xf ? x[k] : ((float)xs[at] + (float)xs[at + 32]) * fx, w[k], a);
+// Whether outputs (m, n .. n + 3) come from the fp32 operands.
+__device__ __forceinline__ bool by_fp32(const GemmSplitParams& p, int m, int n) {
+  const float sx = split_row_factor(p, m);
+  return sx != sx || any_nan(*reinterpret_cast<const f32x4*>(p.sw + n));
+}
+
+// Rows of x and columns of w whose factor is NaN (row_is_wide): their outputs come from the fp32 operands, on
+// v_mfma_f32_32x32x2_f32, 32 tokens (from m1) x 32 features (from n1) of one wave at a time over k in [k0, k1), x from
+// its split rows where there is no fp32 copy. Lane l32 holds row l32 of both, hh the k's half of 8. Rare: no LDS, one
+// step of 32 k loaded ahead. Every row wide: 784 x 4096 x 1024 158 us (fp32 MFMA kernel 88), 4096 x 4096 x 1024 569 (300).
+__device__ __forceinline__ f32x16 split_fp32_block(const GemmSplitParams& p, int m1, int n1, int k0, int k1, int l32, int hh) {
+  const int m = min(m1 + l32, p.M - 1);
+  const float* w = p.wf + (int64_t)min(n1 + l32, p.N - 1) * p.K + 4 * hh;
+  const float* xf = p.xf ? p.xf + (int64_t)m * p.ldx + 4 * hh : nullptr;
+  const f16* xs = p.x + (int64_t)m * 2 * p.K + 4 * hh;
+  const float fx = split_row_factor(p, m);
+  struct Step { f32x4 w[4], x[4]; };
+  auto load = [&](int k, Step& s) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      s.w[i] = *reinterpret_cast<const f32x4*>(w + k + 8 * i);
+      if (xf) {
+        s.x[i] = *reinterpret_cast<const f32x4*>(xf + k + 8 * i);
+      } else {
+        const f16* g = xs + (k >> 5) * 64 + 8 * i;
+        const f16x4 hi = *reinterpret_cast<const f16x4*>(g), lo = *reinterpret_cast<const f16x4*>(g + 32);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) s.x[i][e] = ((float)hi[e] + (float)lo[e]) * fx;
+      }
     }
-    v[0] = e == 0 ? a : v[0]; v[1] = e == 1 ? a : v[1]; v[2] = e == 2 ? a : v[2]; v[3] = e == 3 ? a : v[3];
+  };
+  f32x16 acc = {};
+  Step cur, nxt;
+  load(k0, cur);
+#pragma unroll 1
+  for (int k = k0; k < k1; k += 32) {
+    if (k + 32 < k1) load(k + 32, nxt);
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(cur.w[i][e], cur.x[i][e], acc, 0, 0, 0);
+    cur = nxt;
   }
-  split_store4<EPI, OUTS>(p, m, n, v, bias);
+  return acc;
 }
 
 template <int BM, int BN, int WM, int WN, int NS, int EPI, bool OUTS>
@@ -412,6 +484,15 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_split_kernel(GemmSplitPa
   };
   const int KT = p.K / 32;
   const int kt0 = part_i * KT / p.split, kt1 = (part_i + 1) * KT / p.split;
+  // Whether a row or column of the wave's sub-tile goes by fp32: loaded here, where the products hide it.
+  const int mw = m0 + wm * S::TM, nw = n0 + wn * S::TN;
+  float marks = 0.f;
+#pragma unroll
+  for (int r = 0; r < S::TM; r += 64)
+    if (p.sx && r + lane < S::TM && mw + r + lane < p.M) marks += p.sx[mw + r + lane];
+#pragma unroll
+  for (int c = 0; c < S::TN; c += 64)
+    if (c + lane < S::TN && nw + c + lane < p.N) marks += p.sw[nw + c + lane];
 #pragma unroll
   for (int s = 0; s < NS - 1; ++s)
     if (kt0 + s < kt1) dma_stage(kt0 + s, s);
@@ -512,7 +593,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_split_kernel(GemmSplitPa
     sw = *reinterpret_cast<const f32x4*>(p.sw + n);
     bias = *reinterpret_cast<const f32x4*>(p.bias + n);
   }
-  const bool w_nan = any_nan(sw);
+  const bool w_nan = any_nan(sw), marked = __builtin_amdgcn_ballot_w64(marks != marks) != 0;
   const int64_t npad = (int64_t)tiles_n * BN;
 #pragma unroll
   for (int b = 0; b < S::MB; ++b) {
@@ -529,21 +610,35 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_split_kernel(GemmSplitPa
       const int r = i * RPI + lane / CH, m = m0 + wm * S::TM + 32 * b + r;
       const f32x4 v = *reinterpret_cast<const f32x4*>(stage + r * S::TN + ((c ^ (r % CH)) << 2));
       if (m >= p.M) continue;
-      if (p.split > 1)
-        *reinterpret_cast<f32x4*>(p.part + ((int64_t)part_i * p.M + m) * npad + n) = v;
-      else if (nok) {
+      if (p.split > 1) {
+        if (!marked || !nok || !by_fp32(p, m, n))
+          *reinterpret_cast<f32x4*>(p.part + ((int64_t)part_i * p.M + m) * npad + n) = v;
+      } else if (nok) {
         const float sx = split_row_factor(p, m);
         if (sx == sx && !w_nan) split_store4<EPI, OUTS>(p, m, n, split_unscale(v, sx, sw), bias);
       }
     }
   }
-  const bool rows_nan = p.sx && p.xf;          // (without the fp32 rows no factor is NaN)
-  if (p.split > 1 || !nok || !(w_nan || rows_nan)) return;
+  if (!marked) return;
 #pragma unroll 1
-  for (int r = lane / CH; r < S::TM; r += RPI) {
-    const int m = m0 + wm * S::TM + r;
-    if (m >= p.M) break;
-    if (w_nan || p.sx[m] != p.sx[m]) split_serial4<EPI, OUTS>(p, m, n, bias);   // (w_nan first: sx may be NULL)
+  for (int blk = 0; blk < S::NB * S::MB; ++blk) {
+    const int m1 = mw + 32 * (blk % S::MB), n1 = nw + 32 * (blk / S::MB);
+    const int at = hh ? n1 + l32 : m1 + l32;
+    const float mark = hh ? (at < p.N ? p.sw[at] : 0.f) : (at < p.M && p.sx ? p.sx[at] : 0.f);
+    if (!__builtin_amdgcn_ballot_w64(mark != mark)) continue;
+    const f32x16 v = split_fp32_block(p, m1, n1, kt0 * 32, kt1 * 32, l32, hh);
+#pragma unroll
+    for (int g = 0; g < 4; ++g)                       // (through LDS as above, 8 chunks of 4 features a row)
+      *reinterpret_cast<f32x4*>(stage + l32 * 32 + (((2 * g + hh) ^ (l32 & 7)) << 2)) =
+          f32x4{v[4 * g], v[4 * g + 1], v[4 * g + 2], v[4 * g + 3]};
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int r = 8 * i + (lane >> 3), m2 = m1 + r, n2 = n1 + 4 * (lane & 7);
+      const f32x4 o = *reinterpret_cast<const f32x4*>(stage + r * 32 + (((lane & 7) ^ (r & 7)) << 2));
+      if (m2 >= p.M || n2 >= p.N || !by_fp32(p, m2, n2)) continue;
+      if (p.split > 1) *reinterpret_cast<f32x4*>(p.part + ((int64_t)part_i * p.M + m2) * npad + n2) = o;
+      else split_store4<EPI, OUTS>(p, m2, n2, o, *reinterpret_cast<const f32x4*>(p.bias + n2));
+    }
   }
 }
 
@@ -559,8 +654,8 @@ __global__ __launch_bounds__(256) void gemm_split_reduce_kernel(GemmSplitParams 
   for (int s = 1; s < p.split; ++s) v += *reinterpret_cast<const f32x4*>(src + s * stride);
   const f32x4 sw = *reinterpret_cast<const f32x4*>(p.sw + n), bias = *reinterpret_cast<const f32x4*>(p.bias + n);
   const float sx = split_row_factor(p, m);
-  if (sx == sx && !any_nan(sw)) split_store4<EPI, OUTS>(p, m, n, split_unscale(v, sx, sw), bias);
-  else split_serial4<EPI, OUTS>(p, m, n, bias);
+  if (sx == sx && !any_nan(sw)) v = split_unscale(v, sx, sw);   // (else the parts are fp32 sums)
+  split_store4<EPI, OUTS>(p, m, n, v, bias);
 }
 
 template <int BM, int BN, int WM, int WN, int NS, int EPI, bool OUTS>

@@ -637,6 +637,7 @@ struct SplitScratch {
   qvl_split_dense add(const void* w, const float* bias, const float* gamma, const float* beta, int64_t ln_cols,
                       int64_t n, int64_t k, int groups) {
     SplitWeight& e = p.e[p.count++];
+    p.mark_wide = true;
     e.w = (const float*)w; e.bias = bias; e.gamma = gamma; e.beta = beta; e.ln_cols = (int)ln_cols;
     e.n = (int)n; e.k = (int)k;
     e.out = (_Float16*)rows; e.inv = (float*)inv; e.row_bound = groups || all ? (float*)bound : nullptr;

@@ -85,7 +85,7 @@ struct GemmF32Params {
 
 // fp32 Dense on two-way f16 split operands (qvl_f32_split.hip): x [M] and w [N] rows of K / 32 groups of
 // [32 hi | 32 lo] f16, sx / sw the rows' factors back to their fp32 values (NaN: a row that holds an infinity
-// or a NaN; its outputs are computed from xf [M, ldx] and wf [N, K] in fp32).
+// or a NaN, or too wide a range; its outputs are computed from xf [M, ldx] and wf [N, K] in fp32).
 struct GemmSplitParams {
   const _Float16* x; const float* sx;
   const _Float16* w; const float* sw;
@@ -109,7 +109,8 @@ struct SplitWeight {
   float *inv, *row_bound;
   int n, k, ln_cols, first;
 };
-struct SplitWeights { SplitWeight e[4]; int count; };
+// mark_wide: rows of too wide a range for the split get a NaN factor too, as those with infinities or NaN do.
+struct SplitWeights { SplitWeight e[4]; int count; bool mark_wide; };
 
 // out[i] = the largest of the n[i] values v[i] (>= 0, or NaN, which wins).
 struct GroupMaxes { const float* v[4]; float* out[4]; int n[4]; int count; };
@@ -167,7 +168,8 @@ int gemm_f32_split(const GemmF32Params& g, int epi, hipStream_t stream);
 int gemm_f32_set_plan(int tile);
 constexpr int kSplitMaxK = 8192;   // the longest row the split kernels hold
 int gemm_split(const GemmSplitParams& p, int epi, hipStream_t stream);
-// x [rows] (and, w_rows > 0, w) -> split rows; a row's factor is NaN where it holds an infinity or a NaN.
+// x [rows] (and, w_rows > 0, w) -> split rows; a row's factor is NaN where it holds an infinity or a NaN, or values of too
+// wide a range.
 int split_rows_f32(const float* x, int64_t ldx, void* out, float* inv, int rows, const float* w, void* w_out, float* w_inv,
                    int w_rows, int k, hipStream_t stream);
 int split_weights(SplitWeights p, hipStream_t stream);

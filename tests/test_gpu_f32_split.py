@@ -379,3 +379,40 @@ def test_split_tower_with_tiny_hidden_rows(pkg):
     a, b = tower_pair(pkg, spec, params)
     for x, y in zip(outputs(a, px, grids), outputs(b, px, grids)):
         assert torch.isfinite(x).all() and (x - y).norm() <= 1e-5 * y.norm()
+
+
+# One entry far above the rest of its row, a zero against it: what is left of the row decides the output. From 2^17 the
+# rows go by the fp32 operands; a third of them are left as they were. K with and without K parts, edges of the tiles.
+@pytest.mark.parametrize("M,N,K", [(70, 132, 128), (257, 260, 1024), (33, 64, 4352)])
+@pytest.mark.parametrize("side", ["x", "w"])
+def test_split_dense_outliers_within_a_row(dense, M, N, K, side):
+    for e in (8, 14, 16, 17, 18, 20, 24, 30, 40, 80):
+        x, w, b, r = operands(M, N, K, e)
+        a, other = (x, w) if side == "x" else (w, x)
+        a[:, 3] = torch.where(torch.arange(len(a), device=DEV) % 3 > 0, 2.0 ** e * a.std().item(), 1.0)
+        other[:, 3] = 0.0
+        b.zero_()
+        ref = x.double() @ w[:N].double().t()
+        tol = bound(x, w, N, K)
+        for plan in (0, 1, 2, 3, 4, 6):
+            for epi in (0, 2):
+                y = dense(plan, x, w, b, epi, r if epi else None).double() - (r.double() if epi else 0)
+                assert torch.all((y - ref).abs() <= tol + epi * (ref.abs() + r.abs().double()) * 2.0 ** -23), (e, plan, epi)
+        got, want = dense(0, x, w, b).double(), dense(5, x, w, b).double()
+        assert (got - ref).norm() <= 1.1 * (want - ref).norm(), e
+
+
+def test_split_dense_wide_rows_match_fp32(dense):
+    """Rows whose entries are spread over 60 powers of two, in either operand: no further from float64 than the fp32 MFMA
+    kernel, whatever the other operand picks out of them."""
+    M, N, K = 96, 192, 1024
+    for seed, side in ((1, "x"), (2, "w")):
+        x, w, b, _ = operands(M, N, K, seed)
+        (x if side == "x" else w).mul_(2.0 ** torch.linspace(-60, 0, K, device=DEV))
+        b.zero_()
+        for k in (200, 600, 1000):                          # the other one reads the first k entries alone
+            x1, w1 = x.clone(), w.clone()
+            (w1 if side == "x" else x1)[:, k:] = 0.0
+            ref = x1.double() @ w1[:N].double().t()
+            err = [(dense(plan, x1, w1, b).double() - ref).norm() / ref.norm() for plan in (0, 1, 2, 3, 4, 6, 5)]
+            assert max(err[:-1]) <= 1.1 * err[-1] + 1e-8, (side, k, err)
