@@ -509,10 +509,13 @@ int qvl_encode_vision_split_scratch(void* stream, const qvl_vision_config* cfg, 
                                     void* const* d_deepstack, void* d_workspace, size_t workspace_bytes,
                                     void* d_scratch, size_t scratch_bytes);
 
-/* The largest output bound (qvl_split_dense_weight) of every Dense of the tower: d_bounds [4 * depth + 2 * (1 +
- * n_deepstack) + 1] fp32, qkv, proj, fc1, fc2 of each block, fc1, fc2 of the merger and of each deepstack merger, the
- * patch embed. A non-finite one: that layer's weights hold infinities or NaN, or their norms overflow, and the tower
- * is better run by qvl_encode_vision. */
+/* The largest output bounds (qvl_split_dense_weight) of every Dense of the tower: d_bounds [6 * depth + 2 * (1 +
+ * n_deepstack) + 1] fp32: q, k, v, proj, fc1, fc2 of each block, fc1, fc2 of the merger and of each deepstack merger,
+ * the patch embed. q, k, v and the hidden rows are split by one exponent a layer, from these bounds, with an absolute error
+ * of 2^-39 of them. A non-finite one: that layer's weights hold infinities or NaN, their norms overflow, or (q, k, v and
+ * fc1) more than a quarter of the nonzero rows have bounds below 2^-9 of the largest, too far apart for one exponent.
+ * The tower is then better run by qvl_encode_vision; the split forward stays right for the hidden rows (they go by fp32,
+ * slowly) and loses bits of the smaller q, k and v. */
 int qvl_vision_split_bounds(void* stream, const qvl_vision_config* cfg, const qvl_vision_weights* weights,
                             void* d_scratch, size_t scratch_bytes, float* d_bounds);
 

@@ -235,18 +235,41 @@ __global__ __launch_bounds__(256) void split_weights_kernel(SplitWeights p) {
   if (t == 0) e.row_bound[row] = 1.001f * sqrtf(norm * (float)k) / gs + fabsf(dot) + fabsf(e.bias[row]);
 }
 
-// out = the largest of the n values of v (>= 0 or NaN, which wins). (An atomic maximum per row on one address took the
-// launch above from 10 to 45 us.)
-__device__ __forceinline__ void group_max(const float* __restrict__ v, int n, float* __restrict__ out, float* tmp) {
-  uint32_t mb = 0;
-  for (int i = threadIdx.x; i < n; i += 256) mb = max(mb, __float_as_uint(v[i]) & 0x7fffffffu);
+// One exponent for all outputs of a Dense suits them while their bounds are alike: an output's absolute error is 2^-39 of
+// the largest bound, and the outputs themselves are some 2^-5 of theirs, so bounds down to 2^-9 of the largest keep fp32's
+// 24 bits. kGroupAlike: NaN where more than a quarter of them (zeros aside) are lower, or one is not finite: the Dense
+// then writes fp32 rows in place of split rows, and its reader takes them as such. (An atomic maximum per row on one
+// address took the launch above from 10 to 45 us.)
+// (kGroupAlike: n at most 8192.)
+__device__ __forceinline__ void group_max(const float* __restrict__ v, int n, int kind, float* __restrict__ out, float* tmp) {
+  constexpr int CH = 32;
+  uint32_t u[CH], mb = 0;
+  for (int base = 0; base < n; base += 256 * CH) {           // (once, unless n > 8192)
+#pragma unroll
+    for (int i = 0; i < CH; ++i) {
+      const int at = base + 256 * i + threadIdx.x;
+      u[i] = at < n ? __float_as_uint(v[at]) & 0x7fffffffu : 0;
+    }
+#pragma unroll
+    for (int i = 0; i < CH; ++i) mb = max(mb, u[i]);
+  }
   mb = block_max_bits(mb, tmp);
+  if (kind == kGroupInf) mb = min(mb, 0x7f800000u);
+  if (kind == kGroupAlike && mb >= 0x7f800000u) mb = 0x7fc00000u;
+  if (kind == kGroupAlike && mb < 0x7f800000u) {
+    const uint32_t low = __float_as_uint(__uint_as_float(mb) * 0x1p-9f);
+    uint32_t count = 0;                                      // lower ones, and 2^16 x those not zero
+#pragma unroll
+    for (int i = 0; i < CH; ++i) count += (u[i] ? 0x10000u : 0u) + (u[i] && u[i] < low ? 1u : 0u);
+    count = row_count<256>(count, tmp);
+    if (4 * (count & 0xffffu) > (count >> 16)) mb = 0x7fc00000u;
+  }
   if (threadIdx.x == 0) *out = __uint_as_float(mb);
 }
 
 __global__ __launch_bounds__(256) void group_max_kernel(GroupMaxes g) {
   __shared__ float tmp[4];
-  group_max(g.v[blockIdx.x], g.n[blockIdx.x], g.out[blockIdx.x], tmp);
+  group_max(g.v[blockIdx.x], g.n[blockIdx.x], g.kind[blockIdx.x], g.out[blockIdx.x], tmp);
 }
 
 int split_weights(SplitWeights p, hipStream_t stream) {
@@ -272,6 +295,7 @@ int group_maxes(const GroupMaxes& g, hipStream_t stream) {
 // LayerNorm fp32 (the arithmetic of layernorm_f32_kernel) written as split rows for the Dense that reads it:
 // no fp32 copy of the normalised rows, and no pass to split them. T threads hold a row; MERGE: the 4 waves of a
 // workgroup normalise 4 consecutive rows that form one row of the output (the 2x2 merge), with one exponent.
+// A row that is wide (row_is_wide) is written as it is, fp32, with a NaN factor.
 // Workgroups past the rows take the maxima of `gm` (a layer's output bounds, needed by the launches after this one).
 // ---------------------------------------------------------------------------------------------
 template <int T, int CH, bool MERGE>
@@ -284,7 +308,7 @@ __global__ __launch_bounds__(256) void layernorm_split_kernel(const float* __res
   const int first_max = gridDim.x - gm.count;         // the last workgroups: the layer's output bounds
   if ((int)blockIdx.x >= first_max) {
     const int g = blockIdx.x - first_max;
-    return group_max(gm.v[g], gm.n[g], gm.out[g], tmp);
+    return group_max(gm.v[g], gm.n[g], gm.kind[g], gm.out[g], tmp);
   }
   const int t = threadIdx.x % T, row = blockIdx.x * (256 / T) + threadIdx.x / T;
   if (row >= rows) return;                            // (MERGE: rows % 4 == 0, all waves or none)
@@ -321,18 +345,26 @@ __global__ __launch_bounds__(256) void layernorm_split_kernel(const float* __res
   }
   if constexpr (T > 64 || MERGE) mb = block_max_bits(mb, tmp);
   else mb = wave_max_bits(mb);
-  const float sc = split_scale(__uint_as_float(mb));   // (a NaN row stays NaN in its hi terms)
+  const float sc = split_scale(__uint_as_float(mb));
+  uint32_t small = 0;
+#pragma unroll
+  for (int i = 0; i < CH; ++i) small += count_small(v[i], sc);
+  const bool wide = row_is_wide<MERGE ? 256 : T>(mb, small, v, tmp);
   const int orow = MERGE ? row / 4 : row, ocol = MERGE ? (row & 3) * cols : 0;
   f16* dst = y + (int64_t)orow * 2 * (MERGE ? 4 * cols : cols);
 #pragma unroll
   for (int i = 0; i < CH; ++i) {
     const int c = (t + T * i) * 4;
     if (c >= cols) break;
+    if (wide) {
+      *reinterpret_cast<f32x4*>(reinterpret_cast<float*>(dst) + ocol + c) = v[i];
+      continue;
+    }
     f16x4 hi, lo;
     split4(v[i], sc, hi, lo);
     store_split4(dst, ocol + c, hi, lo);
   }
-  if (t == 0 && (!MERGE || (row & 3) == 0)) inv[orow] = 1.0f / sc;
+  if (t == 0 && (!MERGE || (row & 3) == 0)) inv[orow] = wide ? __uint_as_float(0x7fc00000u) : 1.0f / sc;
 }
 
 // cols a multiple of 64 (32-column groups), at most kSplitMaxK; merge: rows % 4 == 0, cols <= 2048.
@@ -380,17 +412,24 @@ __device__ __forceinline__ void split_store4(const GemmSplitParams& p, int m, in
   }
   if constexpr (EPI == kEpiBiasResidual) v += *reinterpret_cast<const f32x4*>(p.res + (int64_t)m * p.ldr + n);
   if constexpr (OUTS) {
+    const float bound = *p.ybound;
+    if (bound != bound) {                                // (kGroupAlike: fp32 rows)
+      *reinterpret_cast<f32x4*>(reinterpret_cast<float*>(p.ys) + (int64_t)m * p.N + n) = v;
+      return;
+    }
     f16x4 hi, lo;
-    split4(v, split_scale(*p.ybound), hi, lo);
+    split4(v, split_scale(bound), hi, lo);
     store_split4(p.ys + (int64_t)m * 2 * p.N, n, hi, lo);
   } else {
     *reinterpret_cast<f32x4*>(p.y + (int64_t)m * p.ldc + n) = v;
   }
 }
 
-// The factor of row m of x: its own, or one for every row from a bound on |x|.
+// The factor of row m of x: its own, or one for every row from a bound on |x|. NaN: the row goes by fp32.
 __device__ __forceinline__ float split_row_factor(const GemmSplitParams& p, int m) {
-  return p.sx ? p.sx[m] : 1.0f / split_scale(*p.xbound);
+  if (p.sx) return p.sx[m];
+  const float b = *p.xbound;
+  return b == b ? 1.0f / split_scale(b) : b;
 }
 
 // acc 2^-(ex + ew): the smaller factor first, so that neither step leaves the range unless the result does
@@ -410,15 +449,16 @@ __device__ __forceinline__ bool by_fp32(const GemmSplitParams& p, int m, int n) 
 }
 
 // Rows of x and columns of w whose factor is NaN (row_is_wide): their outputs come from the fp32 operands, on
-// v_mfma_f32_32x32x2_f32, 32 tokens (from m1) x 32 features (from n1) of one wave at a time over k in [k0, k1), x from
-// its split rows where there is no fp32 copy. Lane l32 holds row l32 of both, hh the k's half of 8. Rare: no LDS, one
+// v_mfma_f32_32x32x2_f32, 32 tokens (from m1) x 32 features (from n1) of one wave at a time over k in [k0, k1). x comes from
+// xf, or without it from p.x: a row with a NaN factor lies there as fp32, any other as a split row. Lane l32 holds row l32 of both, hh the k's half of 8. Rare: no LDS, one
 // step of 32 k loaded ahead. Every row wide: 784 x 4096 x 1024 158 us (fp32 MFMA kernel 88), 4096 x 4096 x 1024 569 (300).
 __device__ __forceinline__ f32x16 split_fp32_block(const GemmSplitParams& p, int m1, int n1, int k0, int k1, int l32, int hh) {
   const int m = min(m1 + l32, p.M - 1);
   const float* w = p.wf + (int64_t)min(n1 + l32, p.N - 1) * p.K + 4 * hh;
-  const float* xf = p.xf ? p.xf + (int64_t)m * p.ldx + 4 * hh : nullptr;
-  const f16* xs = p.x + (int64_t)m * 2 * p.K + 4 * hh;
   const float fx = split_row_factor(p, m);
+  const float* xf = p.xf ? p.xf + (int64_t)m * p.ldx + 4 * hh
+                         : fx != fx ? reinterpret_cast<const float*>(p.x) + (int64_t)m * p.K + 4 * hh : nullptr;
+  const f16* xs = p.x + (int64_t)m * 2 * p.K + 4 * hh;
   struct Step { f32x4 w[4], x[4]; };
   auto load = [&](int k, Step& s) {
 #pragma unroll
@@ -486,7 +526,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_split_kernel(GemmSplitPa
   const int kt0 = part_i * KT / p.split, kt1 = (part_i + 1) * KT / p.split;
   // Whether a row or column of the wave's sub-tile goes by fp32: loaded here, where the products hide it.
   const int mw = m0 + wm * S::TM, nw = n0 + wn * S::TN;
-  float marks = 0.f;
+  float marks = p.sx ? 0.f : *p.xbound;
 #pragma unroll
   for (int r = 0; r < S::TM; r += 64)
     if (p.sx && r + lane < S::TM && mw + r + lane < p.M) marks += p.sx[mw + r + lane];
@@ -624,7 +664,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_split_kernel(GemmSplitPa
   for (int blk = 0; blk < S::NB * S::MB; ++blk) {
     const int m1 = mw + 32 * (blk % S::MB), n1 = nw + 32 * (blk / S::MB);
     const int at = hh ? n1 + l32 : m1 + l32;
-    const float mark = hh ? (at < p.N ? p.sw[at] : 0.f) : (at < p.M && p.sx ? p.sx[at] : 0.f);
+    const float mark = hh ? (at < p.N ? p.sw[at] : 0.f) : (at < p.M ? split_row_factor(p, at) : 0.f);
     if (!__builtin_amdgcn_ballot_w64(mark != mark)) continue;
     const f32x16 v = split_fp32_block(p, m1, n1, kt0 * 32, kt1 * 32, l32, hh);
 #pragma unroll

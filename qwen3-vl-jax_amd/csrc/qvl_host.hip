@@ -648,6 +648,7 @@ struct SplitScratch {
     for (int g = 0; g < groups; ++g, bound += 4) {
       gm.v[gm.count] = e.row_bound + n / groups * g;
       gm.n[gm.count] = (int)(n / groups);
+      gm.kind[gm.count] = groups == 1 ? kGroupAlike : kGroupInf;   // (the attention has no fp32 form of q, k and v)
       gm.out[gm.count++] = (float*)bound;
     }
     bound += 4 * ((4 - groups % 4) % 4);
@@ -1110,14 +1111,18 @@ int qvl_vision_split_bounds(void* stream, const qvl_vision_config* c, const qvl_
     QVL_TRY_RC(split_weights(s.p, st));
     GroupMaxes g{};
     for (int i = 0; i < s.p.count; ++i) {
-      g.v[i] = s.p.e[i].row_bound;
-      g.n[i] = s.p.e[i].n;
-      g.out[i] = out + i;
+      const SplitWeight& e = s.p.e[i];
+      const int groups = s.p.count == 4 && i == 0 ? 3 : 1;      // (a block's q, k and v)
+      for (int j = 0; j < groups; ++j, ++g.count) {
+        g.v[g.count] = e.row_bound + e.n / groups * j;
+        g.n[g.count] = e.n / groups;
+        g.kind[g.count] = e.gamma ? kGroupAlike : kGroupMax;
+        g.out[g.count] = out + g.count;
+      }
     }
-    g.count = s.p.count;
     return group_maxes(g, st);
   };
-  for (int i = 0; i < c->depth; ++i, bounds += 4) {
+  for (int i = 0; i < c->depth; ++i, bounds += 6) {
     SplitScratch s = split_scratch(c, scratch, true);
     add_block(s, L, W->blocks[i]);
     QVL_TRY_RC(layer(s, bounds));

@@ -85,7 +85,7 @@ struct GemmF32Params {
 
 // fp32 Dense on two-way f16 split operands (qvl_f32_split.hip): x [M] and w [N] rows of K / 32 groups of
 // [32 hi | 32 lo] f16, sx / sw the rows' factors back to their fp32 values (NaN: a row that holds an infinity
-// or a NaN, or too wide a range; its outputs are computed from xf [M, ldx] and wf [N, K] in fp32).
+// or a NaN, or too wide a range; its outputs are computed in fp32 from wf [N, K] and xf [M, ldx], or without xf the row in x).
 struct GemmSplitParams {
   const _Float16* x; const float* sx;
   const _Float16* w; const float* sw;
@@ -94,9 +94,9 @@ struct GemmSplitParams {
   float* y; int64_t ldc;
   int M, N, K;
   const float* xf; int64_t ldx; const float* wf;
-  const float* xbound;             // sx NULL: every row of x carries the exponent of *xbound >= max |x|
+  const float* xbound;             // sx NULL: every row of x carries the exponent of *xbound >= max |x|, or (NaN) is fp32
   _Float16* ys;                    // GELU only, instead of y: the outputs [M, N] as split rows with the
-  const float* ybound;             // exponent of *ybound >= max |y|
+  const float* ybound;             // exponent of *ybound >= max |y|, or (NaN) as fp32 rows
   float* part; int64_t part_elems; // split-K partials (set up by the launcher, as in GemmF32Params)
   int split, group_n;
 };
@@ -112,8 +112,10 @@ struct SplitWeight {
 // mark_wide: rows of too wide a range for the split get a NaN factor too, as those with infinities or NaN do.
 struct SplitWeights { SplitWeight e[4]; int count; bool mark_wide; };
 
-// out[i] = the largest of the n[i] values v[i] (>= 0, or NaN, which wins).
-struct GroupMaxes { const float* v[4]; float* out[4]; int n[4]; int count; };
+// out[i] = the largest of the n[i] values v[i] (>= 0, or NaN, which wins; kGroupInf: an infinity in place of NaN;
+// kGroupAlike: NaN too where an exponent for the largest does not suit the others, or where one is infinite).
+enum { kGroupMax = 0, kGroupInf = 1, kGroupAlike = 2 };
+struct GroupMaxes { const float* v[6]; float* out[6]; int n[6], kind[6]; int count; };
 
 // Floats of split-K partial workspace that lets every GEMM of up to 256x256 tiles split its tail
 // on a device with `cus` compute units (one tail unit per CU, at most one tile of partials each).

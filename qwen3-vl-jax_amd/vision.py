@@ -486,15 +486,15 @@ class Qwen3VisionTransformer:
     def _split_scratch(self):
         """fp32: the device buffer each layer's Dense weights are split into, on the stream before the layer, so that
         its Dense runs on the f16 matrix cores (qvl_encode_vision_split_scratch); or None where the widths or the
-        weights' values rule it out (non-finite weights, or norms that overflow): the forward then splits or not per
-        Dense, as qvl_dense_ws does. No forward keeps anything derived from the weights."""
+        weights' values rule it out (non-finite weights, norms that overflow, rows of a layer too far apart for the one
+        exponent of its outputs): the forward then splits or not per Dense, as qvl_dense_ws does. No forward keeps anything derived from the weights."""
         torch = _torch()
         s = self.spec
         nb = C.c_size_t()
         if self._lib.qvl_vision_split_scratch_size(C.byref(self._cfg), C.byref(nb)) != 0:
             return None
         buf = torch.empty(nb.value, dtype=torch.uint8, device=self.device)
-        bounds = torch.empty(4 * s.depth + 2 * (1 + len(s.deepstack_visual_indexes)) + 1, dtype=torch.float32,
+        bounds = torch.empty(6 * s.depth + 2 * (1 + len(s.deepstack_visual_indexes)) + 1, dtype=torch.float32,
                              device=self.device)
         capi.check(self._lib.qvl_vision_split_bounds(self._stream(), C.byref(self._cfg), C.byref(self._w),
                                                      buf.data_ptr(), nb.value, bounds.data_ptr()),

@@ -416,3 +416,51 @@ def test_split_dense_wide_rows_match_fp32(dense):
             ref = x1.double() @ w1[:N].double().t()
             err = [(dense(plan, x1, w1, b).double() - ref).norm() / ref.norm() for plan in (0, 1, 2, 3, 4, 6, 5)]
             assert max(err[:-1]) <= 1.1 * err[-1] + 1e-8, (side, k, err)
+
+
+@pytest.mark.parametrize("where", ["fc1", "deepstack"])
+def test_split_tower_with_an_outlier_among_the_hidden_rows(pkg, where):
+    """One fc1 row 2^16 above the others and a zero fc2 column against it: the others' exponent is not the outlier's. A
+    tower bound to such weights is not split; one that they were written to afterwards keeps fp32 hidden rows."""
+    spec, params, px, grids = one_block(pkg)
+    t = pkg.Qwen3VisionTransformer(spec).bind(params)
+    st = t.packed_state()
+    pre = "blocks.0." if where == "fc1" else "deepstack.0."
+    st[pre + "fc1.w"][5] *= 2.0 ** 16
+    st[pre + "fc2.w"][:, 5] = 0.0
+    b = pkg.Qwen3VisionTransformer(spec).bind_packed(st)
+    assert t._split is not None and b._split is None
+    for got, want in zip(outputs(t, px, grids), outputs(b, px, grids)):
+        assert torch.isfinite(got).all() and (got - want).norm() <= 3e-6 * want.norm()
+
+
+@pytest.mark.parametrize("part", [0, 1, 2])
+def test_outliers_among_q_k_v_leave_the_tower_unsplit(pkg, part):
+    spec, params, px, grids = one_block(pkg)
+    w = params["visual"]["blocks_0"]["attn"]["qkv"]["kernel"]
+    w[:, part * spec.hidden_size + 7] *= np.float32(2.0 ** 12)
+    assert pkg.Qwen3VisionTransformer(spec).bind(params)._split is None
+    w[:, part * spec.hidden_size + 7] *= np.float32(2.0 ** -8)          # 2^4 above the others: ordinary
+    assert pkg.Qwen3VisionTransformer(spec).bind(params)._split is not None
+
+
+@pytest.mark.parametrize("cols", [1024, 1152])
+def test_split_tower_with_wide_normalised_rows(pkg, lib, cols):
+    """Two entries of opposite sign 2^22 above the rest of a token (their sum does not lift the others) and zero weights
+    against them: the normalised row goes by fp32. The pixel rows are such tokens through an identity patch embed."""
+    spec, params, px, grids = one_block(pkg)
+    if cols == 1152:
+        spec = pkg.spec_8b()
+        spec.depth, spec.deepstack_visual_indexes = 1, (0,)
+        params = pkg.random_params(spec, seed=2)
+    v = params["visual"]
+    v["patch_embed"]["proj"]["kernel"][:] = 0
+    for i in range(cols):
+        v["patch_embed"]["proj"]["kernel"][i, i] = 1.0
+    v["pos_embed"]["embedding"][:] = 0
+    px[::2, 3], px[::2, 9] = 2.0 ** 22, -2.0 ** 22
+    for k in (v["blocks_0"]["attn"]["qkv"]["kernel"], v["blocks_0"]["mlp"]["linear_fc1"]["kernel"]):
+        k[3], k[9] = 0, 0
+    a, b = tower_pair(pkg, spec, params)
+    for got, want in zip(outputs(a, px, grids), outputs(b, px, grids)):
+        assert torch.isfinite(got).all() and (got - want).norm() <= 3e-6 * want.norm()
