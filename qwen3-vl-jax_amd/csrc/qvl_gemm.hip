@@ -1569,10 +1569,11 @@ static int dispatch_gemm(const GemmParams& p, hipStream_t stream) {
       e = plan_gemm<128, 128>(p, cus, kRate128x128, -1);
     }
   }
-  // Long K (fc2, K = 4096 / 4352) from 512 rows: 128x128 tiles split along K where up to 8 parts fill
-  // at least 7/8 of the CUs (one 784-token image's fc2: 23.9 against 25.2 us for 288x128 tiles in 8
-  // parts); at the mergers' 196 rows the cost model's plans stay ahead (25.2 / 26.8 against 20.3 /
-  // 24.2 us on 128x128).
+  // Long K past one round of 32x128 tiles, from 512 rows: 128x128 tiles split along K where up to 8 parts fill at least
+  // 7/8 of the CUs. Cold weights, residual: 576 / 640 x 2048 x 4096 27.8 / 28.1 us against 28.2 / 31.9 for the best of the
+  // larger tiles (288x128) split along K; 1200 and 1280 x 1024 x 4096 27.7 against 27.3 (256x128); the largest that comes
+  // here loses, 1800 x 1024 x 4096 34.6 against 32.0. 1404 x 1152 x 4352 (99 tiles, 198 parts) is left to the cost
+  // model: 34.9 here, 30.2 there.
   if (pick == 0 && whole && p.K > kSmallTileMaxK && rows >= 512 && f.split_mode >= 0 &&
       EPI != kEpiBiasPosEmbed && 2 * tiles128 < cus) {
     const GemmPlan sp = plan_gemm<128, 128>(p, cus, kRate128x128, 1);
@@ -1581,10 +1582,10 @@ static int dispatch_gemm(const GemmParams& p, hipStream_t stream) {
       e = sp;
     }
   }
-  // A folded LayerNorm over more than 16 row groups (the deepstack mergers' 4-token rows: 32 or 36)
-  // combines each row's partials in the workgroup's prologue; on small grids 64-row tiles split
-  // along K spread that over 4x the workgroups (one 784-token image's deepstack fc1, K = 4096:
-  // 27.2 against 33.4 us for 256x128 tiles split 8 ways).
+  // A folded LayerNorm over more than 16 row groups (the deepstack mergers' 4-token rows) combines each row's partials in
+  // the workgroup's prologue; 64-row tiles split along K spread that over more workgroups. What comes here are up to 64 rows
+  // of the 8B shape's fc1, whose weights the few-rows kernel leaves: 49 / 64 x 4608 x 4608, cold weights, 20.9 / 21.2 us
+  // against 29.6 / 29.7 for 256x128 tiles split along K and 32.3 / 33.7 for 32x128.
   if (pick == 0 && whole && LN && p.ln_part && p.ln_groups > 16 && f.split_mode >= 0 &&
       2 * ((rows + 63) / 64) * ((p.N + 127) / 128) <= cus) {
     const GemmPlan sp = plan_gemm<64, 128>(p, cus, kRate128x128, 1);
