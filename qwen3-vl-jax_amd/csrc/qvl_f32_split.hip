@@ -1,17 +1,18 @@
 // fp32 Dense on the f16 matrix cores: each fp32 operand is written as two f16 terms of a power-of-two
 // multiple of it, x 2^e = hi + lo + r (|r| <= 2^-23 |x 2^e|: 11 + 11 significant bits and lo's sign), and
 //   x . w = 2^-(ex + ew) (hi_x . hi_w + hi_x . lo_w + lo_x . hi_w) + (lo_x . lo_w and r terms)
-// runs as three v_mfma_f32_32x32x16_f16 products into one fp32 accumulator. The dropped terms are at most
-// 2^-22 of a product, random in sign; the f16 products themselves are exact in fp32. One fp32 accumulation
-// chain takes 3 K / 16 instruction steps against K / 2 for v_mfma_f32_32x32x2_f32, so the result is nearer to
-// float64 than the fp32 MFMA's: normal operands, K = 1024 / 4096: 3.6e-7 / 7.1e-7 of the result's norm (less
-// where K is split) against 5.7e-7 / 1.1e-6, at 3/16 of its matrix time (MI355X: 2.5 PFLOP/s f16 against 157
-// TFLOP/s fp32).
+// runs as three v_mfma_f32_32x32x16_f16 products: hi . hi into one fp32 accumulator, the two cross products into another
+// (256x256 tiles, whose registers do not hold both, add all three into one). The dropped terms are at most 2^-22 of a
+// product, random in sign; the f16 products themselves are exact in fp32. The large sums then round K / 16 times (3 K / 16
+// on 256x256 tiles) against K / 2 for v_mfma_f32_32x32x2_f32, so the result is nearer to float64 than the fp32 MFMA's:
+// normal operands, K = 1024 / 4096: 2e-7 / 4e-7 of the result's norm (3.6e-7 / 7.1e-7 with one accumulator; less where K
+// is split) against 5.7e-7 / 1.1e-6, at 3/16 of its matrix time (MI355X: 2.5 PFLOP/s f16 against 157 TFLOP/s fp32).
 //
 // Split rows: a row of K values (K a multiple of 32) is K / 32 groups of [32 hi | 32 lo] f16, 128 bytes a
 // group: the same bytes as the fp32 row, and one group is one k-step's LDS row of the bf16 GEMM's layout. The
 // exponent is per row, so that the row's largest value lands in [2^14, 2^15): values down to 2^-17 of it keep
-// 22 bits, smaller ones an absolute error of 2^-39 of it.
+// 22 bits, smaller ones an absolute error of 2^-39 of it. Rows that this does not suit go by fp32 (row_is_wide,
+// group_max).
 #include <math.h>
 
 #include <algorithm>
@@ -93,6 +94,17 @@ __device__ __forceinline__ bool row_is_wide(uint32_t mb, uint32_t small, const f
   return 4 * small > row_count<T>(some, tmp);
 }
 
+// store_split4 of columns c..c+3 by lane t, c = 4 t + a multiple of 8: a pair of lanes trades halves, so that each stores 16
+// bytes and 8 lanes a whole 128-byte group.
+__device__ __forceinline__ void store_split_pair(f16* row, int c, const f16x4& hi, const f16x4& lo, int t) {
+  const u32x2 h = __builtin_bit_cast(u32x2, hi), l = __builtin_bit_cast(u32x2, lo);
+  const bool odd = t & 1;
+  const uint32_t g0 = __builtin_amdgcn_mov_dpp(odd ? h.x : l.x, 0xB1, 0xF, 0xF, true);    // quad_perm 1 0 3 2
+  const uint32_t g1 = __builtin_amdgcn_mov_dpp(odd ? h.y : l.y, 0xB1, 0xF, 0xF, true);
+  f16* at = row + (c >> 5) * 64 + (odd ? 28 : 0) + (c & 31);
+  *reinterpret_cast<u32x4*>(at) = odd ? u32x4{g0, g1, l.x, l.y} : u32x4{h.x, h.y, g0, g1};
+}
+
 // ---------------------------------------------------------------------------------------------
 // fp32 rows -> split rows: a row's maximum, then its values scaled and split. Memory bound (each row read
 // and written once): T = 64 or 256 threads hold a row in registers, CH chunks of 4 values each, so that
@@ -140,7 +152,7 @@ __global__ __launch_bounds__(256) void split_rows_kernel(SplitRowsParams p) {
     if (c >= p.K) break;
     f16x4 hi, lo;
     split4(v[i], s, hi, lo);
-    store_split4(dst, c, hi, lo);
+    store_split_pair(dst, c, hi, lo, t);
     small += count_small(v[i], s);
   }
   const bool wide = row_is_wide<T>(mb, small, v, tmp);
@@ -201,7 +213,7 @@ __global__ __launch_bounds__(256) void split_weights_kernel(SplitWeights p) {
     if (c >= k) break;
     f16x4 hi, lo;
     split4(v[i], s, hi, lo);
-    store_split4(dst, c, hi, lo);
+    store_split_pair(dst, c, hi, lo, t);
     small += count_small(v[i], s);
   }
   const bool wide = T == 64 ? row_is_wide<64>(mb, small, v, tmp) : row_is_wide<256>(mb, small, v, tmp);
@@ -240,29 +252,26 @@ __global__ __launch_bounds__(256) void split_weights_kernel(SplitWeights p) {
 // 24 bits. kGroupAlike: NaN where more than a quarter of them (zeros aside) are lower, or one is not finite: the Dense
 // then writes fp32 rows in place of split rows, and its reader takes them as such. (An atomic maximum per row on one
 // address took the launch above from 10 to 45 us.)
-// (kGroupAlike: n at most 8192.)
 __device__ __forceinline__ void group_max(const float* __restrict__ v, int n, int kind, float* __restrict__ out, float* tmp) {
-  constexpr int CH = 32;
-  uint32_t u[CH], mb = 0;
-  for (int base = 0; base < n; base += 256 * CH) {           // (once, unless n > 8192)
-#pragma unroll
-    for (int i = 0; i < CH; ++i) {
-      const int at = base + 256 * i + threadIdx.x;
-      u[i] = at < n ? __float_as_uint(v[at]) & 0x7fffffffu : 0;
-    }
-#pragma unroll
-    for (int i = 0; i < CH; ++i) mb = max(mb, u[i]);
-  }
+  uint32_t mb = 0;
+#pragma unroll 4
+  for (int i = threadIdx.x; i < n; i += 256) mb = max(mb, __float_as_uint(v[i]) & 0x7fffffffu);
   mb = block_max_bits(mb, tmp);
   if (kind == kGroupInf) mb = min(mb, 0x7f800000u);
-  if (kind == kGroupAlike && mb >= 0x7f800000u) mb = 0x7fc00000u;
-  if (kind == kGroupAlike && mb < 0x7f800000u) {
-    const uint32_t low = __float_as_uint(__uint_as_float(mb) * 0x1p-9f);
-    uint32_t count = 0;                                      // lower ones, and 2^16 x those not zero
-#pragma unroll
-    for (int i = 0; i < CH; ++i) count += (u[i] ? 0x10000u : 0u) + (u[i] && u[i] < low ? 1u : 0u);
-    count = row_count<256>(count, tmp);
-    if (4 * (count & 0xffffu) > (count >> 16)) mb = 0x7fc00000u;
+  if (kind == kGroupAlike) {
+    const float low = __uint_as_float(mb) * 0x1p-9f;
+    uint32_t lower = 0;
+#pragma unroll 4
+    for (int i = threadIdx.x; i < n; i += 256) lower += v[i] < low;
+    lower = row_count<256>(lower, tmp);
+    if (mb >= 0x7f800000u) {
+      mb = 0x7fc00000u;
+    } else if (4 * lower > (uint32_t)n) {               // (zeros count as lower: how many there are is seldom asked)
+      uint32_t some = 0;
+      for (int i = threadIdx.x; i < n; i += 256) some += v[i] > 0.f;
+      some = row_count<256>(some, tmp);
+      if (4 * (lower - ((uint32_t)n - some)) > some) mb = 0x7fc00000u;
+    }
   }
   if (threadIdx.x == 0) *out = __uint_as_float(mb);
 }
@@ -362,7 +371,7 @@ __global__ __launch_bounds__(256) void layernorm_split_kernel(const float* __res
     }
     f16x4 hi, lo;
     split4(v[i], sc, hi, lo);
-    store_split4(dst, ocol + c, hi, lo);
+    store_split_pair(dst, ocol + c, hi, lo, t);
   }
   if (t == 0 && (!MERGE || (row & 3) == 0)) inv[orow] = wide ? __uint_as_float(0x7fc00000u) : 1.0f / sc;
 }

@@ -34,6 +34,8 @@ def _qdtype(t):
 
 def _beside(t, hidden, what: str):
     """t on hidden's GPU: the kernels read its memory there. Host memory is refused; another GPU's tensor is copied."""
+    if t.device == hidden.device:
+        return t
     if t.device.type != hidden.device.type:
         raise ValueError(f"{what} on {t.device}, hidden on {hidden.device}")
     return t.to(hidden.device)
