@@ -204,20 +204,22 @@ __global__ __launch_bounds__(256) void split_weights_kernel(SplitWeights p) {
 #pragma unroll
     for (int j = 0; j < 4; ++j) mb = max(mb, __float_as_uint(v[i][j]) & 0x7fffffffu);
   mb = max_bits(mb);
-  const float s = split_scale(__uint_as_float(mb));
-  f16* dst = e.out + (int64_t)row * 2 * k;
-  uint32_t small = 0;
+  if (e.out) {
+    const float s = split_scale(__uint_as_float(mb));
+    f16* dst = e.out + (int64_t)row * 2 * k;
+    uint32_t small = 0;
 #pragma unroll
-  for (int i = 0; i < CH; ++i) {
-    const int c = (t + i * T) * 4;
-    if (c >= k) break;
-    f16x4 hi, lo;
-    split4(v[i], s, hi, lo);
-    store_split_pair(dst, c, hi, lo, t);
-    small += count_small(v[i], s);
+    for (int i = 0; i < CH; ++i) {
+      const int c = (t + i * T) * 4;
+      if (c >= k) break;
+      f16x4 hi, lo;
+      split4(v[i], s, hi, lo);
+      store_split_pair(dst, c, hi, lo, t);
+      small += count_small(v[i], s);
+    }
+    const bool wide = T == 64 ? row_is_wide<64>(mb, small, v, tmp) : row_is_wide<256>(mb, small, v, tmp);
+    if (t == 0) e.inv[row] = wide && (p.mark_wide || mb >= 0x7f800000u) ? __uint_as_float(0x7fc00000u) : 1.0f / s;
   }
-  const bool wide = T == 64 ? row_is_wide<64>(mb, small, v, tmp) : row_is_wide<256>(mb, small, v, tmp);
-  if (t == 0) e.inv[row] = wide && (p.mark_wide || mb >= 0x7f800000u) ? __uint_as_float(0x7fc00000u) : 1.0f / s;
   if (!e.row_bound) return;
   uint32_t gb = 0;                                                 // the bits of max |gamma w|
   float norm = 0.f, dot = 0.f;

@@ -1107,7 +1107,8 @@ int qvl_vision_split_bounds(void* stream, const qvl_vision_config* c, const qvl_
   QVL_TRY_RC(tower_layout(c, 0, &L));
   if (!bounds) return set_error(QVL_ERR_INVALID_ARG, "vision_split_bounds: NULL bounds");
   hipStream_t st = (hipStream_t)stream;
-  const auto layer = [&](const SplitScratch& s, float* out) {
+  const auto layer = [&](SplitScratch& s, float* out) {
+    for (int i = 0; i < s.p.count; ++i) s.p.e[i].out = nullptr;
     QVL_TRY_RC(split_weights(s.p, st));
     GroupMaxes g{};
     for (int i = 0; i < s.p.count; ++i) {

@@ -102,7 +102,8 @@ struct GemmSplitParams {
 };
 
 // The Dense weights of one layer that one launch writes as split rows (split_weights): w [n][k] packed fp32, gamma /
-// beta [ln_cols] of the LayerNorm before it repeat along the row (NULL: 1 / 0). first: set by the launcher.
+// beta [ln_cols] of the LayerNorm before it repeat along the row (NULL: 1 / 0). out / row_bound NULL: not wanted. first:
+// set by the launcher.
 struct SplitWeight {
   const float *w, *bias, *gamma, *beta;
   _Float16* out;

@@ -499,7 +499,7 @@ class Qwen3VisionTransformer:
         capi.check(self._lib.qvl_vision_split_bounds(self._stream(), C.byref(self._cfg), C.byref(self._w),
                                                      buf.data_ptr(), nb.value, bounds.data_ptr()),
                    "qvl_vision_split_bounds")
-        return buf if bool(torch.isfinite(bounds).all()) else None
+        return buf if np.isfinite(bounds.cpu().numpy()).all() else None
 
     def _vec(self, v):
         torch = _torch()
