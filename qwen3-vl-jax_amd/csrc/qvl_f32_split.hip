@@ -176,10 +176,9 @@ static int split_rows(const SplitRowsParams& p, hipStream_t stream) {
 // A tower splits each layer's weights on the stream right before they are used, so that a forward (or a graph's
 // replay) reads the weights as they are then; all Dense weights of a layer share one launch, a wave or a workgroup
 // holds a row.
-// Memory bound: a 1024-wide block's 48 MB are read and written in 20 us, a copy's 4.7 TB/s (28 us with a wave on every
+// Memory bound: a 1024-wide block's 48 MB are read and written in 21 us, a copy's 4.7 TB/s (28 us with a wave on every
 // row: 16 chunks of a 4096-wide row are too many registers for the waves that keep the loads in flight). A 784-patch
-// forward of 24 blocks takes 4.37 ms with it, 3.85 with weights split beforehand, and 8.8 on the fp32 MFMA kernels.
-// ---------------------------------------------------------------------------------------------
+// forward of 24 blocks takes 4.76 ms with it, 4.12 with weights split beforehand, and 8.8 on the fp32 MFMA kernels.
 template <int CH>
 __global__ __launch_bounds__(256) void split_weights_kernel(SplitWeights p) {
   __shared__ float tmp[4];
