@@ -493,6 +493,8 @@ class Qwen3VisionTransformer:
         nb = C.c_size_t()
         if self._lib.qvl_vision_split_scratch_size(C.byref(self._cfg), C.byref(nb)) != 0:
             return None
+        if torch.cuda.is_current_stream_capturing():      # (the look at the bounds waits for the GPU)
+            return None
         buf = torch.empty(nb.value, dtype=torch.uint8, device=self.device)
         bounds = torch.empty(6 * s.depth + 2 * (1 + len(s.deepstack_visual_indexes)) + 1, dtype=torch.float32,
                              device=self.device)

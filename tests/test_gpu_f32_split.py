@@ -464,3 +464,23 @@ def test_split_tower_with_wide_normalised_rows(pkg, lib, cols):
     a, b = tower_pair(pkg, spec, params)
     for got, want in zip(outputs(a, px, grids), outputs(b, px, grids)):
         assert torch.isfinite(got).all() and (got - want).norm() <= 3e-6 * want.norm()
+
+
+def test_bind_packed_during_a_capture(pkg):
+    """Binding packed buffers launches nothing that a capture refuses; such a tower runs unsplit."""
+    spec, params, px, grids = one_block(pkg)
+    t = pkg.Qwen3VisionTransformer(spec).bind(params)
+    want = outputs(t, px, grids)
+    late = pkg.Qwen3VisionTransformer(spec)
+    late.metadata(grids), late.workspace(24)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        tokens, ds = late.bind_packed(t.packed_state())(px, grids)
+    assert late._split is None
+    for _ in range(3):
+        graph.replay()
+        torch.cuda.synchronize()
+        for a, b in zip((tokens, *ds), want):
+            assert (a - b).norm() <= 3e-6 * b.norm()
+        outputs(t, px, grids)
