@@ -459,9 +459,10 @@ __device__ __forceinline__ bool by_fp32(const GemmSplitParams& p, int m, int n) 
 }
 
 // Rows of x and columns of w whose factor is NaN (row_is_wide): their outputs come from the fp32 operands, on
-// v_mfma_f32_32x32x2_f32, 32 tokens (from m1) x 32 features (from n1) of one wave at a time over k in [k0, k1). x comes from
-// xf, or without it from p.x: a row with a NaN factor lies there as fp32, any other as a split row. Lane l32 holds row l32 of both, hh the k's half of 8. Rare: no LDS, one
-// step of 32 k loaded ahead. Every row wide: 784 x 4096 x 1024 158 us (fp32 MFMA kernel 88), 4096 x 4096 x 1024 569 (300).
+// v_mfma_f32_32x32x2_f32, 32 tokens (from m1) x 32 features (from n1) of one wave at a time over k in [k0, k1). x comes
+// from xf, or without it from p.x: a row with a NaN factor lies there as fp32, any other as a split row. Lane l32 holds
+// row l32 of both, hh the k's half of 8. Rare: no LDS, one step of 32 k loaded ahead. Every row wide: 784 x 4096 x 1024
+// 158 us (fp32 MFMA kernel 88), 4096 x 4096 x 1024 569 (300).
 __device__ __forceinline__ f32x16 split_fp32_block(const GemmSplitParams& p, int m1, int n1, int k0, int k1, int l32, int hh) {
   const int m = min(m1 + l32, p.M - 1);
   const float* w = p.wf + (int64_t)min(n1 + l32, p.N - 1) * p.K + 4 * hh;
